@@ -114,6 +114,29 @@ def test_recognition_batches_together_match_separate(recognizer):
         k0 += n
 
 
+@pytest.mark.parametrize("total", [2, 3, 255, 257, 262])
+def test_recurrence_groups(recognizer, rec_oracle, total):
+    # The recurrence groups 2 lines a workgroup up to 256 lines and 4 past that, longest first:
+    # partly filled last groups, groups that mix lengths (one step to 19) and both forms. The
+    # first and the last batches meet the oracle, and every line has the bits it has alone.
+    rng = np.random.Generator(np.random.PCG64(total))
+    widths = sorted({int(w) for w in rng.integers(5, 78, 12)})[: min(12, total)]
+    counts = [total // len(widths) + (i < total % len(widths)) for i in range(len(widths))]
+    batches = [(rng.uniform(-0.5, 0.5, (n, 64, w)).astype(np.float32), n, w) for n, w in zip(counts, widths)]
+    print(f"recognize {[(n, w) for _, n, w in batches]}", flush=True)
+    logits, lens, best = recognizer.recognize(batches)
+    k0 = 0
+    for i, (d, n, w) in enumerate(batches):
+        T = int(lens[k0])
+        for j in {0, n - 1}:
+            one, _, best1 = recognizer.recognize([(d[j: j + 1], 1, w)])
+            assert np.array_equal(logits[:T, k0 + j], one[:T, 0]), (n, w, j)
+            assert np.array_equal(best[:T, k0 + j], best1[:T, 0])
+        if i in (0, len(batches) - 1):
+            check_recognition(recognizer, rec_oracle, [(d[:3].copy(), min(n, 3), w)], [w] * min(n, 3))
+        k0 += n
+
+
 @pytest.mark.parametrize("tied", [(7, 40, 96), (3, 60), (0, 1)])
 def test_recognition_argmax_ties(ctx, tied):
     """Tied maxima at every step: output-layer columns made identical, with a bias well above

@@ -184,12 +184,19 @@ void argmax_rows(const float *x, int rows, int classes, uint32_t *best, hipStrea
 
 // ---- GRU recurrence (kernels/gru.hip) -------------------------------------------------------
 // One layer, both directions, every line with its own length (gpu.rs:680-819). G [t][n][1536]
-// holds W x + Wb; R [2][768][256] float16 (exact values); Rb [2][768]; Y [t][n][512].
-// steps: the sum of lens (for the probe's work count only).
-void gru_recurrence(const float *G, const uint16_t *R, const float *Rb, float *Y, const uint32_t *lens, int ntot,
-                    int tmax, long long steps, hipStream_t s);
-// The same with float32 recurrent weights, given transposed: Rt [2][256 k][768 rows] (for R
-// that is not float16-valued when rounding it is not allowed; R streams from L2 every step).
+// holds W x + Wb, for the update and reset gates with Rb added; R float16, packed by gru_pack_r;
+// Rb [2][256], the candidate's recurrent bias; Y [t][n][512]; order: the lines, longest first;
+// lines: how many share a workgroup (gru_lines). steps: the sum of lens (for the probe's work
+// count only).
+void gru_recurrence(const float *G, const uint16_t *R, const float *Rb, float *Y, const uint32_t *lens,
+                    const uint32_t *order, int lines, int ntot, long long steps, hipStream_t s);
+// R [2][768][256] float16 in the order that the kernel's wavefronts read it (the same size).
+void gru_pack_r(const uint16_t *r, uint16_t *out);
+// Lines a workgroup (2 or 4) for a pass of ntot lines.
+int gru_lines(int ntot);
+// The same with float32 recurrent weights, given transposed: Rt [2][256 k][768 rows], G = W x + Wb
+// for every gate and Rb [2][768] (for R that is not float16-valued when rounding it is not
+// allowed; R streams from L2 every step).
 void gru_recurrence_f32(const float *G, const float *Rt, const float *Rb, float *Y, const uint32_t *lens, int ntot,
                         long long steps, hipStream_t s);
 

@@ -5,24 +5,37 @@
 //   z = s(G_z + R_z h + Rb_z), r = s(G_r + R_r h + Rb_r), c = tanh(G_h + r (R_h h + Rb_h)),
 //   h' = (1 - z) c + z h, h0 = 0,  with G = W x + Wb precomputed for all steps by one GEMM.
 //
-// Mapping to gfx950: a workgroup owns one direction and 8 lines. R (768 x 256 per direction,
-// float16 values) is loaded once as MFMA A-operand fragments, mostly into VGPRs and the rest
-// into LDS, and stays resident for every time step. The hidden state of the 8 lines is the MFMA B operand: 16 columns, columns
-// 0-7 its float16 "hi" part and columns 8-15 the float16 remainder "lo" (h = hi + lo to about
-// 2^-22), so one v_mfma_f32_16x16x32_f16 per 16 rows and 32 hidden units gives R h for all 8
-// lines at float32-class accuracy. Each wavefront owns UPW hidden units (all three gate rows of
-// them), so the gate nonlinearity needs no exchange across wavefronts.
+// What bounds it is one line's chain of dependent steps: the work of a step is small, and a line
+// cannot start one before the step before it ends. So a workgroup owns one direction and few
+// lines (2 or 4), and its step is made as short as one CU can make it. R (768 x 256 a direction,
+// float16 values) is loaded once, into the registers of 8 wavefronts, and stays for every step.
 //
-// Per step, after the MFMAs, lane (g, r) of a 16-lane row holds rows 4g..4g+3 of column r. The
-// hi and lo columns of a line are summed with one DPP rotation by 8, arranged so that lane r < 8
-// ends with units 4g, 4g+1 of line r and lane r + 8 with units 4g+2, 4g+3 of the same line:
-// every lane does gate arithmetic for two units. The step's G values are loaded at the end of
-// the previous step, so the HBM latency hides behind the barrier (an LDS-only one: the loads and
-// the Y stores stay in flight) and the MFMA phase. The new state goes to a double-buffered LDS
-// copy of the B operand: one barrier per step.
+// R h is a product with 16 rows at least on the matrix cores, and 4 lines are only 8 rows: each
+// line's float16 "hi" part and its float16 remainder "lo" (h = hi + lo to about 2^-22). The
+// sparse instruction v_smfmac_f32_16x16x64_f16 takes an A operand with two of every four k
+// present, and twice the k of the dense one in the same cycles. So the state is the A operand
+// and every part is spread over two rows, one with the first two of each four hidden units and
+// one with the other two: nothing is left out, the four rows of a line add up to R h, and a step
+// takes half the matrix instructions (48 a SIMD, 768 cycles). R is the dense B operand, a column
+// a hidden unit. Lane group g (16 lanes) then holds the four rows of one line in its four
+// accumulators: the sum needs no exchange between lanes. With 2 lines the A rows repeat, so two
+// lane groups hold a line's sums and each takes one of a wavefront's two 16-unit tiles: a lane
+// does the gate arithmetic of one unit a step (two with 4 lines).
+//
+// Every gate's arithmetic runs between the next gate's matrix instructions (reset, candidate,
+// update); only the update gate and the new state follow the last one. G is loaded four steps
+// ahead, the new state goes to a double-buffered LDS copy of the A operand: one barrier a step,
+// for LDS only (the loads and the Y stores stay in flight).
+//
+// Measured (a 200-step pass, us a layer): 36 lines 303 -> 129, 540 lines 424 -> 190, against 8
+// lines a workgroup on the dense instruction with the state as its 16-column operand; 200-pixel
+// line alone (50 steps) 77 -> 39. A step takes 0.59 us with 2 lines, of it 0.32 of matrix
+// instructions; 16 wavefronts (4 a SIMD, part of R in LDS) took 1.6, 4 wavefronts (one unit of
+// one line a lane, R in 384 registers) 0.89.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstring>
 
 #include "../kernels.h"
 #include "../runtime.h"
@@ -31,229 +44,171 @@
 namespace ocr {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-// LDS row of the B operand: 256 units + 16 of padding (34 16-byte units, so the B reads of a step
-// meet distinct bank groups in every access pass and the state writes distinct banks).
-constexpr int H = 256, LINES = 8, HROW = H + 16;
+constexpr int H = 256;
 
 // exp through the hardware base-2 exponential; 1/x through the hardware reciprocal (1 ulp).
 __device__ inline float fast_exp(float v) { return __builtin_amdgcn_exp2f(v * 1.4426950408889634f); }
 __device__ inline float sigm(float v) { return __builtin_amdgcn_rcpf(1.f + fast_exp(-v)); }
 __device__ inline float tanh_f(float v) { return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + fast_exp(2.f * v)); }
 
-// a where the mask's bits are set, b elsewhere (v_bfi_b32): a per-lane choice of a register.
-__device__ inline float sel_bits(unsigned m, float a, float b) {
-    return __uint_as_float((m & __float_as_uint(a)) | (~m & __float_as_uint(b)));
+__device__ inline half16 join(half8 a, half8 b) {
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
 }
 
-// Lane r of each 16-lane row receives the value of lane (r + 8) mod 16 (DPP row_ror:8).
-__device__ inline float ror8(float v) {
-    // (a row rotation has no out-of-row lanes, so bound_ctrl changes nothing; with it the
-    // compiler folds the move into the add that uses it)
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
-}
-
-template <int UPW>
-__global__ __launch_bounds__(H / UPW * 64) void gru_kernel(const float *__restrict__ G, const half8 *__restrict__ R,
-                                                           const float *__restrict__ Rb, float *__restrict__ Y,
-                                                           const uint32_t *__restrict__ lens, int ntot) {
-    constexpr int RT = UPW / 16;  // 16-row tiles per gate per wavefront
-    constexpr int KL = 2;         // k-slices of R kept in LDS ...
-    constexpr int KLQ = UPW == 16 ? 3 : 1;  // ... for the last KLQ gates
-    __shared__ __align__(16) _Float16 hbuf[2][16][HROW];
-    __shared__ float s_rb[768];  // this direction's recurrent bias [z | r | h]
-    __shared__ half8 s_rf[H / UPW][KLQ * RT * KL][64];
+// LG lines a workgroup (2 or 4), 8 wavefronts of 32 hidden units (two 16-unit tiles each).
+template <int LG>
+__global__ __launch_bounds__(512) void gru_kernel(const float *__restrict__ G, const half8 *__restrict__ R,
+                                                  const float *__restrict__ Rb, float *__restrict__ Y,
+                                                  const uint32_t *__restrict__ lens, const uint32_t *__restrict__ order,
+                                                  int ntot) {
+    constexpr int T = 2;         // 16-unit tiles of a wavefront
+    constexpr int REP = 4 / LG;  // lane groups that hold the same line's sums
+    constexpr int U = T / REP;   // units of its line that a lane updates
+    constexpr int D = 4;         // steps that G is loaded ahead (three whole steps pass before its use)
+    static_assert(LG == 2 || LG == 4, "every lane has whole units");
+    // The state as the A operands read it: [k-step][lane group][row][8 halves], row = 4 line + 2
+    // (lo part) + (odd pair): the 64 lanes of a read take 64 neighbouring 16-byte units.
+    __shared__ __align__(16) _Float16 hbuf[2][4][4][4 * LG][8];
+    // With 4 lines the update gate's last k-step of R lives in LDS: the rest fills the registers.
+    constexpr int TL = LG == 4 ? T : 0;
+    __shared__ half8 s_rf[TL ? 8 : 1][TL ? TL : 1][2][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, r = lane & 15;
-    const int dir = blockIdx.y, n0 = blockIdx.x * LINES;
+    const int dir = blockIdx.y, n0 = blockIdx.x * LG;
 
-    // R fragments: rows gate * 256 + unit, unit = wave * UPW + rt * 16 + r; k = kt * 32 + 8g .. +7.
-    // All are held in VGPRs except the last KL k-slices of the last KLQ gates, which live in LDS
-    // (the register file holds the rest of the step's state without spilling).
-    half8 rf[3][RT][8];
+    // R as B operands: column r = unit wave * 32 + t * 16 + r; lane group g holds k-step kt's
+    // k = 8 g .. + 7 and 32 + 8 g .. + 7.
+    half16 rf[3][T][4];
 #pragma unroll
     for (int q = 0; q < 3; q++)
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++)
+        for (int t = 0; t < T; t++)
 #pragma unroll
-            for (int kt = 0; kt < 8; kt++) {
-                const half8 v = R[(size_t(dir) * 768 + q * 256 + wave * UPW + rt * 16 + r) * 32 + kt * 4 + g];
-                if (q >= 3 - KLQ && kt >= 8 - KL) s_rf[wave][((q - (3 - KLQ)) * RT + rt) * KL + kt - (8 - KL)][lane] = v;
-                else rf[q][rt][kt] = v;
+            for (int kt = 0; kt < 4; kt++) {
+                const half8 *src = R + ((((size_t(dir) * 8 + wave) * 3 + q) * T + t) * 4 + kt) * 128 + lane;
+                const half8 v0 = src[0], v1 = src[64];
+                if (q == 0 && kt == 3 && t < TL) {
+                    s_rf[wave][t][0][lane] = v0;
+                    s_rf[wave][t][1][lane] = v1;
+                } else {
+                    rf[q][t][kt] = join(v0, v1);
+                }
             }
+    for (int i = tid; i < int(sizeof(hbuf) / 16); i += 512) reinterpret_cast<uint4 *>(hbuf)[i] = uint4{0, 0, 0, 0};
 
-    for (int i = tid; i < 2 * 16 * HROW; i += blockDim.x) (&hbuf[0][0][0])[i] = (_Float16)0.f;
-    for (int i = tid; i < 768; i += blockDim.x) s_rb[i] = Rb[dir * 768 + i];
-
+    // This lane's line and units. Slots past the last line repeat it (the same values written
+    // twice).
+    const int ls = g % LG, sub = g / LG;
+    const int line = int(order[min(n0 + ls, ntot - 1)]);
+    const int len = int(lens[line]);
     int maxlen = 0;
-    for (int j = 0; j < LINES; j++)
-        if (n0 + j < ntot) maxlen = max(maxlen, int(lens[n0 + j]));
-    // This lane's line and the two units (of each 16-row tile) it updates: lane r < 8 takes
-    // units 4g, 4g+1 of line r, lane r >= 8 units 4g+2, 4g+3 of line r - 8.
-    const bool upper = r >= LINES;
-    const unsigned umask = upper ? ~0u : 0u;
-    const int lr = upper ? r - LINES : r;
-    const int line = n0 + lr;
-    const int len = line < ntot ? int(lens[line]) : 0;
-    const int usub = upper ? 2 : 0;
-    float h[RT][2];
+    for (int j = 0; j < LG; j++) maxlen = max(maxlen, int(lens[order[min(n0 + j, ntot - 1)]]));
+    const size_t row = size_t(dir == 0 ? 0 : max(len - 1, 0)) * ntot + line;
+    const int u0 = (wave * T + sub * U) * 16 + r;
+    const float *gp = G + row * 1536 + dir * 768 + u0;
+    float *yp = Y + row * 512 + dir * 256 + u0;
+    const long gstep = (dir == 0 ? 1536l : -1536l) * ntot, ystep = (dir == 0 ? 512l : -512l) * ntot;
+    float h[U], rb[U];
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) h[rt][0] = h[rt][1] = 0.f;
-    __syncthreads();
-    // G of the step about to run, [gate][rt] pairs of units; loaded one step ahead.
-    auto load_g = [&](int s, float2 (&gv)[3][RT]) {
-        const int t = dir == 0 ? s : len - 1 - s;
-        if (s < len) {
-            const float *gb = G + (size_t(t) * ntot + line) * 1536 + dir * 768 + wave * UPW + 4 * g + usub;
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++)
-                    gv[q][rt] = *reinterpret_cast<const float2 *>(gb + q * 256 + rt * 16);
-        }
-    };
-    float2 gcur[3][RT];
-    load_g(0, gcur);
-    // The recurrent bias of the lane's units, the same every step.
-    float rbv[3][RT][2];
-#pragma unroll
-    for (int q = 0; q < 3; q++)
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-            for (int i = 0; i < 2; i++) rbv[q][rt][i] = s_rb[q * 256 + wave * UPW + rt * 16 + 4 * g + usub + i];
-
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    for (int s = 0; s < maxlen; s++) {
-        const int cur = s & 1;
-        const bool on = s < len;
-        floatx4 acc[3][RT];
+    for (int u = 0; u < U; u++) {
+        h[u] = 0.f;
+        rb[u] = Rb[dir * 256 + u0 + u * 16];
+    }
+    // G of D steps ahead; past its end a line reads its last row again.
+    float gv[D][3][U];
+    auto load_g = [&](int s, float (&v)[3][U]) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++)
-                acc[q][rt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        // R h for row tile rt of the three gates (8 k-slices); the B fragment of k-slice kt + 1
-        // is read from LDS before k-slice kt's MFMAs, so its latency hides behind them.
-        auto mfmas = [&](int rt, int q0 = 0, int q1 = 3) __attribute__((always_inline)) {
-            half8 bb[2];
-            bb[0] = *reinterpret_cast<const half8 *>(&hbuf[cur][r][8 * g]);
+            for (int u = 0; u < U; u++) v[q][u] = gp[q * 256 + u * 16];
+        gp += s + 1 < len ? gstep : 0;
+    };
 #pragma unroll
-            for (int kt = 0; kt < 8; kt++) {
-                if (kt < 7) bb[(kt + 1) & 1] = *reinterpret_cast<const half8 *>(&hbuf[cur][r][(kt + 1) * 32 + 8 * g]);
-                const half8 b = bb[kt & 1];
+    for (int d = 0; d < D; d++) load_g(d, gv[d]);
+    // Even rows of A hold each group of four k's first two values, odd rows the other two.
+    const int idx = (r & 1) ? 0xEEEE : 0x4444;
+    const int arow = r % (4 * LG);
+    // Where the lane's new state goes: tile = 16 k of k-step tile / 4, lane group tile % 4.
+    _Float16 *const hw = &hbuf[0][0][0][4 * ls + ((r >> 1) & 1)][2 * (r >> 2) + (r & 1)] + (wave * T + sub * U) * 32 * LG;
+    constexpr int HB = 4 * 4 * 4 * LG * 8;  // halves of a state buffer
+    __syncthreads();
+
+    auto step = [&](int s, int cur, float (&gc)[3][U]) __attribute__((always_inline)) {
+        half8 a[4];
 #pragma unroll
-                for (int q = q0; q < q1; q++) {
-                    const half8 a = (q >= 3 - KLQ && kt >= 8 - KL)
-                                        ? s_rf[wave][((q - (3 - KLQ)) * RT + rt) * KL + kt - (8 - KL)][lane]
-                                        : rf[q][rt][kt];
-                    acc[q][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[q][rt], 0, 0, 0);
+        for (int kt = 0; kt < 4; kt++) a[kt] = *reinterpret_cast<const half8 *>(hbuf[cur][kt][g][arow]);
+        floatx4 acc[3][T];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[q][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        auto mfmas = [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int t = 0; t < T; t++) {
+                    const half16 b = q == 0 && kt == 3 && t < TL ? join(s_rf[wave][t][0][lane], s_rf[wave][t][1][lane])
+                                                                 : rf[q][t][kt];
+                    acc[q][t] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a[kt], b, acc[q][t], idx, 0, 0);
                 }
+        };
+        // The sum of gate q for the lane's unit u: the four rows of its line.
+        auto total = [&](int q, int u) __attribute__((always_inline)) {
+            const floatx4 c = acc[q][u];
+            float v = (c[0] + c[1]) + (c[2] + c[3]);
+            if (REP == 2) {
+                const floatx4 d = acc[q][T - 1];
+                const float w = (d[0] + d[1]) + (d[2] + d[3]);
+                v = sub ? w : v;
             }
+            return v;
         };
-        // The new state of row tile rt's units (also the step's Y).
-        float hn[RT][2];
-        float zv[RT][2], rv[RT][2];
-        // hi + lo of R h for gate q of row tile rt: lane r < 8 keeps rows 0, 1 and sends rows 2, 3
-        // to lane r + 8 (and the reverse).
-        auto rh_of = [&](int q, int rt, float (&o)[2]) __attribute__((always_inline)) {
-            // The lane's choice between rows 0, 1 and 2, 3 as bit selects on the upper-lane
-            // mask (one bitfield insert each; a ternary on `upper` is compiled as a dynamic
-            // index into the accumulator, a chain of compares and selects).
-            const float send0 = sel_bits(umask, acc[q][rt][0], acc[q][rt][2]);
-            const float send1 = sel_bits(umask, acc[q][rt][1], acc[q][rt][3]);
-            const float keep0 = sel_bits(umask, acc[q][rt][2], acc[q][rt][0]);
-            const float keep1 = sel_bits(umask, acc[q][rt][3], acc[q][rt][1]);
-            o[0] = keep0 + ror8(send0);
-            o[1] = keep1 + ror8(send1);
-        };
-        // The update and reset gates of row tile rt (they need only their own rows' MFMAs).
-        auto gates_zr = [&](int rt) __attribute__((always_inline)) {
-            float rz[2], rr2[2];
-            rh_of(0, rt, rz);
-            rh_of(1, rt, rr2);
+        // Each gate's arithmetic runs between the next gate's MFMAs.
+        auto overlap = []() __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const float gz = i ? gcur[0][rt].y : gcur[0][rt].x;
-                const float gr = i ? gcur[1][rt].y : gcur[1][rt].x;
-                zv[rt][i] = sigm(gz + (rz[i] + rbv[0][rt][i]));
-                rv[rt][i] = sigm(gr + (rr2[i] + rbv[1][rt][i]));
-            }
-        };
-        // The candidate and the new state of row tile rt, branch-free (a line past its end keeps
-        // its state), and the next step's B operand: units u0 and u0 + 1 as one 32-bit word of
-        // hi parts and one of lo parts.
-        auto gates_h = [&](int rt) __attribute__((always_inline)) {
-            float rhh[2];
-            rh_of(2, rt, rhh);
-            const int u0 = wave * UPW + rt * 16 + 4 * g + usub;
-            half2_t hi2, lo2;
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const float gh = i ? gcur[2][rt].y : gcur[2][rt].x;
-                const float z = zv[rt][i], rr = rv[rt][i];
-                const float c = tanh_f(gh + rr * (rhh[i] + rbv[2][rt][i]));
-                hn[rt][i] = (1.f - z) * c + z * h[rt][i];
-                h[rt][i] = on ? hn[rt][i] : h[rt][i];
-                hi2[i] = (_Float16)h[rt][i];
-                lo2[i] = (_Float16)(h[rt][i] - (float)hi2[i]);
-            }
-            *reinterpret_cast<half2_t *>(&hbuf[cur ^ 1][lr][u0]) = hi2;
-            *reinterpret_cast<half2_t *>(&hbuf[cur ^ 1][lr + LINES][u0]) = lo2;
-        };
-        auto gates = [&](int rt) __attribute__((always_inline)) {
-            gates_zr(rt);
-            gates_h(rt);
-        };
-        // Two row tiles: row tile 0's MFMAs; then row tile 1's MFMAs with row tile 0's gate
-        // arithmetic between them (the vector ALU works while the matrix core does); then row
-        // tile 1's gates. One row tile: the update and reset rows' MFMAs, then the candidate
-        // rows' MFMAs with the update and reset gates between them, then the candidate and the
-        // new state.
-        static_assert(RT == 1 || RT == 2, "one or two row tiles a wavefront");
-        if constexpr (RT == 2) {
-            mfmas(0);
-            __builtin_amdgcn_sched_barrier(0);
-            mfmas(1);
-            gates(0);
-#pragma unroll
-            for (int i = 0; i < 24; i++) {
+            for (int i = 0; i < 4 * T; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
                 __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (RT == 1) {
-            mfmas(0, 0, 2);
-            __builtin_amdgcn_sched_barrier(0);
-            mfmas(0, 2, 3);
-            gates_zr(0);
+        };
+        float rr[U], c[U];
+        mfmas(1);
+        __builtin_amdgcn_sched_barrier(0);
+        mfmas(2);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // five VALU
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            gates_h(0);
-        } else {
-            gates(RT - 1);
-        }
-        if (on) {
-            const int t = dir == 0 ? s : len - 1 - s;
+        for (int u = 0; u < U; u++) rr[u] = sigm(total(1, u) + gc[1][u]);
+        overlap();
+        mfmas(0);
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                const int u0 = wave * UPW + rt * 16 + 4 * g + usub;
-                *reinterpret_cast<float2 *>(Y + (size_t(t) * ntot + line) * 512 + dir * 256 + u0) =
-                    make_float2(hn[rt][0], hn[rt][1]);
-            }
+        for (int u = 0; u < U; u++) c[u] = tanh_f(fmaf(rr[u], total(2, u) + rb[u], gc[2][u]));
+        overlap();
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float hn = fmaf(sigm(total(0, u) + gc[0][u]), h[u] - c[u], c[u]);
+            h[u] = s < len ? hn : h[u];
+            const _Float16 hi = (_Float16)h[u], lo = (_Float16)(h[u] - (float)hi);
+            _Float16 *dst = hw + (cur ^ 1) * HB + u * 32 * LG;
+            dst[0] = hi;
+            dst[16] = lo;
         }
-        // The next step's G, in flight across the barrier (which waits for LDS only) and the
-        // next MFMA phase.
-        load_g(s + 1, gcur);
+        __builtin_amdgcn_sched_barrier(0);
+        // Past its end a line writes its last state to its last row again.
+#pragma unroll
+        for (int u = 0; u < U; u++) yp[u * 16] = h[u];
+        yp += s + 1 < len ? ystep : 0;
+        load_g(s + D, gc);
         lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = 0; s < maxlen; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) step(s + d, d & 1, gv[d]);
     }
 }
 
@@ -317,19 +272,37 @@ __global__ __launch_bounds__(256) void gru_f32_kernel(const float *__restrict__ 
 
 }  // namespace
 
-void gru_recurrence(const float *G, const uint16_t *R, const float *Rb, float *Y, const uint32_t *lens, int ntot,
-                    int tmax, long long steps, hipStream_t s) {
-    (void)tmax;
+// 2 lines a workgroup while every workgroup has a CU of its own (256 of them, two directions):
+// 0.65 us a step against 0.81 with 4 lines at 36 lines, 0.82 against 0.86 at 256. Past that 4
+// lines: the longest lines start first, so a 540-line pass (270 workgroups) still ends with its
+// longest line, 190 us against 265 with 2 lines.
+int gru_lines(int ntot) { return ntot <= 256 ? 2 : 4; }
+
+void gru_pack_r(const uint16_t *r, uint16_t *out) {
+    for (int dir = 0; dir < 2; dir++)
+        for (int wave = 0; wave < 8; wave++)
+            for (int q = 0; q < 3; q++)
+                for (int t = 0; t < 2; t++)
+                    for (int kt = 0; kt < 4; kt++)
+                        for (int part = 0; part < 2; part++)
+                            for (int lane = 0; lane < 64; lane++, out += 8) {
+                                const int row = dir * 768 + q * 256 + (wave * 2 + t) * 16 + lane % 16;
+                                std::memcpy(out, r + size_t(row) * 256 + kt * 64 + part * 32 + lane / 16 * 8, 16);
+                            }
+}
+
+void gru_recurrence(const float *G, const uint16_t *R, const float *Rb, float *Y, const uint32_t *lens,
+                    const uint32_t *order, int lines, int ntot, long long steps, hipStream_t s) {
     if (ntot <= 0) return;
-    dim3 grid(unsigned((ntot + LINES - 1) / LINES), 2);
     // Per line step and direction: R h (768 x 256), G read (768 floats), Y written (256 floats).
     ProbeScope probe("gru", s, 2.0 * 2.0 * double(steps) * 768 * 256,
                      2.0 * double(steps) * (768 + 256) * 4 + 2.0 * 768 * 256 * 2);
-    // 16 wavefronts of 16 hidden units (4 a SIMD): the matrix core always has a wavefront to
-    // serve while others do their gate arithmetic (11 % faster per step than 8 of 32 units).
-    constexpr int UPW = 16;
-    hipLaunchKernelGGL((gru_kernel<UPW>), grid, dim3(H / UPW * 64), 0, s, G, reinterpret_cast<const half8 *>(R), Rb,
-                       Y, lens, ntot);
+    auto launch = [&](auto *kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned((ntot + lines - 1) / lines), 2), dim3(512), 0, s, G,
+                           reinterpret_cast<const half8 *>(R), Rb, Y, lens, order, ntot);
+    };
+    if (lines == 2) launch(gru_kernel<2>);
+    else launch(gru_kernel<4>);
     OCR_HIP(hipGetLastError());
 }
 

@@ -111,13 +111,6 @@ Recognizer::Recognizer(Ctx &ctx, const Onnx &onnx, uint32_t lines) : ctx_(ctx), 
         L.input = int(w.dims[2]);
         // W [2][768][in] is already the projection's [1536 outputs][in] (gpu.rs:1466-1472).
         pack_linear(ctx, w.data, 1536, L.input, L.pk, L.w_hi, L.w_lo, L.w_frag);
-        std::vector<float> wb, rb;
-        for (int d = 0; d < 2; d++) {
-            wb.insert(wb.end(), b.data.begin() + d * 1536, b.data.begin() + d * 1536 + 768);
-            rb.insert(rb.end(), b.data.begin() + d * 1536 + 768, b.data.begin() + d * 1536 + 1536);
-        }
-        L.wb = ctx.upload_weights(wb.data(), wb.size());
-        L.rb = ctx.upload_weights(rb.data(), rb.size());
         // R in float16 (gpu.rs:1478-1484): exact for float16-valued weights; otherwise rounded,
         // as the reference does with F16 on (its default). With F16=0 the reference keeps R in
         // float32, and so does this library for R that is not float16-valued: the recurrence
@@ -139,7 +132,20 @@ Recognizer::Recognizer(Ctx &ctx, const Onnx &onnx, uint32_t lines) : ctx_(ctx), 
                         rt[(size_t(d) * 256 + k) * 768 + row] = r.data[(size_t(d) * 768 + row) * 256 + k];
             L.r32 = ctx.upload_weights(rt.data(), rt.size());
         }
-        L.r = ctx.upload_weights(rh.data(), rh.size());
+        std::vector<uint16_t> packed(rh.size());
+        gru_pack_r(rh.data(), packed.data());
+        L.r = ctx.upload_weights(packed.data(), packed.size());
+        // The update and reset gates only ever see Wb + Rb: one bias in the projection, and the
+        // recurrence keeps the candidate's Rb (inside the reset product). The float32 recurrence
+        // takes both biases apart.
+        std::vector<float> wb, rb;
+        for (int d = 0; d < 2; d++) {
+            const float *bw = b.data.data() + d * 1536, *br = bw + 768;
+            for (int i = 0; i < 768; i++) wb.push_back(!L.r32 && i < 512 ? bw[i] + br[i] : bw[i]);
+            rb.insert(rb.end(), br + (L.r32 ? 0 : 512), br + 768);
+        }
+        L.wb = ctx.upload_weights(wb.data(), wb.size());
+        L.rb = ctx.upload_weights(rb.data(), rb.size());
     }
     if (nl != 2) fail(std::to_string(nl) + " GRU layers");
     const Node *mm = nullptr;
@@ -213,8 +219,11 @@ void Recognizer::recognize_device(const Batch *batches, int count, float *logits
     // layout, so the recurrence and the caller see the reference's layout.
     // Lines come in batches of one length each: per step, the runs of lines still going.
     std::vector<int32_t> rows;
+    // The lines, longest first: the recurrence's workgroups start in this order, so the longest
+    // lines never start last, and the lines that share a workgroup are of like length.
+    std::vector<uint32_t> order(ntot);
     {
-        std::vector<std::pair<int, int>> runs;  // (first line, length) of each batch
+        std::vector<std::pair<int, int>> runs;  // (first line, end) of each batch
         size_t total = 0;
         for (int i = 0; i < ntot;) {
             int j = i + 1;
@@ -229,17 +238,26 @@ void Recognizer::recognize_device(const Batch *batches, int count, float *logits
             for (const auto &rn : runs)
                 if (uint32_t(t) < lens[rn.first])
                     for (int i = rn.first; i < rn.second; i++) rows[k++] = t * ntot + i;
+        std::stable_sort(runs.begin(), runs.end(), [&](const std::pair<int, int> &a, const std::pair<int, int> &b) {
+            return lens[a.first] > lens[b.first];
+        });
+        k = 0;
+        for (const auto &rn : runs)
+            for (int i = rn.first; i < rn.second; i++) order[k++] = uint32_t(i);
     }
     const int P = int(rows.size());
     const long long steps = P;
-    // Lengths and rows in one upload, ahead of the trunk's kernels.
-    const size_t rows_at = (size_t(ntot) * 4 + 15) & ~size_t(15);
+    // Lengths, line order and rows in one upload, ahead of the trunk's kernels.
+    const size_t order_at = size_t(ntot) * 4;
+    const size_t rows_at = (size_t(ntot) * 8 + 15) & ~size_t(15);
     std::vector<char> tab(rows_at + rows.size() * 4, 0);
     std::memcpy(tab.data(), lens, size_t(ntot) * 4);
+    std::memcpy(tab.data() + order_at, order.data(), size_t(ntot) * 4);
     std::memcpy(tab.data() + rows_at, rows.data(), rows.size() * 4);
     DBuf tabd(&ctx_, tab.size());
     ctx_.h2d(tabd.get(), tab.data(), tab.size());
     const uint32_t *lensd = reinterpret_cast<const uint32_t *>(tabd.as<char>());
+    const uint32_t *orderd = reinterpret_cast<const uint32_t *>(tabd.as<char>() + order_at);
     const int32_t *rowsd = reinterpret_cast<const int32_t *>(tabd.as<char>() + rows_at);
     std::vector<Graph::Out> trunks;
     // A stage boundary also in the middle of the trunk (its five layers carry similar work), so a
@@ -320,7 +338,7 @@ void Recognizer::recognize_device(const Batch *batches, int count, float *logits
         conv_mfma(ca, st);
         fork();
         if (L.r32) gru_recurrence_f32(G.as<float>(), L.r32, L.rb, Y[l].as<float>(), lensd, ntot, steps, gs);
-        else gru_recurrence(G.as<float>(), L.r, L.rb, Y[l].as<float>(), lensd, ntot, tmax, steps, gs);
+        else gru_recurrence(G.as<float>(), L.r, L.rb, Y[l].as<float>(), lensd, orderd, gru_lines(ntot), ntot, steps, gs);
         if (gs != st && l == 0) {
             OCR_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
             OCR_HIP(hipEventRecord(join, gs));

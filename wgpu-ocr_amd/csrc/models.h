@@ -52,8 +52,8 @@ class Recognizer {
     // layer and the arg-max): each recurrence waits for its input projection on the context's
     // stream, which waits for the first only before the second projection and returns without
     // waiting for the second. What the caller queues meanwhile (from between(), or its next
-    // pass's trunk) runs beside the recurrence, whose workgroups occupy one CU per 8 lines and
-    // direction. logits and best are then written in gru_stream's order: the caller orders its
+    // pass's trunk) runs beside the recurrence, whose workgroups occupy one CU per 2 or 4
+    // lines (gru_lines) and direction. logits and best are then written in gru_stream's order: the caller orders its
     // reads after that stream and marks the buffers as used on it.
     void recognize_device(const Batch *batches, int count, float *logits, uint32_t *best, uint32_t *lens,
                           const std::function<void()> &between = {}, hipStream_t gru_stream = nullptr);
@@ -65,10 +65,10 @@ class Recognizer {
     struct Layer {
         ConvPack pk;  // the input projection as a 1 x 1 convolution: [1536][input]
         const uint16_t *w_hi = nullptr, *w_lo = nullptr, *w_frag = nullptr;
-        const float *wb = nullptr;  // [2][768]
-        const uint16_t *r = nullptr;  // [2][768][256] float16
+        const float *wb = nullptr;  // [2][768]: Wb, and Rb of the update and reset gates if R is float16
+        const uint16_t *r = nullptr;  // R float16, packed by gru_pack_r
         const float *r32 = nullptr;   // [2][256][768] float32 (R transposed), when R stays float32
-        const float *rb = nullptr;    // [2][768]
+        const float *rb = nullptr;    // [2][256]: the candidate's Rb ([2][768], every gate's, for r32)
         int input = 0;
     };
     Ctx &ctx_;

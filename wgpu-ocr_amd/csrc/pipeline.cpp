@@ -77,8 +77,7 @@ struct Pipeline::Impl {
     // both.
     hipStream_t copy = nullptr;
     // The recurrences of a recognition pass run on a stream of their own when pages come from host
-    // memory: a recurrence occupies one CU per 8 lines and direction (a third to a half of the GPU
-    // at the bench's passes), and the detection groups queued between the pass's stages run on
+    // memory: a recurrence occupies one CU per 2 or 4 lines and direction, and the detection groups queued between the pass's stages run on
     // the rest of the CUs meanwhile.
     hipStream_t gru = nullptr;
     PageUploader upl;
