@@ -113,6 +113,37 @@ def test_conv1x1_inexact_weights(ctx, tmp_path, cin, cout, h, w, fam):
     assert calls[fam] >= 1 and calls["conv_mfma"] == 0, calls
 
 
+@pytest.mark.parametrize("cout,pool,h,w", [(16, None, 3, 1), (32, (2, 2), 64, 37), (64, (2, 2), 50, 131), (48, None, 17, 65)])
+def test_direct_conv_inexact_weights(ctx, tmp_path, cout, pool, h, w):
+    # One-channel 3 x 3 convs with float32 weights that are not float16 values (their remainders
+    # go through the matrix cores too), at tile edges. check's bound is that of every split conv:
+    # the parts stand for the weights to 2^-23 of the channel's largest.
+    def net(g, x):
+        y = conv(g, x, 1, cout, exact=False, act="Relu")
+        return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
+    p = build(tmp_path, "d1i", net, (2, 1, h, w))
+    check(ctx, p, RNG.uniform(-0.5, 0.5, (2, 1, h, w)).astype(np.float32))
+
+
+@pytest.mark.parametrize("scale,small", [(1e6, 1), (1e-4, 1), (1, 1e-3), (1, 1e-7)])
+def test_direct_conv_weight_ranges(ctx, tmp_path, scale, small):
+    # Weights far from 1 are scaled before they are split; a channel far below the others (the
+    # last) keeps the layer on the float32 kernel. Compared relative to each channel's largest
+    # output: 9 products, each to 2^-21 of the largest weight and input.
+    w = (RNG.standard_normal((16, 1, 3, 3)) * scale).astype(np.float32)
+    w[3] *= np.float32(small)
+    def net(g, x):
+        return g.add("Conv", [x, g.init("ws", w)], kernel_shape=[3, 3], pads=[1, 1, 1, 1], strides=[1, 1])
+    import ocrhip
+    p = build(tmp_path, "d1s", net, (1, 1, 20, 33))
+    x = RNG.uniform(-0.5, 0.5, (1, 1, 20, 33)).astype(np.float32)
+    got = ocrhip.Graph(ctx, p).run(x)
+    xp = np.pad(x[0, 0].astype(np.float64), 1)
+    want = sum(w[:, 0, i, j, None, None].astype(np.float64) * xp[i: i + 20, j: j + 33] for i in range(3) for j in range(3))
+    top = np.abs(w).reshape(16, -1).max(1)[:, None, None] * 0.5
+    assert (np.abs(got[0] - want) <= 9 * 2.0 ** -21 * top).all()
+
+
 def test_conv_asymmetric_pads(ctx, tmp_path):
     p = build(tmp_path, "ca", lambda g, x: conv(g, x, 8, 12, k=(3, 2), pads=(0, 1, 2, 0)), (1, 8, 9, 10))
     check(ctx, p, RNG.standard_normal((1, 8, 9, 10)).astype(np.float32))
