@@ -61,6 +61,19 @@ def test_conv1x1_gemm(ctx, tmp_path, cin, cout, h, w, act):
     check(ctx, p, RNG.standard_normal((1, cin, h, w)).astype(np.float32))
 
 
+@pytest.mark.parametrize("cin,cout,w,act", [(512, 97, 1, None), (256, 97, 50, "Relu"), (512, 97, 5003, None),
+                                            (132, 40, 30001, "Sigmoid"), (132, 150, 12003, None), (512, 1536, 321, None),
+                                            (128, 272, 82001, "Relu"), (256, 64, 1537, None)])
+def test_conv1x1_row_counts(ctx, tmp_path, cin, cout, w, act):
+    # The GEMM's three forms at the edges of their tiles: one row, few rows (16 x 16), 128 and 64
+    # row tiles with a part of a tile left, K and N that end inside a slice or tile, and enough
+    # 256 x 256 tiles for the persistent form.
+    p = build(tmp_path, "g1r", lambda g, x: conv(g, x, cin, cout, k=(1, 1), pads=(0, 0, 0, 0), act=act), (1, cin, 1, w))
+    x = RNG.standard_normal((1, cin, 1, w)).astype(np.float32)
+    _, calls = _ran(FAST, lambda: check(ctx, p, x))
+    assert calls["gemm_dma"] >= 1, calls
+
+
 def test_conv1x1_and_sigmoid(ctx, tmp_path):
     p = build(tmp_path, "c1", lambda g, x: conv(g, x, 16, 3, k=(1, 1), pads=(0, 0, 0, 0), act="Sigmoid"), (1, 16, 7, 130))
     check(ctx, p, RNG.standard_normal((1, 16, 7, 130)).astype(np.float32))

@@ -11,16 +11,36 @@
 //
 // Roles: the weights are the MFMA's A operand and the activations its B operand, so a lane's four
 // accumulators are four neighbouring output channels of one row and leave as one 16-byte store.
+// Every output is the sum over the K chunks in order, hi before lo, in all three kernels: a row's
+// result does not depend on how many rows a call has.
 //
-// Pipeline (one 32-wide K chunk a stage, three LDS stages): between the MFMAs of stage s the
-// weights of chunk s + 2 arrive by LDS DMA (lane-ordered fragments copied as they are), the
-// float32 activations of chunk s + 2 (loaded during stage s - 1) are split into hi / lo and
-// written to LDS, those of chunk s + 3 are loaded into registers, and in the last step the
-// fragments of chunk s + 1 are read into registers, so the next stage starts on the matrix cores
-// right after the barrier.
-// A workgroup (8 wavefronts, 256 rows x 32 NT columns) is persistent: it keeps one block of
-// output channels (its bias and the row map of its tiles sit in LDS) and walks a contiguous run of
-// row tiles with the pipeline running on across tile boundaries.
+// gemm_dma, for calls of many rows and columns. Pipeline (one 32-wide K chunk a stage, three LDS
+// stages): between the MFMAs of stage s the weights of chunk s + 2 arrive by LDS DMA
+// (lane-ordered fragments copied as they are), the float32 activations of chunk s + 2 (loaded
+// during stage s - 1) are split into hi / lo and written to LDS, those of chunk s + 3 are loaded
+// into registers, and in the last step the fragments of chunk s + 1 are read into registers, so
+// the next stage starts on the matrix cores right after the barrier. A workgroup (8 wavefronts,
+// 256 rows x 256 columns) is persistent: it keeps one block of output channels (its bias and the
+// row map of its tiles sit in LDS) and walks a contiguous run of row tiles with the pipeline
+// running on across tile boundaries, so a tile's stores drain under the next tile's MFMAs: at
+// 71 700 rows x 1536 the stores alone (440 MB) are over half the call.
+//
+// gemm_tile, for the sizes between: a wavefront makes 64 rows x 16 NT columns, 4 of them side by
+// side share the rows. The activations of a chunk are split once for the workgroup into one of
+// two LDS stages; a wavefront's weights are its own, so they come from L2 straight into registers.
+// Chunk s + 2's activations and chunk s + 1's weights are in flight under chunk s's MFMAs, one
+// LDS-only barrier a chunk, and several workgroups a CU cover each other's start and end. Column
+// blocks of the same rows are numbered next to each other on one XCD: its L2 holds the rows they
+// share. 4500 rows (36 lines) x 1536: 28.9 -> 17.0 us for K = 256, 41.0 -> 24.8 for K = 512,
+// against gemm_dma, whose 108 tiles of 256 x 256 leave over half the CUs idle and each a start
+// and an end that nothing covers. Without the stores it would take 11.5 and 19.4. With at most
+// 128 columns two such groups stand on each other (128 rows x 128 columns, 8 wavefronts): the
+// output layer of a 36-line pass 29 -> 16 us, of a 540-line pass 72 -> 56.
+//
+// gemm_thin, for few rows: a wavefront makes 16 rows x 16 columns with its operands read straight
+// from memory, 8 K chunks of them at once and the next 8 in flight. Such calls are one latency
+// after another (row map, operands, output), and this form has the fewest of them: 50 rows x 1536
+// 18 -> 5 us for K = 256, 30 -> 8 for K = 512.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,11 +57,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int GBM = 256;        // rows per tile
-constexpr int RSU = 9;          // LDS units (16 bytes) per row: 4 hi, 4 lo, 1 of padding
-constexpr int ASU = GBM * RSU;  // activation stage size in units
-
-
+constexpr int RSU = 9;  // LDS units (16 bytes) per row: 4 hi, 4 lo, 1 of padding
 
 struct GParams {
     const float *x;
@@ -56,15 +72,14 @@ struct GParams {
     const half8 *wt;  // fragments [n-tile][chunk][64 lanes] of 8 halves
     int ntiles;
     const float *bias;
-    int act;
     int mtiles, nblocks, runs;
     int vec;            // 16-byte output stores (N and the row stride multiples of 4, y aligned)
     const float *zero;  // 64 zero bytes
 };
 
-__device__ inline float gact(float v, int act) {
-    if (act == ACT_RELU) return fmaxf(v, 0.f);
-    if (act == ACT_SIGMOID) return 1.f / (1.f + expf(-v));
+template <int ACT> __device__ inline float gact(float v) {
+    if (ACT == ACT_RELU) return fmaxf(v, 0.f);
+    if (ACT == ACT_SIGMOID) return 1.f / (1.f + expf(-v));
     return v;
 }
 
@@ -73,9 +88,58 @@ __device__ inline int gxcd_index(int b, int G) {
     return x * q + min(x, rem) + (b >> 3);
 }
 
-template <int NT, int ACT>
+// Floats 8 q .. 8 q + 7 of chunk c of a row of x (zeros past K).
+__device__ inline void load_x(const GParams &p, const float *xr, int c, int q, float4 (&v)[2]) {
+    const int k0 = (c >= p.xchunks ? c - p.xchunks : c) * 32 + 8 * q;
+#pragma unroll
+    for (int e = 0; e < 2; e++)
+        v[e] = *reinterpret_cast<const float4 *>(k0 + 4 * e < p.K ? xr + k0 + 4 * e : p.zero);
+}
+
+__device__ inline void split(const float4 (&v)[2], half8 &hi, half8 &lo) {
+    const float xs[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)xs[e];
+        lo[e] = (_Float16)(xs[e] - (float)hi[e]);
+    }
+}
+
+// Columns n .. n + 3 of a row (row m of the GEMM). STREAM: stored past L2, for outputs larger
+// than it (4500 x 1536: 21.3 -> 17.0 us).
+template <int ACT, bool STREAM>
+__device__ inline void put(const GParams &p, int m, int row, int n, const floatx4 &acc, const float4 &b4) {
+    if (m >= p.M || n >= p.N) return;
+    const floatx4 o = {gact<ACT>(acc[0] + b4.x), gact<ACT>(acc[1] + b4.y), gact<ACT>(acc[2] + b4.z), gact<ACT>(acc[3] + b4.w)};
+    float *yr = p.y + size_t(row) * p.ycs + n;
+    if (p.vec) {
+        if (STREAM) __builtin_nontemporal_store(o, reinterpret_cast<floatx4 *>(yr));
+        else *reinterpret_cast<floatx4 *>(yr) = o;
+    } else {
+        yr[0] = o[0];
+        if (n + 1 < p.N) yr[1] = o[1];
+        if (n + 2 < p.N) yr[2] = o[2];
+        if (n + 3 < p.N) yr[3] = o[3];
+    }
+}
+
+__device__ inline float4 bias4(const GParams &p, int n) {
+    float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!p.bias) return b;
+    if (n < p.N) b.x = p.bias[n];
+    if (n + 1 < p.N) b.y = p.bias[n + 1];
+    if (n + 2 < p.N) b.z = p.bias[n + 2];
+    if (n + 3 < p.N) b.w = p.bias[n + 3];
+    return b;
+}
+
+// ---- gemm_dma ---------------------------------------------------------------------------------
+constexpr int GBM = 256;        // rows per tile
+constexpr int ASU = GBM * RSU;  // activation stage size in units
+
+template <int ACT>
 __global__ __launch_bounds__(512, 1) void gemm_dma_kernel(GParams p) {
-    constexpr int WM = 4, WN = 2, MT = 4, NTW = NT * WN;
+    constexpr int NT = 8, WM = 4, WN = 2, MT = 4, NTW = NT * WN;
     constexpr int NWI = (NTW + 7) / 8;  // weight DMA instructions per wavefront and chunk
     __shared__ __align__(16) half8 AS0[ASU];
     __shared__ __align__(16) half8 AS1[ASU];
@@ -206,10 +270,10 @@ __global__ __launch_bounds__(512, 1) void gemm_dma_kernel(GParams p) {
             for (int j = 0; j < NT; j++) {
                 const float4 b4 = *reinterpret_cast<const float4 *>(&BIAS[(wn * NT + j) * 16 + 4 * g]);
                 float4 o;
-                o.x = gact(acc[mt][j][0] + b4.x, ACT);
-                o.y = gact(acc[mt][j][1] + b4.y, ACT);
-                o.z = gact(acc[mt][j][2] + b4.z, ACT);
-                o.w = gact(acc[mt][j][3] + b4.w, ACT);
+                o.x = gact<ACT>(acc[mt][j][0] + b4.x);
+                o.y = gact<ACT>(acc[mt][j][1] + b4.y);
+                o.z = gact<ACT>(acc[mt][j][2] + b4.z);
+                o.w = gact<ACT>(acc[mt][j][3] + b4.w);
                 acc[mt][j] = floatx4{0.f, 0.f, 0.f, 0.f};
                 const int n = n_w + 16 * j;
                 if (orow[mt] < 0 || n >= p.N) continue;
@@ -314,6 +378,146 @@ __global__ __launch_bounds__(512, 1) void gemm_dma_kernel(GParams p) {
     if (pend) epilogue();
 }
 
+// ---- gemm_tile --------------------------------------------------------------------------------
+constexpr int MT = 4;  // 16-row tiles of a wavefront
+
+// 4 wavefronts side by side, WM such rows of wavefronts.
+template <int WM, int NT, int ACT>
+__global__ __launch_bounds__(256 * WM, NT == 4 ? 3 : 4) void gemm_tile_kernel(GParams p) {
+    constexpr int TBM = WM * MT * 16, THREADS = 256 * WM;
+    __shared__ __align__(16) half8 AS[2][TBM * RSU];
+    __shared__ __align__(16) float BIAS[4 * NT * 16];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wid & 3, wm = wid >> 2;
+    const int g = lane >> 4, r = lane & 15;
+    const int v = gxcd_index(blockIdx.x, gridDim.x);
+    const int nb = v % p.nblocks, m0 = v / p.nblocks * TBM;
+    const int nt0 = (nb * 4 + wave) * NT;
+    auto row_at = [&](int m) __attribute__((always_inline)) {
+        m = min(m, p.M - 1);
+        return p.rows ? p.rows[m] : m;
+    };
+    // Loader role: row lr of the tile, floats 8 lq .. 8 lq + 7 of a chunk.
+    const int lr = tid >> 2, lq = tid & 3;
+    const float *const xr = p.x + size_t(row_at(m0 + lr)) * p.xcs;
+    int orow[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) orow[mt] = row_at(m0 + (wm * MT + mt) * 16 + r);
+    for (int i = tid; i < 4 * NT * 16; i += THREADS) {
+        const int n = nb * (4 * NT * 16) + i;
+        BIAS[i] = p.bias && n < p.N ? p.bias[n] : 0.f;
+    }
+    auto stash = [&](const float4 (&x)[2], int st) __attribute__((always_inline)) {
+        half8 hi, lo;
+        split(x, hi, lo);
+        AS[st][lr * RSU + lq] = hi;
+        AS[st][lr * RSU + lq + 4] = lo;
+    };
+    // Weights of chunk c (tiles past the last read the last one again; their columns are not
+    // stored).
+    const half8 *wp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) wp[j] = p.wt + size_t(min(nt0 + j, p.ntiles - 1)) * p.chunks * 64 + lane;
+    auto load_w = [&](half8 (&w)[NT], int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NT; j++) w[j] = wp[j][c * 64];
+    };
+
+    float4 xa[2], xb[2];
+    half8 wa[NT], wb[NT];
+    const int last = p.chunks - 1;
+    load_x(p, xr, 0, lq, xa);
+    load_w(wa, 0);
+    load_x(p, xr, min(1, last), lq, xb);
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[mt][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    stash(xa, 0);
+    lds_barrier();
+
+    // Chunk c in LDS stage st: xc takes chunk c + 2, xn holds chunk c + 1, wc the weights, wn
+    // takes the next ones (past the last chunk the last is loaded again and not used).
+    auto stage = [&](int c, int st, float4 (&xc)[2], const float4 (&xn)[2], const half8 (&wc)[NT],
+                     half8 (&wn)[NT]) __attribute__((always_inline)) {
+        load_w(wn, min(c + 1, last));
+        load_x(p, xr, min(c + 2, last), lq, xc);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const int u = ((wm * MT + mt) * 16 + r) * RSU + g;
+            const half8 ah = AS[st][u], al = AS[st][u + 4];
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wc[j], ah, acc[mt][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wc[j], al, acc[mt][j], 0, 0, 0);
+        }
+        if (c < last) {
+            stash(xn, st ^ 1);
+            lds_barrier();
+        }
+    };
+    for (int c = 0; c <= last; c += 2) {
+        stage(c, 0, xa, xb, wa, wb);
+        if (c < last) stage(c + 1, 1, xb, xa, wb, wa);
+    }
+    float4 b4[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) b4[j] = *reinterpret_cast<const float4 *>(&BIAS[(wave * NT + j) * 16 + 4 * g]);
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+            put<ACT, NT == 4>(p, m0 + (wm * MT + mt) * 16 + r, orow[mt], (nt0 + j) * 16 + 4 * g, acc[mt][j], b4[j]);
+}
+
+template <int ACT>
+__global__ __launch_bounds__(256, 2) void gemm_thin_kernel(GParams p) {
+    constexpr int KB = 8;  // chunks asked for at once
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const int wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rt = wid / p.ntiles, nt = wid - rt * p.ntiles, m = rt * 16 + r;
+    if (rt * 16 >= p.M) return;
+    const int row = p.rows ? p.rows[min(m, p.M - 1)] : min(m, p.M - 1);
+    const half8 *wp = p.wt + size_t(nt) * p.chunks * 64 + lane;
+    const float *xr = p.x + size_t(row) * p.xcs;
+    const int n = nt * 16 + 4 * g, last = p.chunks - 1;
+    struct Batch {
+        float4 x[KB][2];
+        half8 w[KB];
+    } b0, b1;
+    // Chunks c0 .. c0 + KB - 1 (the last again past the end).
+    auto load = [&](Batch &b, int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < KB; c++) {
+            b.w[c] = wp[min(c0 + c, last) * 64];
+            load_x(p, xr, min(c0 + c, last), g, b.x[c]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Batch &b, int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < KB; c++) {
+            if (c0 + c > last) break;
+            half8 hi, lo;
+            split(b.x[c], hi, lo);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b.w[c], hi, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b.w[c], lo, acc, 0, 0, 0);
+        }
+    };
+    const float4 b4 = bias4(p, n);
+    load(b0, 0);
+    for (int c = 0; c <= last; c += 2 * KB) {
+        if (c + KB <= last) load(b1, c + KB);
+        compute(b0, c);
+        if (c + 2 * KB <= last) load(b0, c + 2 * KB);
+        compute(b1, c + KB);
+    }
+    put<ACT, false>(p, m, row, n, acc, b4);
+}
+
 int gcu_count() {
     static int n = 0;
     if (!n) {
@@ -324,6 +528,16 @@ int gcu_count() {
     }
     return n;
 }
+
+// Calls of at most this many 16 x 16 x 32 blocks take gemm_thin. At the line both forms take
+// about the same: 1536 columns, K = 256: 400 rows (19 200) 12.3 us against gemm_tile's 14.4, 800
+// rows 16.7 against 14.7; K = 512: 200 rows (20 000) 14.2 against 17.7, 400 rows 20.8 against 17.3;
+// 97 columns, K = 512: 1600 rows (11 200) 8 against 14, 4500 rows (31 600) 17 against 13.
+constexpr double THIN_BLOCKS = 20000;
+// Calls of at least this many 256 x 256 tiles take gemm_dma (two and a half a CU): 30 000 rows x
+// 1536 (708 tiles) 81 and 123 us for K = 256 and 512 against gemm_tile's 96 and 130, 71 700 rows
+// 176 and 275 against 223 and 310; 16 000 rows (378) 59 and 81 for gemm_tile.
+constexpr double BIG_TILES = 640;
 
 const float *gzero() { return static_cast<const float *>(zero_block64()); }
 
@@ -338,10 +552,9 @@ bool gemm_dma(const ConvArgs &a, hipStream_t s) {
     if (a.act != ACT_NONE && a.act != ACT_RELU && a.act != ACT_SIGMOID) return false;
     if (a.rows && (a.x.n != 1 || a.x.h != 1)) return false;
     const int K = a.x.c, N = a.y.c;
-    // Four or more K chunks: the row map of a tile stays in LDS until its epilogue.
     if (K % 4 || a.x.cs % 4 || (reinterpret_cast<uintptr_t>(a.x.p) & 15) || pk.frag_chunks() < 4 || N < 1) return false;
     const double m = double(a.x.n) * a.x.h * a.x.w;
-    if (m >= 2147483647.0 - GBM) return false;
+    if (m >= 2147483647.0 - 2 * GBM) return false;
     GParams p{};
     p.x = a.x.p;
     p.xcs = a.x.cs;
@@ -356,22 +569,36 @@ bool gemm_dma(const ConvArgs &a, hipStream_t s) {
     p.wt = reinterpret_cast<const half8 *>(a.wt_frag);
     p.ntiles = pk.nblocks * pk.bn / 16;
     p.bias = a.bias;
-    p.act = a.act;
-    const int nt = N > 128 ? 8 : 4, bn = 32 * nt;
-    p.mtiles = (p.M + GBM - 1) / GBM;
-    p.nblocks = (N + bn - 1) / bn;
-    p.runs = std::max(1, std::min(p.mtiles, gcu_count() / p.nblocks));
     p.vec = (N % 4 == 0 && a.y.cs % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y.p) & 15) == 0) ? 1 : 0;
     p.zero = gzero();
     if (p.M == 0) return true;
-    const int grid = p.runs * p.nblocks;
+    const double thin = std::ceil(p.M / 16.0) * p.ntiles;
+    const double big = std::ceil(p.M / double(GBM)) * std::ceil(N / 256.0);
+    const bool few = thin * p.chunks <= THIN_BLOCKS, many = N > 128 && big >= BIG_TILES;
+    const bool narrow = p.ntiles <= 8;
+    double blocks;
+    if (few) {
+        blocks = std::ceil(thin / 4);
+    } else if (many) {
+        p.mtiles = (p.M + GBM - 1) / GBM;
+        p.nblocks = (N + 255) / 256;
+        p.runs = std::max(1, std::min(p.mtiles, gcu_count() / p.nblocks));
+        blocks = double(p.runs) * p.nblocks;
+    } else {
+        p.nblocks = (p.ntiles + (narrow ? 7 : 15)) / (narrow ? 8 : 16);
+        blocks = std::ceil(p.M / (narrow ? 128.0 : 64.0)) * p.nblocks;
+    }
+    if (blocks > 2147483647.0) return false;
+    const dim3 grid{unsigned(blocks)};
     const double flops = 2.0 * p.M * double(N) * K;
     const double bytes = 4.0 * (double(p.M) * K + double(p.M) * N) + 2.0 * double(pk.frag_halves());
     ProbeScope probe("gemm_dma", s, flops, bytes);
     auto launch = [&](auto ACTc) {
         constexpr int A = decltype(ACTc)::value;
-        if (nt == 8) hipLaunchKernelGGL((gemm_dma_kernel<8, A>), dim3(unsigned(grid)), dim3(512), 0, s, p);
-        else hipLaunchKernelGGL((gemm_dma_kernel<4, A>), dim3(unsigned(grid)), dim3(512), 0, s, p);
+        if (few) hipLaunchKernelGGL((gemm_thin_kernel<A>), grid, dim3(256), 0, s, p);
+        else if (many) hipLaunchKernelGGL((gemm_dma_kernel<A>), grid, dim3(512), 0, s, p);
+        else if (narrow) hipLaunchKernelGGL((gemm_tile_kernel<2, 2, A>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((gemm_tile_kernel<1, 4, A>), grid, dim3(256), 0, s, p);
     };
     if (a.act == ACT_RELU) launch(std::integral_constant<int, ACT_RELU>{});
     else if (a.act == ACT_SIGMOID) launch(std::integral_constant<int, ACT_SIGMOID>{});
