@@ -345,6 +345,56 @@ def test_fused_attention_shapes(ctx, tmp_path, n, t, dim, heads):
     check(ctx, p, RNG.standard_normal((n, t, dim)).astype(np.float32))
 
 
+def _layer_norm(g, x, k):
+    b = synth_pp._B("ln", 3)
+    b.g = g
+    b.rng = RNG
+    return b.layer_norm(x, k)
+
+
+def _linear(g, x, k, n, exact, act=None):
+    y = g.add("MatMul", [x, w(g, (k, n), k, exact)])
+    y = g.add("Add", [y, g.init(g.fresh("lb"), (RNG.standard_normal(n) * 0.1).astype(np.float32))])
+    return g.add("Mul", [y, g.add("Sigmoid", [y])]) if act else y
+
+
+@pytest.mark.parametrize("n,t,dim,heads,hidden,exact", [(1, 1, 120, 8, 240, True), (2, 17, 120, 8, 256, False),
+                                                        (3, 109, 48, 12, 33, True), (2, 200, 128, 8, 100, False),
+                                                        (1, 33, 36, 9, 16, True), (2, 40, 132, 11, 300, True)])
+def test_transformer_block_shapes(ctx, tmp_path, n, t, dim, heads, hidden, exact):
+    # A block whose parts run joined (normalised QKV, attention with its projection, the MLP): rows
+    # and keys at the edges of 16 and 32, heads of 4, 15 and 16 values and more heads than a
+    # workgroup has wavefronts, hidden sizes up to the joined kernel's most; the last case is too
+    # wide for it and runs in parts.
+    def fn(g, x):
+        x = g.add("Add", [x, _linear(g, _attention(g, _layer_norm(g, x, dim), dim, heads), dim, dim, exact)])
+        y = _linear(g, _layer_norm(g, x, dim), dim, hidden, exact, act=True)
+        x = g.add("Add", [x, _linear(g, y, hidden, dim, exact)])
+        return g.add("Sqrt", [g.add("Relu", [x])])
+    p = build(tmp_path, "block", fn, (n, t, dim))
+    check(ctx, p, RNG.standard_normal((n, t, dim)).astype(np.float32))
+
+
+def test_output_memory(ctx, tmp_path):
+    # The last step writes the caller's memory; where that is unaligned or the input itself, the
+    # output still arrives whole.
+    import ctypes
+    import ocrhip
+    p = build(tmp_path, "om", lambda g, x: g.add("MatMul", [x, w(g, (64, 64), 64)]), (3, 5, 64))
+    x = RNG.standard_normal((3, 5, 64)).astype(np.float32)
+    graph, lib = ocrhip.NdGraph(ctx, p), ocrhip.lib()
+    want = graph.run(x)
+    shape = (ctypes.c_int64 * 3)(*x.shape)
+    buf = ocrhip.DeviceBuffer(ctx, 4 * x.size + 8192)
+    for off_in, off_out in ((0, 4096), (0, 4100), (0, 0), (16, 20)):
+        assert lib.ocr_memcpy_h2d(ctx.handle, buf.ptr + off_in, x.ctypes.data, x.nbytes) == 0
+        assert lib.ocr_nd_run_device(graph.handle, buf.ptr + off_in, shape, 3, buf.ptr + off_out) == 0
+        got = np.empty_like(want)
+        assert lib.ocr_memcpy_d2h(ctx.handle, got.ctypes.data, buf.ptr + off_out, got.nbytes) == 0
+        assert np.array_equal(got, want), (off_in, off_out)
+    buf.free()
+
+
 def test_unsupported_and_bad_shapes_raise(ctx, tmp_path):
     import ocrhip
     p = build(tmp_path, "bad", lambda g, x: g.add("Tanh", [x]), (1, 4))

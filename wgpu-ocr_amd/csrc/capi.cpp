@@ -839,8 +839,9 @@ int ocr_nd_run_device(ocr_nd *g, const float *d_in, const int64_t *in_shape, uin
         NdTensor x;
         x.p = const_cast<float *>(d_in);
         x.shape = shape_in(in_shape, rank);
-        NdTensor y = g->graph.run(c, x);
-        OCR_HIP(hipMemcpyAsync(d_out, y.p, y.count() * sizeof(float), hipMemcpyDeviceToDevice, c.stream()));
+        NdTensor y = g->graph.run(c, x, d_out);
+        if (y.p != d_out)
+            OCR_HIP(hipMemcpyAsync(d_out, y.p, y.count() * sizeof(float), hipMemcpyDeviceToDevice, c.stream()));
     });
 }
 

@@ -1,6 +1,7 @@
 // Multi-head self-attention of the N-D executor in one launch: the exporter's chain from the
 // fused QKV projection (reshape, transpose, slice q / k / v, scale q, q k^T, softmax over the last
-// axis, times v, transpose, reshape; src/nd.rs:291-391 runs it as separate programs) on gfx950.
+// axis, times v, transpose, reshape; src/nd.rs:291-391 runs it as separate programs) on gfx950,
+// for heads of under 4 or over 16 values (the others run on the matrix cores, ndblock.hip).
 //
 // x is [n][T][3 H d] (q, then k, then v, each H heads of d values), y is [n][T][H d]. A workgroup
 // takes 32 queries of one head of one image; eight lanes share a query, each walking every eighth
@@ -105,13 +106,13 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
 
 void nd_attention(const float *x, int n, int t, int heads, int d, float scale, float *y, hipStream_t s) {
     if (n <= 0 || t <= 0) return;
+    if (nd_attention_mfma(x, n, t, heads, d, scale, y, s)) return;
     if (d <= 0 || d > 64) fail("nd_attention: " + std::to_string(d) + " values a head (at most 64)");
     AttnParams p{x, y, n, t, heads, d, scale};
     const dim3 grid{unsigned((t + 31) / 32), unsigned(heads), unsigned(n)};
     const double tt = double(t);
     ProbeScope probe("nd_attention", s, 4.0 * n * heads * tt * tt * d, 4.0 * n * tt * (3.0 * heads * d + heads * d));
-    if (d <= 16) hipLaunchKernelGGL((attention_kernel<16, 256>), grid, dim3(256), 0, s, p);
-    else if (d <= 32) hipLaunchKernelGGL((attention_kernel<32, 256>), grid, dim3(256), 0, s, p);
+    if (d <= 32) hipLaunchKernelGGL((attention_kernel<32, 256>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((attention_kernel<64, 128>), grid, dim3(256), 0, s, p);
     OCR_HIP(hipGetLastError());
 }

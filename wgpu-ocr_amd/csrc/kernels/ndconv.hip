@@ -31,30 +31,11 @@
 #include "../kernels.h"
 #include "../nd_kernels.h"
 #include "../runtime.h"
+#include "nd_device.h"
 
 namespace ocr {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
 namespace {
-
-__device__ inline float act_dev(float v, int act) {
-    if (act == ACT_RELU) return fmaxf(v, 0.f);
-    if (act == ACT_SIGMOID) return 1.f / (1.f + expf(-v));
-    if (act == ACT_GELU) return 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
-    if (act == ACT_SILU) return v / (1.f + expf(-v));
-    return v;
-}
-
-__device__ inline void split8(const float (&v)[8], half8 &hi, half8 &lo) {
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const _Float16 h = (_Float16)v[j];
-        hi[j] = h;
-        lo[j] = (_Float16)(v[j] - (float)h);
-    }
-}
 
 // ---- conv_nchw -------------------------------------------------------------------------------
 struct NchwParams {
@@ -420,14 +401,7 @@ struct RowsParams {
 // The B operand of one 16-row tile: rows r0 + r, inputs c0 + 8g .. c0 + 8g + 7, split hi / lo.
 __device__ inline void rows_frag(const RowsParams &p, int row, int c0, half8 &hi, half8 &lo) {
     float v[8];
-    if (row < p.m && p.vec && c0 + 8 <= p.k) {
-        const float4 *src = reinterpret_cast<const float4 *>(p.x + size_t(row) * p.k + c0);
-        const float4 q0 = src[0], q1 = src[1];
-        v[0] = q0.x, v[1] = q0.y, v[2] = q0.z, v[3] = q0.w, v[4] = q1.x, v[5] = q1.y, v[6] = q1.z, v[7] = q1.w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = (row < p.m && c0 + j < p.k) ? p.x[size_t(row) * p.k + c0 + j] : 0.f;
-    }
+    row_chunk(p.x, row, p.m, p.k, c0, p.vec, v);
     split8(v, hi, lo);
 }
 
@@ -766,6 +740,7 @@ bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s) {
     if (pk.kh != 1 || pk.kw != 1 || pk.cin != a.k || pk.cout != a.n || !a.wt_hi) return false;
     if (!pk.exact && !a.wt_lo) return false;
     if (pk.bn != 16 && pk.bn != 32 && pk.bn != 64) return false;
+    if (a.gb) return false;
     if (a.m <= 0) return true;
     if (pk.nblocks > 65535) return false;
     RowsParams p = rows_params(a);
@@ -816,7 +791,7 @@ bool nd_head_argmax(const NdRowsArgs &a, float *part, int parts, hipStream_t s) 
     const ConvPack &pk = a.pk;
     if (pk.kh != 1 || pk.kw != 1 || pk.cin != a.k || pk.cout != a.n || pk.bn != 64 || !a.wt_hi) return false;
     if (!pk.exact && !a.wt_lo) return false;
-    if (pk.chunks > 8 || a.res || a.act != ACT_NONE) return false;
+    if (pk.chunks > 8 || a.res || a.gb || a.act != ACT_NONE) return false;
     if (a.m <= 0) return true;
     RowsParams p = rows_params(a);
     p.amax = reinterpret_cast<float2 *>(part);

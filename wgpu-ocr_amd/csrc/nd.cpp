@@ -127,6 +127,11 @@ NdGraph NdGraph::build(Ctx &ctx, const Onnx &onnx, bool stop_before_softmax) {
             gb.insert(gb.end(), bt.data.begin(), bt.data.end());
             op.gb = ctx.upload_weights(gb.data(), gb.size());
             op.len = int(gm.data.size());
+            const size_t pad = (gm.data.size() + 31) / 32 * 32;
+            std::vector<float> padded(2 * pad, 0.f);
+            std::copy(gm.data.begin(), gm.data.end(), padded.begin());
+            std::copy(bt.data.begin(), bt.data.end(), padded.begin() + long(pad));
+            op.gb32 = ctx.upload_weights(padded.data(), padded.size());
             op.eps = s.eps;
             op.inputs = {n.inputs.at(0)};
             break;
@@ -232,12 +237,67 @@ NdGraph NdGraph::build(Ctx &ctx, const Onnx &onnx, bool stop_before_softmax) {
     g.nodes_ = std::move(plan.nodes);
     g.input = plan.input;
     g.output = plan.output;
+    g.join_ops();
     for (size_t k = 0; k < g.ops.size(); k++) {
         for (const auto &nm : g.ops[k].inputs) g.last_use_[nm] = k;
         if (!g.ops[k].residual.empty()) g.last_use_[g.ops[k].residual] = k;
         if (!g.ops[k].in_scale.empty()) g.last_use_[g.ops[k].in_scale] = k;
     }
     return g;
+}
+
+// Steps of a transformer block that run as one launch: a LayerNorm with the Linear that alone
+// reads it, a Linear with the Linear that alone reads it (an MLP) and an attention with its
+// projection, as far as the kernels hold their rows. A joined step runs at the place of its last
+// part. The graph's last step stays on its own (run_argmax runs a head without its logits).
+void NdGraph::join_ops() {
+    if (no_ndconv()) return;
+    std::map<std::string, int> readers;
+    for (const NdOp &op : ops) {
+        for (const auto &nm : op.inputs) readers[nm]++;
+        readers[op.residual]++;
+        readers[op.in_scale]++;
+    }
+    // The step before k that makes its input 0, when nothing else reads that.
+    auto maker = [&](size_t k) -> int {
+        if (ops[k].inputs.empty()) return -1;
+        const std::string &in = ops[k].inputs[0];
+        if (in == output || readers[in] != 1) return -1;
+        for (size_t j = 0; j < k; j++)
+            if (ops[j].output == in) return int(j);
+        return -1;
+    };
+    auto is_rows = [](const NdOp &op) { return op.kind == NdKind::Linear && op.pk.kh == 1 && op.pk.kw == 1 && !op.then; };
+    std::vector<bool> gone(ops.size(), false);
+    for (size_t k = 0; k + 1 < ops.size(); k++) {
+        if (!is_rows(ops[k])) continue;
+        const int j = maker(k);
+        if (j < 0 || gone[size_t(j)]) continue;
+        NdOp &a = ops[size_t(j)], &b = ops[k];
+        if (a.kind == NdKind::LayerNorm && a.len == b.k && nd_rows_fit(b.pk)) {
+            b.gb32 = a.gb32;
+            b.len = a.len;
+            b.eps = a.eps;
+            b.inputs[0] = a.inputs[0];
+        } else if ((is_rows(a) && a.residual.empty() && a.n == b.k && nd_mlp_fits(a.pk, b.pk)) ||
+                   (a.kind == NdKind::Attention && !a.then)) {
+            NdOp joined = a;
+            joined.then = std::make_shared<NdOp>(b);
+            joined.output = b.output;
+            joined.residual = b.residual;
+            b = std::move(joined);
+        } else {
+            continue;
+        }
+        gone[size_t(j)] = true;
+    }
+    size_t n = 0;
+    for (size_t k = 0; k < ops.size(); k++)
+        if (!gone[k]) {
+            if (n != k) ops[n] = std::move(ops[k]);
+            n++;
+        }
+    ops.resize(n);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -264,7 +324,8 @@ NdValue NdGraph::get(const std::map<std::string, NdValue> &vals, const std::stri
     fail("missing value " + name);
 }
 
-NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std::string, NdValue> *vals_out) const {
+NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std::string, NdValue> *vals_out,
+                          float *dst) const {
     // Without a context only shapes are worked out (no memory, no launches).
     const bool shapes_only = ctx == nullptr;
     const hipStream_t st = shapes_only ? nullptr : ctx->stream();
@@ -272,16 +333,50 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
     NdValue xin;
     xin.t = x;
     vals[input] = xin;
+    size_t oi = 0;
     auto alloc = [&](const std::vector<int64_t> &shape) {
         NdTensor t;
         t.shape = shape;
+        if (dst && ops[oi].output == output) {
+            // The output goes straight to the caller's memory, where that is as aligned as the
+            // pool's is and no part of the input, which other steps may still read.
+            const uintptr_t d0 = reinterpret_cast<uintptr_t>(dst), d1 = d0 + t.count() * sizeof(float);
+            const uintptr_t x0 = reinterpret_cast<uintptr_t>(x.p), x1 = x0 + x.count() * sizeof(float);
+            if (d0 % 16 == 0 && (d1 <= x0 || x1 <= d0)) {
+                t.p = dst;
+                return t;
+            }
+        }
         if (!shapes_only) {
             t.buf = std::make_shared<DBuf>(ctx, std::max<size_t>(t.count(), 1) * sizeof(float));
             t.p = t.buf->as<float>();
         }
         return t;
     };
-    for (size_t oi = 0; oi < nops; oi++) {
+    // The arguments of a Linear of the rows x [m][k], and its residual's shape check.
+    auto rows_args = [&](const NdOp &op, const float *px, size_t m, const std::vector<int64_t> &shape, float *y) {
+        NdRowsArgs ra;
+        if (!op.residual.empty()) {
+            const NdTensor res = get(vals, op.residual).t;
+            if (res.shape != shape)
+                fail("residual " + shape_str(res.shape) + " for a MatMul giving " + shape_str(shape));
+            ra.res = res.p;
+        }
+        ra.x = px;
+        ra.m = int(m);
+        ra.k = op.k;
+        ra.n = op.n;
+        ra.wt_hi = op.whi;
+        ra.wt_lo = op.wlo;
+        ra.pk = op.pk;
+        ra.bias = op.b;
+        ra.y = y;
+        ra.act = op.act;
+        ra.gb = op.gb32;
+        ra.eps = op.eps;
+        return ra;
+    };
+    for (; oi < nops; oi++) {
         const NdOp &op = ops[oi];
         const Node &n = nodes_[size_t(op.node)];
         auto arg = [&](size_t k) { return get(vals, op.inputs.at(k)); };
@@ -404,28 +499,22 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 fail("MatMul: " + shape_str(a.shape) + " by [" + std::to_string(op.k) + ", " + std::to_string(op.n) + "]");
             const size_t m = a.count() / size_t(op.k);
             auto shape = a.shape;
-            shape.back() = op.n;
+            shape.back() = op.then ? op.then->n : op.n;
             out.t = alloc(shape);
             if (shapes_only || m == 0) break;
             if (m > 0x7fffffff) fail("MatMul: too many rows");
-            NdTensor res;
-            if (!op.residual.empty()) {
-                res = get(vals, op.residual).t;
-                if (res.shape != out.t.shape)
-                    fail("residual " + shape_str(res.shape) + " for a MatMul giving " + shape_str(out.t.shape));
+            if (op.then) {
+                NdRowsArgs ra = rows_args(op, a.p, m, shape, nullptr);
+                ra.res = nullptr;
+                const NdRowsArgs rb = rows_args(*op.then, nullptr, m, shape, out.t.p);
+                nd_rows_block(ra, &rb, st);
+                break;
             }
-            NdRowsArgs ra;
-            ra.res = res.p;
-            ra.x = a.p;
-            ra.m = int(m);
-            ra.k = op.k;
-            ra.n = op.n;
-            ra.wt_hi = op.whi;
-            ra.wt_lo = op.wlo;
-            ra.pk = op.pk;
-            ra.bias = op.b;
-            ra.y = out.t.p;
-            ra.act = op.act;
+            const NdRowsArgs ra = rows_args(op, a.p, m, shape, out.t.p);
+            if (ra.gb) {
+                nd_rows_block(ra, nullptr, st);
+                break;
+            }
             if (!no_ndconv() && nd_gemm_rows(ra, st)) break;
             ConvArgs ca;
             ca.x = Act{a.p, 1, 1, int(m), op.k, op.k};
@@ -435,7 +524,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
             ca.bias = op.b;
             ca.act = op.act;
             ca.pk = op.pk;
-            ca.res = res.p;
+            ca.res = ra.res;
             ca.res_cs = op.n;
             conv_mfma(ca, st);
             break;
@@ -472,10 +561,29 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 for (size_t d = 0; d < 3; d++)
                     if (s3[d] == -1) s3[d] = od[d];
             if (s3 != std::vector<int64_t>(od, od + 3)) fail("attention: output reshape to " + shape_str(s3));
-            out.t = alloc({nb, tt, heads * hd});
+            const int64_t od3 = heads * hd;
+            if (op.then && op.then->k != od3)
+                fail("MatMul: " + shape_str({nb, tt, od3}) + " by [" + std::to_string(op.then->k) + ", " +
+                     std::to_string(op.then->n) + "]");
+            const std::vector<int64_t> shape = {nb, tt, op.then ? int64_t(op.then->n) : od3};
+            out.t = alloc(shape);
             if (shapes_only || nb * tt == 0) break;
             if (hd > 64 || nb > 65535 || heads > 65535) fail("attention: heads of " + std::to_string(hd) + " values");
-            nd_attention(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, out.t.p, st);
+            if (!op.then) {
+                nd_attention(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, out.t.p, st);
+                break;
+            }
+            const size_t m = size_t(nb * tt);
+            if (m > 0x7fffffff) fail("MatMul: too many rows");
+            NdRowsArgs ra = rows_args(*op.then, nullptr, m, shape, out.t.p);
+            if (nd_attention_proj_fits(int(heads), int(hd), op.then->pk)) {
+                nd_attention_proj(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, ra, st);
+                break;
+            }
+            const DBuf rows(ctx, m * size_t(od3) * sizeof(float));
+            nd_attention(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, rows.as<float>(), st);
+            ra.x = rows.as<float>();
+            if (!nd_gemm_rows(ra, st)) fail("attention projection: shape");
             break;
         }
         case NdKind::LayerNorm: {
@@ -843,7 +951,9 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
     return it->second.t;
 }
 
-NdTensor NdGraph::run(Ctx &ctx, const NdTensor &x) const { return run_ops(&ctx, x, ops.size(), nullptr); }
+NdTensor NdGraph::run(Ctx &ctx, const NdTensor &x, float *dst) const {
+    return run_ops(&ctx, x, ops.size(), nullptr, dst);
+}
 
 std::vector<int64_t> NdGraph::output_shape(const std::vector<int64_t> &in) const {
     NdTensor x;

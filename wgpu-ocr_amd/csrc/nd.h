@@ -47,11 +47,15 @@ struct NdOp {
     // Linear: [k] -> [n]
     int k = 0, n = 0;
     // LayerNorm
-    const float *gb = nullptr;
+    const float *gb = nullptr, *gb32 = nullptr;  // gb32: gamma and beta each padded to a multiple of 32
     int len = 0;
     float eps = 1e-5f;
     // Affine
     const float *st = nullptr;
+    // What runs in the same launch: a Linear's or MLP's LayerNorm (gb32, len, eps above, its
+    // input is then the LayerNorm's), and the Linear that this step's rows go through (an MLP's second, an
+    // attention's projection), whose output and residual are this op's.
+    std::shared_ptr<NdOp> then;
     // Attention: inputs are the QKV projection, the first and the last Reshape's shapes
     float scale = 1.f;
 };
@@ -61,8 +65,10 @@ class NdGraph {
     // nd.rs:505: `stop_before_softmax` returns the logits a final Softmax would read.
     static NdGraph build(Ctx &ctx, const Onnx &onnx, bool stop_before_softmax);
 
-    // nd.rs:834: the graph on x (device memory, row-major); returns the output tensor.
-    NdTensor run(Ctx &ctx, const NdTensor &x) const;
+    // nd.rs:834: the graph on x (device memory, row-major); returns the output tensor. With dst
+    // (room for the output) the last step writes there where it can; the returned tensor says
+    // where the output is.
+    NdTensor run(Ctx &ctx, const NdTensor &x, float *dst = nullptr) const;
     // The arg-max over the last axis of the output per row (first index on ties, nd.rs:383).
     // When the graph ends in a Linear (the CTC head), its logits are never written: the GEMM
     // keeps per-block (max, index) pairs that one more kernel reduces.
@@ -83,7 +89,9 @@ class NdGraph {
     std::map<std::string, DevW> weights_;
     std::map<std::string, std::vector<int64_t>> ints_;
     std::map<std::string, size_t> last_use_;
-    NdTensor run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std::string, NdValue> *vals) const;
+    void join_ops();
+    NdTensor run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std::string, NdValue> *vals,
+                     float *dst = nullptr) const;
     NdValue get(const std::map<std::string, NdValue> &vals, const std::string &name) const;
 };
 

@@ -91,8 +91,18 @@ struct NdRowsArgs {
     const float *bias = nullptr, *res = nullptr;
     float *y = nullptr;
     int act = ACT_NONE;
+    // LayerNorm of x's rows first (nd_rows_block): gamma, then beta, each padded with zeros to a
+    // multiple of 32; or null.
+    const float *gb = nullptr;
+    float eps = 0.f;
 };
 bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s);
+// a, which may have a LayerNorm, and if b is given b applied to the rows that a gives, which are
+// then never written (kernels/ndblock.hip). Packs that fit: at most 128 inputs, a multiple of 4,
+// and with b at most 256 hidden values.
+bool nd_rows_fit(const ConvPack &w1);
+bool nd_mlp_fits(const ConvPack &w1, const ConvPack &w2);
+void nd_rows_block(const NdRowsArgs &a, const NdRowsArgs *b, hipStream_t s);
 // The CTC head without its logits: per row of x, nd_head_parts partial (max, index bits) pairs of
 // x W + b (first index on ties) at part[row * parts + j], for nd_argmax_partials. Needs 64-column
 // blocks and k <= 256. False (nothing launched) otherwise.
@@ -111,6 +121,13 @@ void nd_threshold_bits(const float *prob, int w, int h, float thr, uint32_t *bit
 // Multi-head self-attention from a fused QKV projection: x [n][t][3 heads d] (q, k, v blocks of
 // heads x d), y[i][j][h d + c] = sum_k softmax_k(scale q_j . k_k) v_k[c] (kernels/attn.hip).
 void nd_attention(const float *x, int n, int t, int heads, int d, float scale, float *y, hipStream_t s);
+// The same on the matrix cores, for heads of 4 to 16 values (kernels/ndblock.hip). False
+// (nothing launched) otherwise.
+bool nd_attention_mfma(const float *x, int n, int t, int heads, int d, float scale, float *y, hipStream_t s);
+// And with the projection w of its rows (w.x unused, w.m = n t), whose input is never written:
+// heads of 4 to 16 values, 256 values in all.
+bool nd_attention_proj_fits(int heads, int d, const ConvPack &pk);
+void nd_attention_proj(const float *x, int n, int t, int heads, int d, float scale, const NdRowsArgs &w, hipStream_t s);
 
 // Batched C[b] = A[b] (M x K) * B[b] (K x N) on the matrix cores, both operands float32 split
 // into float16 hi + lo (three passes: hi*hi, hi*lo, lo*hi), float32 accumulation. Element
