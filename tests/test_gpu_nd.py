@@ -345,6 +345,70 @@ def test_fused_attention_shapes(ctx, tmp_path, n, t, dim, heads):
     check(ctx, p, RNG.standard_normal((n, t, dim)).astype(np.float32))
 
 
+def _pool2(g, x):
+    return g.add("MaxPool", [x], kernel_shape=[2, 2], strides=[2, 2])
+
+
+def _up(g, x, f):
+    sc = g.init(g.fresh("sc"), np.array([1, 1, f, f], np.float32))
+    return g.add("Resize", [x, "", sc], mode="nearest", coordinate_transformation_mode="asymmetric", nearest_mode="floor")
+
+
+@pytest.mark.parametrize("n,cin,cout,h,w,exact", [(3, 20, 16, 41, 101, True), (1, 64, 40, 64, 289, False),
+                                                  (2, 33, 64, 120, 90, True), (1, 3, 70, 96, 200, True)])
+def test_3x3_nchw_many_rows(ctx, tmp_path, n, cin, cout, h, w, exact):
+    # Images of many rows: tiles of 8 x 32 pixels with a part of a tile left on both sides, channel
+    # counts that end inside a chunk or block, with a residual.
+    def fn(g, x):
+        y = g.add("Relu", [bn(g, conv(g, x, cin, cout, exact=exact, bias=False), cout)])
+        return g.add("Add", [g.add("Relu", [conv(g, y, cout, cout)]), y])
+    p = build(tmp_path, "c3r", fn, (n, cin, h, w))
+    check(ctx, p, RNG.standard_normal((n, cin, h, w)).astype(np.float32))
+
+
+@pytest.mark.parametrize("n,c,h,w,cout", [(4, 16, 64, 96, 16), (1, 16, 16, 24, 16), (2, 8, 88, 160, 40), (2, 12, 64, 96, 16),
+                                          (4, 32, 32, 104, 32)])
+def test_conv_of_upscaled_parts(ctx, tmp_path, n, c, h, w, cout):
+    # What a Concat of Resizes would write is read from the parts: by the 3 x 3 conv on tiles, or
+    # written out after all (few tiles, a part of 12 channels). A Resize is also a 1 x 1 and a
+    # 3 x 3 conv's residual, and one is read by an op that is no conv.
+    def fn(g, x):
+        p1 = _pool2(g, x)
+        p2 = _pool2(g, p1)
+        u1 = _up(g, p1, 2.0)
+        cat = g.add("Concat", [_up(g, p2, 4.0), u1, x], axis=1)
+        y = g.add("Relu", [conv(g, cat, 3 * c, cout)])
+        a = g.add("Add", [conv(g, y, cout, c, k=1), u1])
+        b = g.add("Add", [conv(g, a, c, c), _up(g, p1, 2.0)])
+        return g.add("Add", [b, g.add("Relu", [_up(g, p2, 4.0)])])
+    p = build(tmp_path, "parts", fn, (n, c, h, w))
+    check(ctx, p, RNG.standard_normal((n, c, h, w)).astype(np.float32))
+
+
+@pytest.mark.parametrize("n,c1,c2,h,w,k", [(2, 256, 256, 1, 109, 3), (1, 32, 40, 5, 61, 1), (3, 64, 16, 9, 30, 3), (2, 24, 40, 6, 50, 1)])
+def test_conv_of_two_tensors(ctx, tmp_path, n, c1, c2, h, w, k):
+    # A conv over a Concat of two tensors reads both where they lie (the first of a multiple of 32
+    # channels; the last case is written out).
+    def fn(g, x):
+        a = g.add("Relu", [conv(g, x, 16, c1, k=1)])
+        b = g.add("Relu", [conv(g, x, 16, c2, k=1)])
+        return g.add("Relu", [conv(g, g.add("Concat", [a, b], axis=1), c1 + c2, 40, k=k)])
+    p = build(tmp_path, "two", fn, (n, 16, h, w))
+    check(ctx, p, RNG.standard_normal((n, 16, h, w)).astype(np.float32))
+
+
+@pytest.mark.parametrize("cin,cout,h,w,exact", [(7, 20, 3, 5, True), (64, 16, 9, 31, False), (100, 70, 12, 40, True),
+                                                (250, 64, 5, 33, True), (128, 256, 6, 218, False)])
+def test_1x1_nchw_channel_edges(ctx, tmp_path, cin, cout, h, w, exact):
+    # 1 x 1 convs whose channels end inside a chunk and take one to two batches of chunks, with a
+    # GELU and a residual.
+    def fn(g, x):
+        y = conv(g, x, cin, cout, k=1, exact=exact)
+        return g.add("Add", [g.add("Relu", [conv(g, y, cout, cout, k=1, exact=exact)]), y])
+    p = build(tmp_path, "c1e", fn, (2, cin, h, w))
+    check(ctx, p, RNG.standard_normal((2, cin, h, w)).astype(np.float32))
+
+
 def _layer_norm(g, x, k):
     b = synth_pp._B("ln", 3)
     b.g = g

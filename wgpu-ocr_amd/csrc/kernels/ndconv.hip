@@ -43,6 +43,8 @@ struct NchwParams {
     float *y;
     const half8 *wt, *wt_lo;  // [nblock][chunk][tap][bn][32] float16 (hi; lo when not exact)
     const float *bias, *affine, *res, *in_scale;
+    const float *x2;  // channels c1 .. of the input, or null
+    int c1, res_up;   // res_up: the residual is upscaled by 2^res_up as it is read
     int n, cin, h, w, cout, oh, ow;
     int bn, chunks, kh, kw, pt, pl, act;
     int flat;        // 1 x 1: pixels run over the flattened plane (h * w of them)
@@ -53,7 +55,65 @@ struct NchwParams {
 
 // WPB wavefronts a workgroup: 4, or 16 for launches of few tiles and long K (up to 16 wavefronts
 // share one tile's K steps).
-template <int MT, int NT, bool LO, int WPB>
+// The outputs of a wavefront's tile: pixels x0 .. (of row oy, or of the flattened plane) of image
+// img, channels of block nb.
+template <int MT, int NT, bool EXT>
+__device__ inline void store_nchw(const NchwParams &p, const floatx4 (&acc)[MT][NT], int img, int oy, int x0, int nb, int r, int g) {
+    // Lane (r, g) holds pixels 16m + 4g .. 16m + 4g + 3 of its tile for output channel 16t + r:
+    // one 16-byte store where the four are whole and aligned.
+    const int olim = p.flat ? p.oh * p.ow : p.ow;
+    const size_t oplane = size_t(p.oh) * p.ow;
+    const bool vec = (p.flat ? (oplane & 3) == 0 : (p.ow & 3) == 0) && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 &&
+                     (!p.res || (reinterpret_cast<uintptr_t>(p.res) & 15) == 0);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int co = nb * p.bn + 16 * t + r;
+        if (co >= p.cout) continue;
+        const float b = p.bias ? p.bias[co] : 0.f;
+        const float as = p.affine ? p.affine[co] : 1.f, at = p.affine ? p.affine[p.cout + co] : 0.f;
+        const size_t o0 = (size_t(img) * p.cout + co) * oplane + (p.flat ? 0 : size_t(oy) * p.ow);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const int px = x0 + 16 * m + 4 * g;
+            if (px >= olim) continue;
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                float u = acc[m][t][k] + b;
+                if (p.affine) u = u * as + at;
+                v[k] = act_dev(u, p.act);
+            }
+            float *dst = p.y + o0 + px;
+            if (EXT && p.res_up) {
+                const int rh = p.oh >> p.res_up, rw = p.ow >> p.res_up;
+                const float *rp = p.res + (size_t(img) * p.cout + co) * rh * rw;
+                int yy = p.flat ? px / p.ow : oy, xx = px - (p.flat ? yy * p.ow : 0);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (px + k < olim) v[k] += rp[(yy >> p.res_up) * rw + (xx >> p.res_up)];
+                    if (p.flat && ++xx == p.ow) xx = 0, yy++;
+                    else if (!p.flat) xx++;
+                }
+            }
+            const bool res = p.res && !(EXT && p.res_up);
+            if (vec && px + 4 <= olim) {
+                if (res) {
+                    const float4 q = *reinterpret_cast<const float4 *>(p.res + o0 + px);
+                    v[0] += q.x, v[1] += q.y, v[2] += q.z, v[3] += q.w;
+                }
+                *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (px + k < olim) dst[k] = v[k] + (res ? p.res[o0 + px + k] : 0.f);
+            }
+        }
+    }
+}
+
+// EXT: an input scale, a second input tensor or an upscaled residual (the plain form needs fewer
+// registers: 52 against 60, 17 against 21 us for the recogniser's 64 -> 128 conv).
+template <int MT, int NT, bool LO, int WPB, bool EXT>
 __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
     extern __shared__ float s_red[];  // ksplit > 1: [wave][MT * NT * 4][64 lanes]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -83,7 +143,8 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             oy = line - img * p.oh;
         }
         const int taps = p.kh * p.kw, steps = p.chunks * taps;
-        const float *xim = p.x + size_t(img) * p.cin * plane;
+        const float *xim = p.x + size_t(img) * (EXT && p.x2 ? p.c1 : p.cin) * plane;
+        const float *xim2 = EXT && p.x2 ? p.x2 + size_t(img) * (p.cin - p.c1) * plane : nullptr;
         // K step s is (chunk, tap); steps whose kernel row reads only padding are skipped (the
         // same for the whole wavefront).
         auto valid_from = [&](int s) {
@@ -111,7 +172,9 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             // offsets from it (an image holds fewer than 2^30 values, checked by the host). The
             // reads are unconditional, from a position inside the image (channel clamped to the
             // last, pixel to the row's first), and the values outside are zeroed after.
-            const float *xrow = xim + (p.flat ? 0 : size_t(oy + ky - p.pt) * p.w);
+            const bool second = EXT && p.x2 && chunk * 32 >= p.c1;
+            const int cs = second ? p.c1 : 0;
+            const float *xrow = (second ? xim2 : xim) + (p.flat ? 0 : size_t(oy + ky - p.pt) * p.w);
             const bool full = c0 + 8 <= p.cin;
 #pragma unroll
             for (int m = 0; m < MT; m++) {
@@ -121,9 +184,9 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     const int ci = full ? c0 + j : min(c0 + j, p.cin - 1);
-                    const unsigned boff = (unsigned(ci) * planeu + pxc) * 4u;
+                    const unsigned boff = (unsigned(ci - cs) * planeu + pxc) * 4u;
                     float t = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xrow) + boff);
-                    if (p.in_scale) t *= p.in_scale[size_t(img) * p.cin + ci];
+                    if (EXT && p.in_scale) t *= p.in_scale[size_t(img) * p.cin + ci];
                     xv[m][j] = (in && (full || c0 + j < p.cin)) ? t : 0.f;
                 }
             }
@@ -185,50 +248,103 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
         }
     }
     if (!live) return;
-    // Lane (r, g) holds pixels 16m + 4g .. 16m + 4g + 3 of its tile for output channel 16t + r:
-    // one 16-byte store where the four are whole and aligned.
-    const int olim = p.flat ? p.oh * p.ow : p.ow;
-    const size_t oplane = size_t(p.oh) * p.ow;
-    const bool vec = (p.flat ? (oplane & 3) == 0 : (p.ow & 3) == 0) && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 &&
-                     (!p.res || (reinterpret_cast<uintptr_t>(p.res) & 15) == 0);
+    store_nchw<MT, NT, EXT>(p, acc, img, oy, x0, nb, r, g);
+}
+
+// 1 x 1 convs: a wavefront makes 16 pixels of the flattened plane x 16 NT channels, with the
+// operands of KC chunks (128 input channels at most) asked for at once: conv_nchw has one chunk's
+// in flight, and a wavefront's time is its chunks' latencies one after another. The
+// loads' addresses step by a plane (one multiply a chunk), and every load is issued before the first
+// value is looked at. 16 lines: 64 -> 128 channels at 12 x 218 17 -> 14 us, the SE-scaled 128 -> 256 at
+// 6 x 218 37 -> 23; one line 7-13 -> 4-8 us a conv.
+template <int NT, int KC, bool LO, bool EXT>
+__global__ __launch_bounds__(256) void conv_px_kernel(NchwParams p) {
+    const int lane = threadIdx.x & 63, tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nb = blockIdx.y;
+    if (tile >= p.tiles) return;
+    const int r = lane & 15, g = lane >> 4;
+    const int img = tile / p.tiles_line, x0 = (tile - img * p.tiles_line) * 16;
+    const unsigned plane = unsigned(p.h) * unsigned(p.w), px = min(unsigned(x0 + r), plane - 1u);
+    const int c1 = EXT && p.x2 ? p.c1 : p.cin;
+    const float *xa = p.x + size_t(img) * c1 * plane, *xb = EXT && p.x2 ? p.x2 + size_t(img) * (p.cin - c1) * plane : nullptr;
+    // The lo products' sums apart: half as many roundings in the large sums.
+    floatx4 acc[1][NT], accl[NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int co = nb * p.bn + 16 * t + r;
-        if (co >= p.cout) continue;
-        const float b = p.bias ? p.bias[co] : 0.f;
-        const float as = p.affine ? p.affine[co] : 1.f, at = p.affine ? p.affine[p.cout + co] : 0.f;
-        const size_t o0 = (size_t(img) * p.cout + co) * oplane + (p.flat ? 0 : size_t(oy) * p.ow);
+    for (int t = 0; t < NT; t++) acc[0][t] = accl[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < p.chunks; k0 += KC) {
+        half8 a[KC][NT], al[LO ? KC : 1][NT];
+        float v[KC][8], sc[EXT ? KC : 1][8];
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-            const int px = x0 + 16 * m + 4 * g;
-            if (px >= olim) continue;
-            float v[4];
+        for (int k = 0; k < KC; k++) {
+            const int chunk = min(k0 + k, p.chunks - 1), c0 = chunk * 32 + 8 * g;
+            const size_t wo = size_t(nb * p.chunks + chunk) * (p.bn * 4) + size_t(r) * 4 + g;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                float u = acc[m][t][k] + b;
-                if (p.affine) u = u * as + at;
-                v[k] = act_dev(u, p.act);
+            for (int t = 0; t < NT; t++) {
+                a[k][t] = p.wt[wo + t * 64];
+                if constexpr (LO) al[k][t] = p.wt_lo[wo + t * 64];
             }
-            float *dst = p.y + o0 + px;
-            if (vec && px + 4 <= olim) {
-                if (p.res) {
-                    const float4 q = *reinterpret_cast<const float4 *>(p.res + o0 + px);
-                    v[0] += q.x, v[1] += q.y, v[2] += q.z, v[3] += q.w;
-                }
-                *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
+            const bool second = EXT && p.x2 && chunk * 32 >= c1;
+            const float *x = second ? xb : xa;
+            // Channels past the last read the last; their weights' products are left out below.
+            const int cl = (second ? p.cin - c1 : c1) - 1;
+            int ci = c0 - (second ? c1 : 0);
+            unsigned at = unsigned(min(ci, cl)) * plane + px;
 #pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (px + k < olim) dst[k] = v[k] + (p.res ? p.res[o0 + px + k] : 0.f);
+            for (int j = 0; j < 8; j++) {
+                v[k][j] = x[at];
+                if constexpr (EXT) sc[k][j] = p.in_scale ? p.in_scale[size_t(img) * p.cin + min(c0 + j, p.cin - 1)] : 1.f;
+                at += ci++ < cl ? plane : 0u;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            if (k0 + k >= p.chunks) break;
+            const int c0 = (k0 + k) * 32 + 8 * g;
+            half8 hi, lo;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (EXT && p.in_scale) v[k][j] *= sc[EXT ? k : 0][j];
+                v[k][j] = c0 + j < p.cin ? v[k][j] : 0.f;
+            }
+            split8(v[k], hi, lo);
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, a[k][t], acc[0][t], 0, 0, 0);
+                accl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, a[k][t], accl[t], 0, 0, 0);
+                if constexpr (LO) accl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, al[k][t], accl[t], 0, 0, 0);
             }
         }
     }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[0][t][k] += accl[t][k];
+    store_nchw<1, NT, EXT>(p, acc, img, 0, x0, nb, r, g);
+}
+
+template <int NT, int KC>
+void launch_px(const NchwParams &p, bool lo, dim3 grid, hipStream_t s) {
+    const bool ext = p.in_scale || p.x2 || p.res_up;
+    if (lo && ext) hipLaunchKernelGGL((conv_px_kernel<NT, KC, true, true>), grid, dim3(256), 0, s, p);
+    else if (lo) hipLaunchKernelGGL((conv_px_kernel<NT, KC, true, false>), grid, dim3(256), 0, s, p);
+    else if (ext) hipLaunchKernelGGL((conv_px_kernel<NT, KC, false, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((conv_px_kernel<NT, KC, false, false>), grid, dim3(256), 0, s, p);
+}
+
+template <int NT>
+void launch_px_kc(const NchwParams &p, bool lo, dim3 grid, hipStream_t s) {
+    if (p.chunks == 1) launch_px<NT, 1>(p, lo, grid, s);
+    else if (p.chunks == 2) launch_px<NT, 2>(p, lo, grid, s);
+    else launch_px<NT, 4>(p, lo, grid, s);
 }
 
 template <int MT, int NT, int WPB>
 void launch_nchw(const NchwParams &p, bool lo, dim3 grid, size_t lds, hipStream_t s) {
-    if (lo) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, true, WPB>), grid, dim3(64 * WPB), lds, s, p);
-    else hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, false, WPB>), grid, dim3(64 * WPB), lds, s, p);
+    const bool ext = p.in_scale || p.x2 || p.res_up;
+    if (lo && ext) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, true, WPB, true>), grid, dim3(64 * WPB), lds, s, p);
+    else if (lo) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, true, WPB, false>), grid, dim3(64 * WPB), lds, s, p);
+    else if (ext) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, false, WPB, true>), grid, dim3(64 * WPB), lds, s, p);
+    else hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, false, WPB, false>), grid, dim3(64 * WPB), lds, s, p);
 }
 
 template <int MT, int WPB = 4>
@@ -568,6 +684,7 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
     const ConvPack &pk = a.pk;
     if (pk.kh > 3 || pk.kw > 3 || pk.cin != a.cin || pk.cout != a.cout || !a.wt_hi) return false;
     if (!pk.exact && !a.wt_lo) return false;
+    if (a.x2 && (a.c1 < 32 || a.c1 % 32 || a.c1 >= a.cin)) return false;
     if (pk.bn != 16 && pk.bn != 32 && pk.bn != 64) return false;
     NchwParams p{};
     p.x = a.x;
@@ -578,6 +695,9 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
     p.affine = a.affine;
     p.res = a.res;
     p.in_scale = a.in_scale;
+    p.x2 = a.x2;
+    p.c1 = a.c1;
+    p.res_up = a.res_up;
     p.n = a.n;
     p.cin = a.cin;
     p.h = a.h;
@@ -622,6 +742,9 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
     if (waves < 1024 && steps >= 16 && (nt <= 2 || pk.exact)) ks = waves < 512 ? 16 : 8, wpb = 16, mt = 1;
     else if (waves < 1024 && steps >= 8) ks = 4;
     else if (waves < 2048 && steps >= 4) ks = 2;
+    // 1 x 1 convs of few K steps: conv_px, unsplit.
+    const bool px = p.flat && mt == 1 && wpb == 4 && steps <= 16;
+    if (px) ks = 1;
     if (ks > 1 && mt * nt > 8) mt = std::max(1, 8 / nt);
     p.tiles_line = int(std::ceil(lim / (16.0 * mt)));
     if (tiles_of(mt) > 0x3fffffff) return false;
@@ -636,7 +759,10 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
                          2.0 * double(pk.halves()) * (pk.exact ? 1 : 2);
     ProbeScope probe("nd_conv_nchw", s, flops, bytes);
     const bool lo = !pk.exact;
-    if (wpb == 16) launch_nchw_nt<1, 16>(p, nt, lo, grid, lds, s);
+    if (px && nt == 1) launch_px_kc<1>(p, lo, grid, s);
+    else if (px && nt == 2) launch_px_kc<2>(p, lo, grid, s);
+    else if (px) launch_px_kc<4>(p, lo, grid, s);
+    else if (wpb == 16) launch_nchw_nt<1, 16>(p, nt, lo, grid, lds, s);
     else if (mt == 4) launch_nchw_nt<4>(p, nt, lo, grid, lds, s);
     else if (mt == 2) launch_nchw_nt<2>(p, nt, lo, grid, lds, s);
     else launch_nchw_nt<1>(p, nt, lo, grid, lds, s);

@@ -291,6 +291,22 @@ void NdGraph::join_ops() {
         }
         gone[size_t(j)] = true;
     }
+    // Concats over channels, then Resizes, that only convs on the matrix cores read.
+    for (const char *kind : {"Concat", "Resize"})
+        for (size_t k = 0; k < ops.size(); k++) {
+            NdOp &op = ops[k];
+            const Node &nd = nodes_[size_t(op.node)];
+            if (gone[k] || op.kind != NdKind::Generic || nd.op != kind || op.output == output) continue;
+            bool ok = nd.op == "Resize" || (op.inputs.size() <= size_t(ND_SOURCES) && nd.int_("axis").value_or(0) == 1);
+            for (size_t j = 0; ok && j < ops.size(); j++) {
+                const NdOp &o = ops[j];
+                for (size_t i = 0; i < o.inputs.size(); i++)
+                    if (o.inputs[i] == op.output) ok &= (o.kind == NdKind::Conv && o.mfma && i == 0) || (o.parts && nd.op == "Resize");
+                if (o.residual == op.output) ok &= o.kind == NdKind::Conv && o.mfma;
+                if (o.in_scale == op.output) ok = false;
+            }
+            op.parts = ok;
+        }
     size_t n = 0;
     for (size_t k = 0; k < ops.size(); k++)
         if (!gone[k]) {
@@ -376,6 +392,43 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         ra.eps = op.eps;
         return ra;
     };
+    // A tensor in memory: t itself, or its parts written out.
+    auto solid = [&](const NdTensor &t) {
+        if (t.parts.empty()) return t;
+        NdTensor y;
+        y.shape = t.shape;
+        y.buf = std::make_shared<DBuf>(ctx, std::max<size_t>(y.count(), 1) * sizeof(float));
+        y.p = y.buf->as<float>();
+        const auto os = strides_of(y.shape);
+        size_t c0 = 0;
+        for (const NdPart &part : t.parts) {
+            const auto &ps = part.t.shape;
+            const float *src = part.t.p;
+            std::vector<int64_t> us = {ps[0], ps[1], ps[2] << part.up, ps[3] << part.up};
+            DBuf up;
+            if (part.up) {
+                const bool whole = t.parts.size() == 1;
+                if (!whole) up = DBuf(ctx, size_t(us[0] * us[1] * us[2] * us[3]) * sizeof(float));
+                float *dst_up = whole ? y.p : up.as<float>();
+                nd_resize_nearest(src, dst_up, size_t(us[0] * us[1]), int(ps[2]), int(ps[3]), int(us[2]), int(us[3]),
+                                  float(1 << part.up), float(1 << part.up), st);
+                if (whole) break;
+                src = dst_up;
+            }
+            const auto is = strides_of(us);
+            NdIndex ix;
+            ix.total = size_t(us[0] * us[1] * us[2] * us[3]);
+            ix.rank = 4;
+            for (size_t d = 0; d < 4; d++) {
+                ix.dims[d] = size_t(us[d]);
+                ix.s0[d] = is[d];
+                ix.s1[d] = os[d];
+            }
+            nd_copy(src, y.p, ix, 0, c0 * os[1], st);
+            c0 += size_t(us[1]);
+        }
+        return y;
+    };
     for (; oi < nops; oi++) {
         const NdOp &op = ops[oi];
         const Node &n = nodes_[size_t(op.node)];
@@ -383,7 +436,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         auto flt = [&](size_t k) {
             NdValue v = arg(k);
             if (v.is_int) fail(n.op + ": input " + std::to_string(k) + " is not float");
-            return v.t;
+            return solid(v.t);
         };
         auto ints = [&](size_t k) {
             NdValue v = arg(k);
@@ -393,7 +446,8 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         NdValue out;
         switch (op.kind) {
         case NdKind::Conv: {
-            const NdTensor a = flt(0);
+            if (arg(0).is_int) fail(n.op + ": input 0 is not float");
+            NdTensor a = arg(0).t;
             if (a.shape.size() != 4) fail("Conv input " + shape_str(a.shape));
             const int nb = int(a.shape[0]), cin = int(a.shape[1]), h = int(a.shape[2]), w = int(a.shape[3]);
             if (cin != op.cin) fail("Conv expects " + std::to_string(op.cin) + " channels, has " + std::to_string(cin));
@@ -417,7 +471,13 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 if (sc.count() != size_t(nb) * cin) fail("input scale " + shape_str(sc.shape) + " for " + shape_str(a.shape));
             }
             if (shapes_only) break;
+            if (!op.mfma) {
+                a = solid(a);
+                res = solid(res);
+                sc = solid(sc);
+            }
             if (op.mfma) {
+                sc = solid(sc);
                 NdMfmaConvArgs ma;
                 ma.x = a.p;
                 ma.n = nb;
@@ -438,7 +498,28 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 ma.pt = pt;
                 ma.pl = pl;
                 ma.act = op.act;
-                if (!no_ndconv() && nd_conv_nchw_mfma(ma, st)) break;
+                if (!res.parts.empty()) {
+                    if (res.parts.size() != 1) res = solid(res);
+                    else ma.res_up = res.parts[0].up;
+                    ma.res = res.parts.empty() ? res.p : res.parts[0].t.p;
+                }
+                if (!no_ndconv()) {
+                    std::vector<NdConvSource> src;
+                    for (const NdPart &part : a.parts)
+                        src.push_back({part.t.p, 0, int(part.t.shape[1]), int(part.t.shape[2]), int(part.t.shape[3]), part.up});
+                    if (nd_conv_tile(ma, src.empty() ? nullptr : src.data(), int(src.size()), st)) break;
+                    if (src.size() == 2 && !src[0].up && !src[1].up && src[0].c % 32 == 0) {
+                        ma.x = src[0].p;
+                        ma.x2 = src[1].p;
+                        ma.c1 = src[0].c;
+                    } else {
+                        a = solid(a);
+                        ma.x = a.p;
+                    }
+                    if (nd_conv_nchw_mfma(ma, st)) break;
+                }
+                a = solid(a);
+                res = solid(res);
                 ConvArgs ca;
                 ca.x = Act{a.p, nb, h, w, cin, cin};
                 ca.y = Act{out.t.p, nb, oh, ow, op.cout, op.cout};
@@ -800,6 +881,16 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                         if (int(d) != ax && p.t.shape[d] != parts[0].t.shape[d]) fail("Concat shapes differ");
                     shape[size_t(ax)] += p.t.shape[size_t(ax)];
                 }
+                if (op.parts && !shapes_only && r == 4 && ax == 1 &&
+                    std::all_of(parts.begin(), parts.end(), [](const NdValue &v) { return v.t.parts.size() <= 1; })) {
+                    out.t.shape = shape;
+                    for (const auto &p : parts) {
+                        if (p.t.parts.empty()) out.t.parts.push_back({p.t, 0});
+                        else out.t.parts.push_back(p.t.parts[0]);
+                    }
+                    break;
+                }
+                for (auto &p : parts) p.t = solid(p.t);
                 out.t = alloc(shape);
                 if (shapes_only) break;
                 const auto os = strides_of(shape);
@@ -852,6 +943,12 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 if (a.shape.size() != 4 || sc[0] != 1.f || sc[1] != 1.f) fail("Resize scales on batch or channels");
                 const int h = int(a.shape[2]), w = int(a.shape[3]);
                 const int oh = int(std::floor(float(h) * sc[2])), ow = int(std::floor(float(w) * sc[3]));
+                const int up = sc[2] == 2.f ? 1 : sc[2] == 4.f ? 2 : sc[2] == 8.f ? 3 : 0;
+                if (op.parts && !shapes_only && up && sc[2] == sc[3] && a.count()) {
+                    out.t.shape = {a.shape[0], a.shape[1], oh, ow};
+                    out.t.parts.push_back({a, up});
+                    break;
+                }
                 out.t = alloc({a.shape[0], a.shape[1], oh, ow});
                 if (!shapes_only)
                     nd_resize_nearest(a.p, out.t.p, size_t(a.shape[0] * a.shape[1]), h, w, oh, ow, sc[2], sc[3], st);

@@ -15,11 +15,19 @@
 
 namespace ocr {
 
+// A float tensor in device memory, or one that no memory holds yet: the parts that a Concat over
+// axis 1 would write, each a nearest-neighbour upscaling of a tensor by 2^up (p is then null).
+struct NdPart;
 struct NdTensor {
     std::shared_ptr<DBuf> buf;  // owner (null for weights and caller memory)
     float *p = nullptr;
     std::vector<int64_t> shape;
+    std::vector<NdPart> parts;
     size_t count() const;
+};
+struct NdPart {
+    NdTensor t;
+    int up = 0;
 };
 
 struct NdValue {
@@ -46,6 +54,9 @@ struct NdOp {
     std::string residual, in_scale;
     // Linear: [k] -> [n]
     int k = 0, n = 0;
+    // A Resize or Concat that only convs read, as their input or residual, or a Concat of this
+    // kind: its result stays parts.
+    bool parts = false;
     // LayerNorm
     const float *gb = nullptr, *gb32 = nullptr;  // gb32: gamma and beta each padded to a multiple of 32
     int len = 0;

@@ -69,6 +69,7 @@ bool nd_conv_small(const NdConvArgs &a, hipStream_t s);
 // A group-1, stride-1 conv up to 3 x 3 in NCHW on the matrix cores (kernels/ndconv.hip), with
 // the weights packed by pack_conv_weights: act(affine(acc + b)) + res, in_scale[n][cin] applied to
 // the input first. False (nothing launched) for shapes it does not take.
+constexpr int ND_SOURCES = 4;
 struct NdMfmaConvArgs {
     const float *x = nullptr;
     int n = 0, cin = 0, h = 0, w = 0;
@@ -78,7 +79,19 @@ struct NdMfmaConvArgs {
     ConvPack pk;
     const float *bias = nullptr, *affine = nullptr, *res = nullptr, *in_scale = nullptr;
     int pt = 0, pl = 0, act = ACT_NONE;
+    int res_up = 0;             // res is [n][cout][oh >> res_up][ow >> res_up], upscaled (nearest) as it is read
+    const float *x2 = nullptr;  // channels c1 .. of the input ([n][cin - c1][h][w], x then has c1), c1 % 32 == 0
+    int c1 = 0;
 };
+// Channels c0 .. c0 + c - 1 of a conv's input: [n][c][h][w], upscaled (nearest) by 2^up as read.
+struct NdConvSource {
+    const float *p;
+    int c0, c, h, w, up;
+};
+// 3 x 3, pad 1 over images of many rows (kernels/ndconv3.hip), the input a.x or the nsrc sources
+// in order (c0 is set here), each from a multiple of 8 channels. False (nothing launched) for
+// shapes it does not take: few tiles (of one plain source), x2, res_up, in_scale.
+bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hipStream_t s);
 bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s);
 
 // y [m][n] = act(x [m][k] W + b) (+ res [m][n]) with W packed as n rows of k (pack_conv_weights,
