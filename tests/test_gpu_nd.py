@@ -280,6 +280,17 @@ def test_linear_row_gemm_shapes(ctx, tmp_path, shape, k, n, exact):
     check(ctx, p, RNG.standard_normal(shape).astype(np.float32))
 
 
+@pytest.mark.parametrize("rows,k,n,exact", [(3305, 120, 1301, True), (4100, 200, 1100, False), (3296, 64, 1344, True)])
+def test_linear_many_columns(ctx, tmp_path, rows, k, n, exact):
+    # Enough rows and columns for ranges of column blocks a wavefront; rows, K and N that end inside
+    # a tile, chunk and block.
+    def fn(g, x):
+        y = g.add("MatMul", [x, w(g, (k, n), k, exact=exact)])
+        return g.add("Add", [y, g.init("lb", (RNG.standard_normal(n) * 0.1).astype(np.float32))])
+    p = build(tmp_path, "wide", fn, (1, rows, k))
+    check(ctx, p, RNG.standard_normal((1, rows, k)).astype(np.float32))
+
+
 @pytest.mark.parametrize("k,n,exact", [(120, 200, True), (256, 300, False), (64, 1000, True)])
 def test_head_argmax_first_index_on_ties(ctx, tmp_path, k, n, exact):
     """The fused head: classes come in pairs with the same weights and bias, so every row's

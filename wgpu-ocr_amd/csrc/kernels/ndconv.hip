@@ -678,6 +678,86 @@ __global__ __launch_bounds__(256) void gemm_rows_amax_kernel(RowsParams p) {
     }
 }
 
+// Many columns (the CTC head's logits): a wavefront keeps its 16 RT rows' operands in registers
+// and walks a range of 64-column blocks, the next block's weights in flight. Bound by its stores
+// (130 MB for 1744 rows x 18 708). The ranges of a row lie next to each other in a workgroup and,
+// by number, on one XCD: rows end anywhere in a 128-byte line, and the two parts of a line meet
+// in one L2. 104 -> 66 us, against 32 x 64 tiles whose column
+// neighbours ran on other XCDs.
+template <int RT, int KC, bool LO>
+__global__ __launch_bounds__(256) void gemm_rows_wide_kernel(RowsParams p) {
+    constexpr int NT = 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int G = gridDim.x, b8 = blockIdx.x & 7;
+    const int wid = (b8 * (G >> 3) + min(b8, G & 7) + (int(blockIdx.x) >> 3)) * 4 + wave;
+    const int rt = wid / p.parts, part = wid - rt * p.parts;
+    if (rt >= p.rtiles) return;
+    const int r = lane & 15, g = lane >> 4;
+    const int r0 = rt * 16 * RT;
+    const int nb0 = part * p.nb_per_wave, nb1 = min(p.nblocks, nb0 + p.nb_per_wave);
+    half8 a[KC][NT];
+    auto load = [&](int nb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                a[c][t] = p.wt[size_t(nb * p.chunks + min(c, p.chunks - 1)) * 256 + t * 64 + r * 4 + g];
+    };
+    load(min(nb0, p.nblocks - 1));
+    half8 bh[RT][KC], bl[RT][KC];
+#pragma unroll
+    for (int m = 0; m < RT; m++)
+#pragma unroll
+        for (int c = 0; c < KC; c++) rows_frag(p, r0 + 16 * m + r, c * 32 + 8 * g, bh[m][c], bl[m][c]);
+    for (int nb = nb0; nb < nb1; nb++) {
+        float bias[NT][4];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) bias[t][k] = p.bias ? p.bias[min(nb * 64 + 16 * t + 4 * g + k, p.n - 1)] : 0.f;
+        floatx4 acc[RT][NT];
+#pragma unroll
+        for (int m = 0; m < RT; m++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KC; c++) {
+            if (c >= p.chunks) break;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int m = 0; m < RT; m++) {
+                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c][t], bh[m][c], acc[m][t], 0, 0, 0);
+                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c][t], bl[m][c], acc[m][t], 0, 0, 0);
+                    if constexpr (LO)
+                        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            p.wt_lo[size_t(nb * p.chunks + c) * 256 + t * 64 + r * 4 + g], bh[m][c], acc[m][t], 0, 0, 0);
+                }
+        }
+        if (nb + 1 < nb1) load(nb + 1);
+#pragma unroll
+        for (int m = 0; m < RT; m++) {
+            const int row = r0 + 16 * m + r;
+            if (row >= p.m) continue;
+            float *dst = p.y + size_t(row) * p.n + nb * 64 + 4 * g;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int co = nb * 64 + 16 * t + 4 * g;
+                floatx4 v;
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = act_dev(acc[m][t][k] + bias[t][k], p.act);
+                if ((p.n & 3) == 0 && co + 4 <= p.n) {
+                    *reinterpret_cast<floatx4 *>(dst + 16 * t) = v;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        if (co + k < p.n) dst[16 * t + k] = v[k];
+                }
+            }
+        }
+    }
+}
+
 }  // namespace
 
 bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
@@ -878,6 +958,24 @@ bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s) {
     if (waves(rt, ts) < 2048) rt = 1;
     while (waves(rt, ts) < 2048 && ts < ntf) ts *= 2;
     const int nt = ntf / ts;
+    const bool lo = !pk.exact, k8 = pk.chunks > 4;
+    // A full column block and 32 rows a wavefront with wavefronts to spare: ranges of blocks.
+    if (rt == 2 && nt == 4 && pk.nblocks >= 16 && pk.chunks <= 8 && !a.res) {
+        p.rtiles = (a.m + 31) / 32;
+        p.nb_per_wave = std::max(1, int(waves(2, 1) / 3072));
+        p.parts = (pk.nblocks + p.nb_per_wave - 1) / p.nb_per_wave;
+        const double groups = std::ceil(double(p.rtiles) * p.parts / 4);
+        if (groups > 0x7fffffff) return false;
+        ProbeScope probe("nd_gemm_rows", s, 2.0 * a.m * double(a.k) * a.n,
+                         4.0 * (double(a.m) * a.k + double(a.m) * a.n) + 2.0 * double(pk.halves()) * (lo ? 2 : 1));
+        const dim3 grid{unsigned(groups)};
+        if (lo && k8) hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 8, true>), grid, dim3(256), 0, s, p);
+        else if (lo) hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 4, true>), grid, dim3(256), 0, s, p);
+        else if (k8) hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 8, false>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 4, false>), grid, dim3(256), 0, s, p);
+        OCR_HIP(hipGetLastError());
+        return true;
+    }
     p.rtiles = (a.m + 16 * rt - 1) / (16 * rt);
     p.tsplit = ts;
     const double blocks = std::ceil(double(p.rtiles) * ts / 4);
@@ -885,7 +983,6 @@ bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s) {
     const dim3 grid{unsigned(blocks), unsigned(pk.nblocks)};
     ProbeScope probe("nd_gemm_rows", s, 2.0 * a.m * double(a.k) * a.n,
                      4.0 * (double(a.m) * a.k + double(a.m) * a.n) + 2.0 * double(pk.halves()) * (pk.exact ? 1 : 2));
-    const bool lo = !pk.exact, k8 = pk.chunks > 4;
 #define ROWS_LAUNCH(RT, NT)                                                                          \
     do {                                                                                             \
         if (lo && k8) hipLaunchKernelGGL((gemm_rows_kernel<RT, NT, 8, true>), grid, dim3(256), 0, s, p);   \
