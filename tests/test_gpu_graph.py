@@ -329,6 +329,21 @@ def test_shape_errors(ctx, tmp_path):
         gr.run(np.zeros((1, 3, 5, 5), np.float32))  # wrong channel count
 
 
+@pytest.mark.parametrize("n,cin,cout,h,w,pool", [(1, 32, 64, 40, 300, (2, 2)), (2, 64, 32, 61, 150, None), (3, 128, 256, 4, 301, (2, 1)),
+                                                 (1, 48, 20, 119, 203, None), (1, 16, 32, 1, 3, None), (1, 40, 16, 2, 8, (2, 1)),
+                                                 (1, 36, 17, 5, 9, (2, 2))])
+def test_conv3x3_both_forms(ctx, tmp_path, n, cin, cout, h, w, pool):
+    # Enough pixels for the persistent kernel's tiles, and few ones for the direct form: odd sizes,
+    # channels that end inside a slice and block, inexact weights every second case.
+    def net(g, x):
+        y = conv(g, x, cin, cout, act="Relu", exact=w % 2 == 1)
+        return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
+    p = build(tmp_path, "c3f", net, (n, cin, h, w))
+    x = RNG.standard_normal((n, cin, h, w)).astype(np.float32)
+    _, calls = _ran(FAST, lambda: check(ctx, p, x))
+    assert calls["conv3x3_dma"] >= 1, calls
+
+
 @pytest.mark.parametrize("cin,cout,h,w,pool,two", [(32, 64, 17, 45, (2, 2), False), (64, 128, 16, 37, (2, 1), False),
                                                    (128, 256, 4, 53, (2, 1), False), (16, 97, 9, 23, (2, 1), True),
                                                    (256, 128, 13, 19, (2, 2), True), (20, 48, 31, 70, (2, 2), False),
