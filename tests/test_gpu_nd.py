@@ -319,6 +319,36 @@ def test_head_argmax_first_index_on_ties(ctx, tmp_path, k, n, exact):
     assert np.array_equal(got, np.argmax(head.run(x), axis=-1))
 
 
+@pytest.mark.parametrize("c,h,wd,stride,k", [(2, 3, 1, (1, 1), 3), (3, 4, 3, (1, 1), 3), (3, 5, 4, (2, 2), 3), (3, 5, 5, (1, 1), 3),
+                                             (2, 6, 6, (2, 2), 3), (2, 7, 7, (1, 2), 3), (2, 5, 9, (2, 2), 5), (2, 5, 4, (1, 1), 5),
+                                             (2, 5, 6, (2, 1), 5)])
+def test_depthwise_row_ends(ctx, tmp_path, c, h, wd, stride, k):
+    # Rows that end inside or before a 16-byte load, at every shift.
+    p = build(tmp_path, "dwe", lambda g, x: conv(g, x, c, c, k=k, stride=stride, group=c, exact=False), (2, c, h, wd))
+    check(ctx, p, RNG.standard_normal((2, c, h, wd)).astype(np.float32))
+
+
+@pytest.mark.parametrize("cin,cout,h,wd,s", [(6, 5, 7, 9, 2), (4, 3, 16, 17, 2), (3, 6, 5, 5, 1), (4, 2, 3, 3, 3)])
+def test_conv_transpose_channel_blocks(ctx, tmp_path, cin, cout, h, wd, s):
+    # Output channels that do not fill a thread's four, and planes that end inside a workgroup.
+    p = build(tmp_path, "ctb", lambda g, x: g.add("ConvTranspose", [x, w(g, (cin, cout, s, s), cin, exact=False),
+                                                                     g.init("tb", np.full(cout, 0.1, np.float32))],
+                                                  kernel_shape=[s, s], strides=[s, s]), (2, cin, h, wd))
+    check(ctx, p, RNG.standard_normal((2, cin, h, wd)).astype(np.float32))
+
+
+@pytest.mark.parametrize("h,wd", [(1, 1), (3, 31), (2, 32), (5, 33), (4, 64), (3, 255), (2, 257), (7, 736)])
+def test_threshold_bits_widths(ctx, h, wd):
+    # One bit a pixel, rows of whole words: the bits past a row's end are zero, equal is not above.
+    import ocrhip
+    prob = RNG.choice(np.array([0.0, 0.3, np.nextafter(np.float32(0.3), np.float32(1)), 1.0], np.float32), (h, wd))
+    got = ocrhip.db_threshold(ctx, prob, 0.3)
+    on = np.zeros((h, (wd + 31) // 32 * 32), np.uint8)
+    on[:, :wd] = prob > np.float32(0.3)
+    want = np.packbits(on, axis=1, bitorder="little").view(np.uint32)
+    assert np.array_equal(np.asarray(got, np.uint32).reshape(want.shape), want)
+
+
 @pytest.mark.parametrize("cin,cout,k,s,act", [(16, 16, 2, 2, "Relu"), (16, 1, 2, 2, "Sigmoid"), (8, 5, 3, 3, "Relu"),
                                              (6, 4, 3, 2, "Sigmoid"), (5, 7, 4, 4, None)])
 def test_conv_transpose_nchw_shapes(ctx, tmp_path, cin, cout, k, s, act):
