@@ -376,8 +376,7 @@ int ocr_detect(ocr_detector *det, const float *input, uint32_t h, uint32_t w, fl
         need(input, "input");
         need(prob, "prob");
         det->owner->ctx->bind();
-        std::vector<float> out = det->det->detect(input, int(h), int(w));
-        std::copy(out.begin(), out.end(), prob);
+        det->det->detect(input, int(h), int(w), prob);
     });
 }
 

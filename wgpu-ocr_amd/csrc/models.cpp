@@ -42,13 +42,12 @@ void Detector::detect_pages_device(const uint8_t *const *rgb, const int *w, cons
     mask_up(mp.data(), count, DET_MW, thr, st);
 }
 
-std::vector<float> Detector::detect(const float *input, int h, int w) {
+void Detector::detect(const float *input, int h, int w, float *prob) {
     Act in{nullptr, 1, h, w, 1, 1};
     DBuf inbuf(&ctx_, in.count() * sizeof(float));
     in.p = inbuf.as<float>();
     ctx_.h2d(in.p, input, in.count() * sizeof(float));
     Graph::Out out = graph_.run(ctx_, in);
-    std::vector<float> prob(out.act.count());
     // The output is NHWC; for one channel that is NCHW too.
     if (out.act.c != 1) {
         std::vector<float> nhwc(out.act.count());
@@ -56,10 +55,9 @@ std::vector<float> Detector::detect(const float *input, int h, int w) {
         const size_t hw = size_t(out.act.h) * out.act.w;
         for (size_t p = 0; p < hw; p++)
             for (int c = 0; c < out.act.c; c++) prob[c * hw + p] = nhwc[p * out.act.c + c];
-        return prob;
+        return;
     }
-    ctx_.d2h(prob.data(), out.act.p, prob.size() * sizeof(float));
-    return prob;
+    ctx_.d2h(prob, out.act.p, out.act.count() * sizeof(float));
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -22,7 +22,7 @@ class Detector {
     void detect_pages_device(const uint8_t *const *rgb, const int *w, const int *h, int count, float thr,
                              uint32_t *const *bits);
     // Detector::detect (gpu.rs:1425-1430): the probability map of a [1, 1, h, w] host input.
-    std::vector<float> detect(const float *input, int h, int w);
+    void detect(const float *input, int h, int w, float *prob);
 
   private:
     Ctx &ctx_;
