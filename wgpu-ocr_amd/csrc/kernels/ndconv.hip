@@ -9,12 +9,14 @@
 // x 16 output channels of the packed float16 weights, one 16-byte read a lane. The float32
 // inputs are split into float16 hi + lo (x = hi + lo to about 2^-22) and both go through the
 // matrix core, accumulating in float32: float32-class results. A lane's four accumulators are
-// four neighbouring pixels of one output channel, stored with one 16-byte write. A wavefront owns 16 MT pixels of one output row (of the flattened plane for a
-// 1 x 1 conv) and 16 NT output channels; when there are too few such tiles to fill the GPU, up
-// to four wavefronts of a workgroup share one tile's K steps and add their accumulators through
-// LDS in a fixed order. Kernel rows that fall wholly into the padding are skipped (a 3 x 3 conv
+// four neighbouring pixels of one output channel, stored with one 16-byte write. A wavefront owns
+// 16 MT pixels of one output row (of the flattened plane for a 1 x 1 conv) and 16 NT output
+// channels; when there are too few such tiles to fill the GPU, up to four wavefronts of a workgroup
+// share one tile's K steps and add their accumulators through LDS in a fixed order. Kernel rows that fall wholly into the padding are skipped (a 3 x 3 conv
 // over a one-row tensor does one row of work).
 //
+// conv_px: 1 x 1 convolutions of up to 512 channels in tiles of 16 pixels, several K steps'
+// operands asked for at once.
 // conv_dw: depthwise convolution, one thread four neighbouring outputs, the taps summed in the
 // order the general kernel sums them (the same float32 results).
 // conv_small: group-1 convolutions with at most 27 taps in all (the 3-channel stems), one thread
@@ -23,6 +25,7 @@
 // 16 RT x 16 NT tile with its operands read straight from memory; with `amax` the logits are
 // never written: each wavefront walks a range of 64-column blocks keeping every row's best
 // (value, index), first index on ties, and writes one partial a row (the CTC head).
+// gemm_rows_wide: the same walk with the products stored (many columns).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -65,6 +68,29 @@ __device__ inline void store_nchw(const NchwParams &p, const floatx4 (&acc)[MT][
     const size_t oplane = size_t(p.oh) * p.ow;
     const bool vec = (p.flat ? (oplane & 3) == 0 : (p.ow & 3) == 0) && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 &&
                      (!p.res || (reinterpret_cast<uintptr_t>(p.res) & 15) == 0);
+    // An upscaled residual's values, asked for together (of the last channel past it, and of the
+    // line's last pixel past that).
+    float rv[EXT ? MT : 1][EXT ? NT : 1][4];
+    if constexpr (EXT) {
+        if (p.res_up) {
+            const int rh = p.oh >> p.res_up, rw = p.ow >> p.res_up;
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                int px = min(x0 + 16 * m + 4 * g, olim - 1), yy = p.flat ? px / p.ow : oy, xx = px - (p.flat ? yy * p.ow : 0);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const unsigned at = unsigned((yy >> p.res_up) * rw + (xx >> p.res_up));
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        const int co = min(nb * p.bn + 16 * t + r, p.cout - 1);
+                        rv[m][t][k] = (p.res + (size_t(img) * p.cout + co) * rh * rw)[at];
+                    }
+                    if (++px < olim && ++xx == p.ow) xx = 0, yy++;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         const int co = nb * p.bn + 16 * t + r;
@@ -85,15 +111,8 @@ __device__ inline void store_nchw(const NchwParams &p, const floatx4 (&acc)[MT][
             }
             float *dst = p.y + o0 + px;
             if (EXT && p.res_up) {
-                const int rh = p.oh >> p.res_up, rw = p.ow >> p.res_up;
-                const float *rp = p.res + (size_t(img) * p.cout + co) * rh * rw;
-                int yy = p.flat ? px / p.ow : oy, xx = px - (p.flat ? yy * p.ow : 0);
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    if (px + k < olim) v[k] += rp[(yy >> p.res_up) * rw + (xx >> p.res_up)];
-                    if (p.flat && ++xx == p.ow) xx = 0, yy++;
-                    else if (!p.flat) xx++;
-                }
+                for (int k = 0; k < 4; k++) v[k] += rv[EXT ? m : 0][EXT ? t : 0][k];
             }
             const bool res = p.res && !(EXT && p.res_up);
             if (vec && px + 4 <= olim) {

@@ -436,6 +436,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         auto flt = [&](size_t k) {
             NdValue v = arg(k);
             if (v.is_int) fail(n.op + ": input " + std::to_string(k) + " is not float");
+            if (v.t.parts.empty()) return std::move(v.t);
             return solid(v.t);
         };
         auto ints = [&](size_t k) {
@@ -446,8 +447,9 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         NdValue out;
         switch (op.kind) {
         case NdKind::Conv: {
-            if (arg(0).is_int) fail(n.op + ": input 0 is not float");
-            NdTensor a = arg(0).t;
+            NdValue in = arg(0);
+            if (in.is_int) fail(n.op + ": input 0 is not float");
+            NdTensor a = std::move(in.t);
             if (a.shape.size() != 4) fail("Conv input " + shape_str(a.shape));
             const int nb = int(a.shape[0]), cin = int(a.shape[1]), h = int(a.shape[2]), w = int(a.shape[3]);
             if (cin != op.cin) fail("Conv expects " + std::to_string(op.cin) + " channels, has " + std::to_string(cin));
@@ -890,7 +892,8 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                     }
                     break;
                 }
-                for (auto &p : parts) p.t = solid(p.t);
+                for (auto &p : parts)
+                    if (!p.t.parts.empty()) p.t = solid(p.t);
                 out.t = alloc(shape);
                 if (shapes_only) break;
                 const auto os = strides_of(shape);
