@@ -14,7 +14,8 @@
 // x 16 NT output columns and walks the input channels one 32-channel chunk (and tap) at a time:
 // the kernel is one pass over its operands, bound by loads in flight across wavefronts, so
 // registers go to occupancy (5 wavefronts a SIMD at RT = 2, NT = 4; 2 with four chunks' operands
-// held at once, 28 % slower over the detector's upsamplers).
+// held at once, 28 % slower over the detector's upsamplers at four pages; launches of few wavefronts
+// do hold four).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,7 +52,8 @@ __device__ inline float ct_act(float v, int act) {
     return v;
 }
 
-template <int RT, int NT, bool LO>
+// U > 1: that many (chunk, tap) steps are asked for at once.
+template <int RT, int NT, bool LO, int U>
 __global__ __launch_bounds__(256) void convt_rows_kernel(CtParams p) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wid = blockIdx.x * 4 + wave, nb = blockIdx.y;
@@ -74,6 +76,67 @@ __global__ __launch_bounds__(256) void convt_rows_kernel(CtParams p) {
         pi[m] = rem / p.gw;
         pj[m] = rem - pi[m] * p.gw;
     }
+    if constexpr (U > 1) {
+    const int steps = p.chunks * p.taps;
+    for (int k0 = 0; k0 < steps; k0 += U) {
+        half8 a[U][NT], al[U][NT];
+        float v[U][RT][8];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (k0 + u >= steps) break;
+            const int k = k0 + u, c = k / p.taps, tap = k - c * p.taps;
+            const int da = p.ty - 1 - tap / p.tx, db = p.tx - 1 - (tap - (tap / p.tx) * p.tx);
+            const size_t wo = (size_t(nb * p.chunks + c) * p.taps + tap) * (p.bn * 4) + size_t(r) * 4 + g;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                a[u][t] = p.wt[wo + (t0 + t) * 64];
+                if constexpr (LO) al[u][t] = p.wt_lo[wo + (t0 + t) * 64];
+            }
+            const int c0 = c * 32 + 8 * g;
+#pragma unroll
+            for (int m = 0; m < RT; m++) {
+                const int iy = pi[m] - da, ix = pj[m] - db;
+                const bool in = pimg[m] >= 0 && unsigned(iy) < unsigned(p.h) && unsigned(ix) < unsigned(p.w);
+                const size_t px = in ? (size_t(pimg[m]) * p.h + iy) * p.w + ix : 0;
+                float(&x)[8] = v[u][m];
+                if (p.vecx) {
+                    // Without a branch, so the loads of all steps go out together: a quadruple
+                    // outside is read from a place inside and made zero.
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const float4 q = *reinterpret_cast<const float4 *>(p.x + px * p.xcs + min(c0 + 4 * e, p.cin - 4));
+                        const bool ok = in && c0 + 4 * e < p.cin;
+                        x[4 * e] = ok ? q.x : 0.f, x[4 * e + 1] = ok ? q.y : 0.f;
+                        x[4 * e + 2] = ok ? q.z : 0.f, x[4 * e + 3] = ok ? q.w : 0.f;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; j++) x[j] = (in && c0 + j < p.cin) ? p.x[px * p.xcs + c0 + j] : 0.f;
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (k0 + u >= steps) break;
+#pragma unroll
+            for (int m = 0; m < RT; m++) {
+                half8 bh, bl;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const _Float16 hv = (_Float16)v[u][m][j];
+                    bh[j] = hv;
+                    bl[j] = (_Float16)(v[u][m][j] - (float)hv);
+                }
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u][t], bh, acc[m][t], 0, 0, 0);
+                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u][t], bl, acc[m][t], 0, 0, 0);
+                    if constexpr (LO) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u][t], bh, acc[m][t], 0, 0, 0);
+                }
+            }
+        }
+    }
+    } else {
     for (int k = 0; k < p.chunks * p.taps; k++) {
         const int c = k / p.taps, tap = k - c * p.taps;
         const int da = p.ty - 1 - tap / p.tx, db = p.tx - 1 - (tap - (tap / p.tx) * p.tx);
@@ -114,6 +177,7 @@ __global__ __launch_bounds__(256) void convt_rows_kernel(CtParams p) {
                 acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], bl[m], acc[m][t], 0, 0, 0);
                 if constexpr (LO) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], bh[m], acc[m][t], 0, 0, 0);
             }
+    }
     }
     // Lane (r, g) holds columns 4g..4g+3 of n-tile t for position 16m + r.
 #pragma unroll
@@ -194,14 +258,19 @@ bool convt_rows(const Act &x, const Act &y, const uint16_t *whi, const uint16_t 
     p.vecx = (x.c % 4 == 0 && x.cs % 4 == 0 && (reinterpret_cast<uintptr_t>(x.p) & 15) == 0) ? 1 : 0;
     p.vecy = (y.c % 4 == 0 && y.cs % 4 == 0 && (reinterpret_cast<uintptr_t>(y.p) & 15) == 0) ? 1 : 0;
     if (p.npx == 0) return true;
-    // 32 positions a wavefront, then 16, then a part of the column block, until there are 2048
-    // wavefronts (8 a CU) or no smaller split.
+    // 32 positions a wavefront, then 16 below 2048 wavefronts (8 a CU), then a part of the column block
+    // until there are 1024 or no smaller split. Up to 2048 wavefronts of 16 positions ask for four
+    // steps at once, which makes up for their number: 256 -> 128 channels, 2 x 3, at 50 x 37 24.2 us
+    // with a step at a time and 3808 wavefronts, 23.3 with four, 18.0 with four and 1904; at 3750
+    // wavefronts (100 x 150 positions) four steps take 14.6 us and one 12.4, and with 32 positions two
+    // steps 22.4 against 16.2.
     const int ntf = pk.bn / 16;
     auto waves = [&](int rt, int ts) { return std::ceil(npx / (16.0 * rt)) * ts * pk.nblocks; };
     int rt = 2, ts = 1;
     if (waves(rt, ts) < 2048) rt = 1;
-    while (waves(rt, ts) < 2048 && ts < ntf) ts *= 2;
+    while (waves(rt, ts) < 1024 && ts < ntf) ts *= 2;
     const int nt = ntf / ts;
+    const bool few = rt == 1 && waves(rt, ts) <= 2048;
     p.rtiles = int((npx + 16 * rt - 1) / (16 * rt));
     p.tsplit = ts;
     const double blocks = std::ceil(double(p.rtiles) * ts / 4);
@@ -211,10 +280,13 @@ bool convt_rows(const Act &x, const Act &y, const uint16_t *whi, const uint16_t 
                      4.0 * (double(x.n) * x.h * x.w * x.c + double(y.n) * y.h * y.w * y.c) +
                          2.0 * double(pk.halves()) * (pk.exact ? 1 : 2));
     const bool lo = !pk.exact;
-#define CT_LAUNCH(RT, NT)                                                                        \
-    do {                                                                                         \
-        if (lo) hipLaunchKernelGGL((convt_rows_kernel<RT, NT, true>), grid, dim3(256), 0, st, p); \
-        else hipLaunchKernelGGL((convt_rows_kernel<RT, NT, false>), grid, dim3(256), 0, st, p);   \
+#define CT_LAUNCH(RT, NT)                                                                                      \
+    do {                                                                                                       \
+        constexpr int U = RT == 1 ? 4 : 1;                                                                     \
+        if (lo && few) hipLaunchKernelGGL((convt_rows_kernel<RT, NT, true, U>), grid, dim3(256), 0, st, p);     \
+        else if (lo) hipLaunchKernelGGL((convt_rows_kernel<RT, NT, true, 1>), grid, dim3(256), 0, st, p);       \
+        else if (few) hipLaunchKernelGGL((convt_rows_kernel<RT, NT, false, U>), grid, dim3(256), 0, st, p);     \
+        else hipLaunchKernelGGL((convt_rows_kernel<RT, NT, false, 1>), grid, dim3(256), 0, st, p);              \
     } while (0)
     if (rt == 2) {
         if (nt == 1) CT_LAUNCH(2, 1);
