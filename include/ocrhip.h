@@ -194,7 +194,8 @@ int ocr_recognize_device(ocr_recognizer *rec, const ocr_batch *d_batches, uint32
  * "conv_mfma", "gru", "conv_transpose", "conv_direct", "conv_generic", "maxpool", "mask_up",
  * "grey_resize", "line_crop", "avgpool_t", "argmax", "copy") is bracketed by HIP events on its
  * own stream. stop waits for them and returns the launches, their summed duration in ms and
- * their summed algorithmic FLOPs and bytes. */
+ * their summed algorithmic FLOPs and bytes. Where a family has several kernels that a rule on
+ * sizes picks from, each is a name of its own as well ("gemm_thin" of "gemm_dma"). */
 int ocr_probe_start(const char *family);
 int ocr_probe_stop(const char *family, uint32_t *calls, double *ms, double *flops, double *bytes);
 

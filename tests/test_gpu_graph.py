@@ -61,17 +61,33 @@ def test_conv1x1_gemm(ctx, tmp_path, cin, cout, h, w, act):
     check(ctx, p, RNG.standard_normal((1, cin, h, w)).astype(np.float32))
 
 
-@pytest.mark.parametrize("cin,cout,w,act", [(512, 97, 1, None), (256, 97, 50, "Relu"), (512, 97, 5003, None),
-                                            (132, 40, 30001, "Sigmoid"), (132, 150, 12003, None), (512, 1536, 321, None),
-                                            (128, 272, 82001, "Relu"), (256, 64, 1537, None)])
-def test_conv1x1_row_counts(ctx, tmp_path, cin, cout, w, act):
+@pytest.mark.parametrize("cin,cout,w,act,form", [
+    (512, 97, 1, None, "gemm_thin"), (256, 97, 50, "Relu", "gemm_thin"), (512, 97, 5003, None, "gemm_tile_128"),
+    (132, 40, 30001, "Sigmoid", "gemm_tile_128"), (132, 150, 12003, None, "gemm_tile_256"),
+    (512, 1536, 321, None, "gemm_tile_256"), (128, 272, 82001, "Relu", "gemm_persistent"), (256, 64, 1537, None, "gemm_thin")])
+def test_conv1x1_row_counts(ctx, tmp_path, cin, cout, w, act, form):
     # The GEMM's three forms at the edges of their tiles: one row, few rows (16 x 16), 128 and 64
     # row tiles with a part of a tile left, K and N that end inside a slice or tile, and enough
     # 256 x 256 tiles for the persistent form.
     p = build(tmp_path, "g1r", lambda g, x: conv(g, x, cin, cout, k=(1, 1), pads=(0, 0, 0, 0), act=act), (1, cin, 1, w))
     x = RNG.standard_normal((1, cin, 1, w)).astype(np.float32)
-    _, calls = _ran(FAST, lambda: check(ctx, p, x))
-    assert calls["gemm_dma"] >= 1, calls
+    _, calls = _ran(("gemm_dma", form), lambda: check(ctx, p, x))
+    assert calls["gemm_dma"] == calls[form] == 1, calls
+
+
+@pytest.mark.parametrize("cin,cout,exact", [(128, 272, True), (160, 300, False)])
+def test_conv1x1_forms_same_bits(ctx, tmp_path, cin, cout, exact):
+    # A row gives the same bits in every form of the GEMM: all rows, then some of them alone.
+    import ocrhip
+    p = build(tmp_path, "g1b", lambda g, x: conv(g, x, cin, cout, k=(1, 1), pads=(0, 0, 0, 0), exact=exact), (1, cin, 1, 64))
+    gr = ocrhip.Graph(ctx, p)
+    x = RNG.standard_normal((1, cin, 1, 82001)).astype(np.float32)
+    whole = None
+    for w, form in ((82001, "gemm_persistent"), (9001, "gemm_tile_256"), (35, "gemm_thin")):
+        got, calls = _ran((form,), lambda: gr.run(np.ascontiguousarray(x[..., :w])))
+        assert calls[form] == 1, (form, calls)
+        whole = got if whole is None else whole
+        assert np.array_equal(got, whole[..., :w]), form
 
 
 def test_conv1x1_and_sigmoid(ctx, tmp_path):
@@ -329,10 +345,11 @@ def test_shape_errors(ctx, tmp_path):
         gr.run(np.zeros((1, 3, 5, 5), np.float32))  # wrong channel count
 
 
-@pytest.mark.parametrize("n,cin,cout,h,w,pool", [(1, 32, 64, 40, 300, (2, 2)), (2, 64, 32, 61, 150, None), (3, 128, 256, 4, 301, (2, 1)),
-                                                 (1, 48, 20, 119, 203, None), (1, 16, 32, 1, 3, None), (1, 40, 16, 2, 8, (2, 1)),
-                                                 (1, 36, 17, 5, 9, (2, 2))])
-def test_conv3x3_both_forms(ctx, tmp_path, n, cin, cout, h, w, pool):
+@pytest.mark.parametrize("n,cin,cout,h,w,pool,form", [
+    (1, 32, 64, 40, 300, (2, 2), "conv3_persistent"), (2, 64, 32, 61, 150, None, "conv3_persistent"),
+    (3, 128, 256, 4, 301, (2, 1), "conv3_persistent"), (1, 48, 20, 119, 203, None, "conv3_persistent"),
+    (1, 16, 32, 1, 3, None, "conv3_thin"), (1, 40, 16, 2, 8, (2, 1), "conv3_thin"), (1, 36, 17, 5, 9, (2, 2), "conv3_thin")])
+def test_conv3x3_both_forms(ctx, tmp_path, n, cin, cout, h, w, pool, form):
     # Enough pixels for the persistent kernel's tiles, and few ones for the direct form: odd sizes,
     # channels that end inside a slice and block, inexact weights every second case.
     def net(g, x):
@@ -340,8 +357,25 @@ def test_conv3x3_both_forms(ctx, tmp_path, n, cin, cout, h, w, pool):
         return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
     p = build(tmp_path, "c3f", net, (n, cin, h, w))
     x = RNG.standard_normal((n, cin, h, w)).astype(np.float32)
-    _, calls = _ran(FAST, lambda: check(ctx, p, x))
-    assert calls["conv3x3_dma"] >= 1, calls
+    _, calls = _ran(("conv3x3_dma", form), lambda: check(ctx, p, x))
+    assert calls["conv3x3_dma"] == calls[form] == 1, calls
+
+
+@pytest.mark.parametrize("cin,cout,pool,exact", [(32, 64, None, True), (64, 48, (2, 2), False), (128, 256, (2, 1), True)])
+def test_conv3x3_forms_same_bits(ctx, tmp_path, cin, cout, pool, exact):
+    # An image gives the same bits alone (conv3_thin) as among many (the persistent kernel).
+    import ocrhip
+    def net(g, x):
+        y = conv(g, x, cin, cout, act="Relu", exact=exact)
+        return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
+    p = build(tmp_path, "c3b", net, (1, cin, 14, 45))
+    gr = ocrhip.Graph(ctx, p)
+    x = RNG.standard_normal((24, cin, 14, 45)).astype(np.float32)
+    many, calls = _ran(("conv3_persistent",), lambda: gr.run(x))
+    assert calls["conv3_persistent"] == 1, calls
+    one, calls = _ran(("conv3_thin",), lambda: gr.run(x[5:6]))
+    assert calls["conv3_thin"] == 1, calls
+    assert np.array_equal(one[0], many[5])
 
 
 @pytest.mark.parametrize("cin,cout,h,w,pool,two", [(32, 64, 17, 45, (2, 2), False), (64, 128, 16, 37, (2, 1), False),

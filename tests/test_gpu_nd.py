@@ -42,6 +42,15 @@ def check(ctx, path, x, tol=1e-4, stop=False):
     return got, want
 
 
+def ran(names, fn):
+    """Runs fn with the kernel families or forms probed; returns {name: launches}."""
+    import ocrhip
+    for f in names:
+        ocrhip.probe_start(f)
+    fn()
+    return {f: ocrhip.probe_stop(f)["calls"] for f in names}
+
+
 def w(g, shape, fan, exact=True):
     a = RNG.standard_normal(shape).astype(np.float32) * np.float32(np.sqrt(2 / fan))
     return g.init(g.fresh("w"), f16x(a) if exact else a)
@@ -288,7 +297,8 @@ def test_linear_many_columns(ctx, tmp_path, rows, k, n, exact):
         y = g.add("MatMul", [x, w(g, (k, n), k, exact=exact)])
         return g.add("Add", [y, g.init("lb", (RNG.standard_normal(n) * 0.1).astype(np.float32))])
     p = build(tmp_path, "wide", fn, (1, rows, k))
-    check(ctx, p, RNG.standard_normal((1, rows, k)).astype(np.float32))
+    x = RNG.standard_normal((1, rows, k)).astype(np.float32)
+    assert ran(["nd_rows_wide"], lambda: check(ctx, p, x)) == {"nd_rows_wide": 1}
 
 
 @pytest.mark.parametrize("k,n,exact", [(120, 200, True), (256, 300, False), (64, 1000, True)])
@@ -325,7 +335,8 @@ def test_head_argmax_first_index_on_ties(ctx, tmp_path, k, n, exact):
 def test_depthwise_row_ends(ctx, tmp_path, c, h, wd, stride, k):
     # Rows that end inside or before a 16-byte load, at every shift.
     p = build(tmp_path, "dwe", lambda g, x: conv(g, x, c, c, k=k, stride=stride, group=c, exact=False), (2, c, h, wd))
-    check(ctx, p, RNG.standard_normal((2, c, h, wd)).astype(np.float32))
+    x = RNG.standard_normal((2, c, h, wd)).astype(np.float32)
+    assert ran(["nd_conv_dw", "nd_conv_dw_wide"], lambda: check(ctx, p, x)) == {"nd_conv_dw": 1, "nd_conv_dw_wide": int(wd >= 4)}
 
 
 @pytest.mark.parametrize("cin,cout,h,wd,s", [(6, 5, 7, 9, 2), (4, 3, 16, 17, 2), (3, 6, 5, 5, 1), (4, 2, 3, 3, 3)])
@@ -383,7 +394,9 @@ def test_fused_attention_shapes(ctx, tmp_path, n, t, dim, heads):
     import ocrhip
     p = build(tmp_path, "attn", lambda g, x: _attention(g, x, dim, heads), (n, t, dim))
     assert any(line.startswith("attention") for line in ocrhip.nd_plan(p))
-    check(ctx, p, RNG.standard_normal((n, t, dim)).astype(np.float32))
+    x = RNG.standard_normal((n, t, dim)).astype(np.float32)
+    calls = ran(["nd_attention", "nd_attention_mfma"], lambda: check(ctx, p, x))
+    assert calls == {"nd_attention": 1, "nd_attention_mfma": int(4 <= dim // heads <= 16)}
 
 
 def _pool2(g, x):
@@ -435,7 +448,32 @@ def test_conv_of_two_tensors(ctx, tmp_path, n, c1, c2, h, w, k):
         b = g.add("Relu", [conv(g, x, 16, c2, k=1)])
         return g.add("Relu", [conv(g, g.add("Concat", [a, b], axis=1), c1 + c2, 40, k=k)])
     p = build(tmp_path, "two", fn, (n, 16, h, w))
-    check(ctx, p, RNG.standard_normal((n, 16, h, w)).astype(np.float32))
+    x = RNG.standard_normal((n, 16, h, w)).astype(np.float32)
+    assert ran(["nd_copy"], lambda: check(ctx, p, x)) == {"nd_copy": 2 if c1 % 32 else 0}
+
+
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("scale,up", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("n,c1,c2,h,w", [(2, 32, 40, 6, 50), (1, 64, 8, 2, 26)])
+def test_conv_of_two_tensors_scaled(ctx, tmp_path, n, c1, c2, h, w, k, scale, up, exact):
+    # The same with an input scale, whose channels run on over both tensors (the second ends inside
+    # a chunk), and with an upscaled residual, read where they lie.
+    c, cout = c1 + c2, 24
+    def fn(g, x):
+        a = g.add("Relu", [conv(g, x, 16, c1, k=1)])
+        b = g.add("Relu", [conv(g, x, 16, c2, k=1)])
+        y = g.add("Concat", [a, b], axis=1)
+        if scale:
+            se = conv(g, g.add("GlobalAveragePool", [x]), 16, c, k=1)
+            y = g.add("Mul", [y, g.add("HardSigmoid", [se], alpha=0.2, beta=0.5)])
+        y = conv(g, y, c, cout, k=k, exact=exact)
+        if up:
+            y = g.add("Add", [y, _up(g, _pool2(g, conv(g, x, 16, cout, k=1)), 2.0)])
+        return g.add("Sigmoid", [y])
+    p = build(tmp_path, "twos", fn, (n, 16, h, w))
+    x = RNG.standard_normal((n, 16, h, w)).astype(np.float32)
+    assert ran(["nd_copy", "nd_resize"], lambda: check(ctx, p, x)) == {"nd_copy": 0, "nd_resize": 0}
 
 
 @pytest.mark.parametrize("cin,cout,h,w,exact", [(7, 20, 3, 5, True), (64, 16, 9, 31, False), (100, 70, 12, 40, True),
@@ -447,7 +485,8 @@ def test_1x1_nchw_channel_edges(ctx, tmp_path, cin, cout, h, w, exact):
         y = conv(g, x, cin, cout, k=1, exact=exact)
         return g.add("Add", [g.add("Relu", [conv(g, y, cout, cout, k=1, exact=exact)]), y])
     p = build(tmp_path, "c1e", fn, (2, cin, h, w))
-    check(ctx, p, RNG.standard_normal((2, cin, h, w)).astype(np.float32))
+    x = RNG.standard_normal((2, cin, h, w)).astype(np.float32)
+    assert ran(["nd_conv_px"], lambda: check(ctx, p, x)) == {"nd_conv_px": 2}
 
 
 def _layer_norm(g, x, k):
@@ -477,7 +516,10 @@ def test_transformer_block_shapes(ctx, tmp_path, n, t, dim, heads, hidden, exact
         x = g.add("Add", [x, _linear(g, y, hidden, dim, exact)])
         return g.add("Sqrt", [g.add("Relu", [x])])
     p = build(tmp_path, "block", fn, (n, t, dim))
-    check(ctx, p, RNG.standard_normal((n, t, dim)).astype(np.float32))
+    x = RNG.standard_normal((n, t, dim)).astype(np.float32)
+    calls = ran(["nd_layer_norm", "nd_rows_norm", "nd_mlp", "nd_attention_proj"], lambda: check(ctx, p, x))
+    fits = dim <= 128
+    assert calls == {"nd_layer_norm": 0 if fits else 2, "nd_rows_norm": int(fits), "nd_mlp": int(fits), "nd_attention_proj": 1}
 
 
 def test_output_memory(ctx, tmp_path):

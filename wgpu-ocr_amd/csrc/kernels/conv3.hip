@@ -759,7 +759,7 @@ void c3_launch(const ConvArgs *args, int count, int pool, hipStream_t s) {
     p.runs = std::max(1, std::min(p.tiles, cus / p.nblocks));
     p.zero = zero_block();
     const int grid = p.runs * p.nblocks;
-    ProbeScope probe("conv3x3_dma", s, flops, bytes);
+    ProbeScope probe("conv3x3_dma", s, flops, bytes, few ? "conv3_thin" : "conv3_persistent");
     auto launch = [&](auto ACTc) {
         constexpr int A = decltype(ACTc)::value;
         // 16 wavefronts (4 a SIMD): 128-channel blocks as 4 x 4 wavefronts of 2 n-tiles, 64-channel

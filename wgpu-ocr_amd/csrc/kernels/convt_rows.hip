@@ -278,7 +278,7 @@ bool convt_rows(const Act &x, const Act &y, const uint16_t *whi, const uint16_t 
     const dim3 grid{unsigned(blocks), unsigned(pk.nblocks)};
     ProbeScope probe("conv_transpose", st, 2.0 * npx * p.taps * double(x.c) * pk.cout,
                      4.0 * (double(x.n) * x.h * x.w * x.c + double(y.n) * y.h * y.w * y.c) +
-                         2.0 * double(pk.halves()) * (pk.exact ? 1 : 2));
+                         2.0 * double(pk.halves()) * (pk.exact ? 1 : 2), few ? "convt_four_steps" : "convt_one_step");
     const bool lo = !pk.exact;
 #define CT_LAUNCH(RT, NT)                                                                                      \
     do {                                                                                                       \

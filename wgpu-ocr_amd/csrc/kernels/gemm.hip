@@ -592,7 +592,8 @@ bool gemm_dma(const ConvArgs &a, hipStream_t s) {
     const dim3 grid{unsigned(blocks)};
     const double flops = 2.0 * p.M * double(N) * K;
     const double bytes = 4.0 * (double(p.M) * K + double(p.M) * N) + 2.0 * double(pk.frag_halves());
-    ProbeScope probe("gemm_dma", s, flops, bytes);
+    ProbeScope probe("gemm_dma", s, flops, bytes,
+                     few ? "gemm_thin" : many ? "gemm_persistent" : narrow ? "gemm_tile_128" : "gemm_tile_256");
     auto launch = [&](auto ACTc) {
         constexpr int A = decltype(ACTc)::value;
         if (few) hipLaunchKernelGGL((gemm_thin_kernel<A>), grid, dim3(256), 0, s, p);

@@ -423,7 +423,8 @@ void nd_rows_block(const NdRowsArgs &a, const NdRowsArgs *b, hipStream_t s) {
     p.w1 = packed(a);
     if (b) p.w2 = packed(*b);
     ProbeScope probe("nd_gemm_rows", s, 2.0 * a.m * (double(a.k) * a.n + (b ? double(b->k) * b->n : 0.0)),
-                     4.0 * a.m * (double(a.k) + (b ? b->n : a.n)) + weight_bytes(a) + (b ? weight_bytes(*b) : 0.0));
+                     4.0 * a.m * (double(a.k) + (b ? b->n : a.n)) + weight_bytes(a) + (b ? weight_bytes(*b) : 0.0),
+                     b ? "nd_mlp" : "nd_rows_norm");
     const dim3 grid{unsigned((a.m + 15) / 16)};
     const bool lo = p.w1.lo || p.w2.lo;
     if (b && lo) hipLaunchKernelGGL((rows_block_kernel<true, true>), grid, dim3(512), 0, s, p);
@@ -461,7 +462,7 @@ void nd_attention_proj(const float *x, int n, int t, int heads, int d, float sca
     p.w = packed(w);
     const double tt = double(t), m = double(n) * t;
     ProbeScope probe("nd_attention", s, 4.0 * n * heads * tt * tt * d + 2.0 * m * w.k * w.n,
-                     4.0 * m * (3.0 * w.k + w.n) + weight_bytes(w));
+                     4.0 * m * (3.0 * w.k + w.n) + weight_bytes(w), "nd_attention_proj");
     const dim3 grid{unsigned(n * p.qtiles)}, block{unsigned(64 * std::min(heads, 8))};
     if (p.w.lo) hipLaunchKernelGGL((attention_proj_kernel<true>), grid, block, 0, s, p);
     else hipLaunchKernelGGL((attention_proj_kernel<false>), grid, block, 0, s, p);
@@ -473,7 +474,8 @@ bool nd_attention_mfma(const float *x, int n, int t, int heads, int d, float sca
     if (n <= 0 || t <= 0) return true;
     const AttnParams p = attn_params(x, n, t, heads, d, scale, y);
     const double tt = double(t);
-    ProbeScope probe("nd_attention", s, 4.0 * n * heads * tt * tt * d, 4.0 * n * tt * (3.0 * heads * d + heads * d));
+    ProbeScope probe("nd_attention", s, 4.0 * n * heads * tt * tt * d, 4.0 * n * tt * (3.0 * heads * d + heads * d),
+                     "nd_attention_mfma");
     hipLaunchKernelGGL(attention_kernel, dim3(unsigned(n * p.qtiles), unsigned((heads + 3) / 4)), dim3(256), 0, s, p);
     OCR_HIP(hipGetLastError());
     return true;

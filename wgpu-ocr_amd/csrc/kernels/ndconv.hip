@@ -889,7 +889,7 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
     const double flops = 2.0 * a.n * a.oh * a.ow * a.cout * a.cin * pk.kh * pk.kw;
     const double bytes = 4.0 * (double(a.n) * a.h * a.w * a.cin + double(a.n) * a.oh * a.ow * a.cout) +
                          2.0 * double(pk.halves()) * (pk.exact ? 1 : 2);
-    ProbeScope probe("nd_conv_nchw", s, flops, bytes);
+    ProbeScope probe("nd_conv_nchw", s, flops, bytes, px ? "nd_conv_px" : ks > 1 ? "nd_conv_split" : "nd_conv_direct");
     const bool lo = !pk.exact;
     if (px && nt == 1) launch_px_kc<1>(p, lo, grid, s);
     else if (px && nt == 2) launch_px_kc<2>(p, lo, grid, s);
@@ -928,9 +928,9 @@ bool nd_conv_dw(const NdConvArgs &a, hipStream_t s) {
     const double blocks = double(p.tiles_plane) * planes;
     if (blocks > 0x7fffffff) return false;
     const dim3 grid{unsigned(blocks)};
-    ProbeScope probe("nd_conv_dw", s, 2.0 * double(planes) * opl * a.kh * a.kw,
-                     4.0 * (double(planes) * a.h * a.w + double(planes) * opl));
     const bool wide = a.w >= 4 && a.pl == a.kw / 2;
+    ProbeScope probe("nd_conv_dw", s, 2.0 * double(planes) * opl * a.kh * a.kw,
+                     4.0 * (double(planes) * a.h * a.w + double(planes) * opl), wide ? "nd_conv_dw_wide" : nullptr);
     bool ok;
     if (wide) ok = a.kh == 3 ? launch_dw<3, true>(p, a.sh, a.sw, grid, s) : launch_dw<5, true>(p, a.sh, a.sw, grid, s);
     else ok = a.kh == 3 ? launch_dw<3, false>(p, a.sh, a.sw, grid, s) : launch_dw<5, false>(p, a.sh, a.sw, grid, s);
@@ -1022,7 +1022,7 @@ bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s) {
         const double groups = std::ceil(double(p.rtiles) * p.parts / 4);
         if (groups > 0x7fffffff) return false;
         ProbeScope probe("nd_gemm_rows", s, 2.0 * a.m * double(a.k) * a.n,
-                         4.0 * (double(a.m) * a.k + double(a.m) * a.n) + 2.0 * double(pk.halves()) * (lo ? 2 : 1));
+                         4.0 * (double(a.m) * a.k + double(a.m) * a.n) + 2.0 * double(pk.halves()) * (lo ? 2 : 1), "nd_rows_wide");
         const dim3 grid{unsigned(groups)};
         if (lo && k8) hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 8, true>), grid, dim3(256), 0, s, p);
         else if (lo) hipLaunchKernelGGL((gemm_rows_wide_kernel<2, 4, true>), grid, dim3(256), 0, s, p);

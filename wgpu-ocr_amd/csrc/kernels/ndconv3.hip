@@ -211,7 +211,7 @@ bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hi
     double in = 0;
     for (int k = 0; k < nsrc; k++) in += double(a.n) * src[k].c * src[k].h * src[k].w;
     ProbeScope probe("nd_conv_nchw", s, 2.0 * px * a.cout * a.cin * 9,
-                     4.0 * (in + px * a.cout) + 2.0 * double(pk.halves()) * (pk.exact ? 1 : 2));
+                     4.0 * (in + px * a.cout) + 2.0 * double(pk.halves()) * (pk.exact ? 1 : 2), "nd_conv_tile");
     const dim3 grid{unsigned(blocks), unsigned(pk.nblocks)};
     auto launch = [&](auto *exact, auto *lo) {
         if (pk.exact) hipLaunchKernelGGL(exact, grid, dim3(256), 0, s, p);

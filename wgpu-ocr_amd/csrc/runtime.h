@@ -115,21 +115,26 @@ class Probe {
     hipEvent_t take();
 };
 
-// Brackets one launch when its family is probed (no cost otherwise beyond a flag check).
+// Brackets one launch when its family is probed (no cost otherwise beyond a flag check). form:
+// the kernel that a family with several picked for this launch, a name of its own to probe.
 class ProbeScope {
   public:
-    ProbeScope(const char *family, hipStream_t s, double flops, double bytes) : fam_(family), s_(s) {
-        on_ = Probe::get().active(family);
-        if (on_) Probe::get().record(fam_, s_, true, flops, bytes);
+    ProbeScope(const char *family, hipStream_t s, double flops, double bytes, const char *form = nullptr)
+        : names_{family, form}, s_(s) {
+        for (int k = 0; k < 2; k++) {
+            on_[k] = names_[k] && Probe::get().active(names_[k]);
+            if (on_[k]) Probe::get().record(names_[k], s_, true, flops, bytes);
+        }
     }
     ~ProbeScope() {
-        if (on_) Probe::get().record(fam_, s_, false, 0, 0);
+        for (int k = 0; k < 2; k++)
+            if (on_[k]) Probe::get().record(names_[k], s_, false, 0, 0);
     }
 
   private:
-    const char *fam_;
+    const char *names_[2];
     hipStream_t s_;
-    bool on_ = false;
+    bool on_[2] = {false, false};
 };
 
 // A pooled device buffer owned by one holder; goes back to the pool when destroyed. Its work
