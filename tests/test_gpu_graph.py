@@ -144,20 +144,52 @@ def test_conv1x1_inexact_weights(ctx, tmp_path, cin, cout, h, w, fam):
 
 @pytest.mark.parametrize("cout,pool,h,w", [(16, None, 3, 1), (32, (2, 2), 64, 37), (64, (2, 2), 50, 131), (48, None, 17, 65)])
 def test_direct_conv_inexact_weights(ctx, tmp_path, cout, pool, h, w):
-    # One-channel 3 x 3 convs with float32 weights that are not float16 values (their remainders
-    # go through the matrix cores too), at tile edges. check's bound is that of every split conv:
-    # the parts stand for the weights to 2^-23 of the channel's largest.
+    # One-channel 3 x 3 convs with float32 weights that are not float16 values (float32 products on
+    # the matrix cores), at tile edges.
     def net(g, x):
         y = conv(g, x, 1, cout, exact=False, act="Relu")
         return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
     p = build(tmp_path, "d1i", net, (2, 1, h, w))
-    check(ctx, p, RNG.uniform(-0.5, 0.5, (2, 1, h, w)).astype(np.float32))
+    x = RNG.uniform(-0.5, 0.5, (2, 1, h, w)).astype(np.float32)
+    _, calls = _ran(("conv_direct", "conv1_f32"), lambda: check(ctx, p, x))
+    assert calls == {"conv_direct": 1, "conv1_f32": 1}
+
+
+@pytest.mark.parametrize("pool", [None, (2, 2)])
+@pytest.mark.parametrize("scale", [1, 2.0 ** -24, 2.0 ** 40])
+def test_direct_conv_float32_products(ctx, tmp_path, pool, scale):
+    # Float32 weights and inputs go into the products whole, whatever their range: a kernel with one
+    # tap gives each product rounded once, bit for bit, also for inputs that float16 parts would
+    # cut off or overflow. With nine taps the error is a float32 sum's: nine products and eight
+    # additions, each half an ulp (2^-24) of at most the sum of the magnitudes.
+    def run(w):
+        def net(g, x):
+            y = g.add("Conv", [x, g.init("ws", w), g.init("b", np.zeros(16, np.float32))], kernel_shape=[3, 3],
+                      pads=[1, 1, 1, 1], strides=[1, 1])
+            return g.add("MaxPool", [y], kernel_shape=list(pool), strides=list(pool)) if pool else y
+        import ocrhip
+        got, calls = _ran(("conv1_f32",), lambda: ocrhip.Graph(ctx, build(tmp_path, "d1p", net, x.shape)).run(x))
+        assert calls["conv1_f32"] == 1
+        return got[0]
+
+    def pooled(a):
+        return a if not pool else a.reshape(16, 9, 2, 17, 2).max((2, 4))
+    x = (RNG.standard_normal((1, 1, 18, 34)) * scale).astype(np.float32)
+    xp = np.pad(x[0, 0], 1)
+    taps = np.stack([xp[i: i + 18, j: j + 34] for i in range(3) for j in range(3)])
+    one = np.zeros((16, 9), np.float32)
+    at = np.arange(16) % 9
+    one[np.arange(16), at] = RNG.standard_normal(16).astype(np.float32)
+    assert np.array_equal(run(one.reshape(16, 1, 3, 3)), pooled(one[np.arange(16), at][:, None, None] * taps[at]))
+    w = RNG.standard_normal((16, 9)).astype(np.float32)
+    want = np.einsum("ct,tyx->cyx", w.astype(np.float64), taps.astype(np.float64))
+    bound = 17 * 2.0 ** -24 * np.einsum("ct,tyx->cyx", np.abs(w).astype(np.float64), np.abs(taps).astype(np.float64))
+    assert (np.abs(run(w.reshape(16, 1, 3, 3)) - pooled(want)) <= pooled(bound)).all()
 
 
 @pytest.mark.parametrize("scale,small", [(1e6, 1), (1e-4, 1), (1, 1e-3), (1, 1e-7)])
 def test_direct_conv_weight_ranges(ctx, tmp_path, scale, small):
-    # Weights far from 1 are scaled before they are split; a channel far below the others (the
-    # last) keeps the layer on the float32 kernel. Compared relative to each channel's largest
+    # Weights far from 1, and a channel far below the others. Compared relative to each channel's largest
     # output: 9 products, each to 2^-21 of the largest weight and input.
     w = (RNG.standard_normal((16, 1, 3, 3)) * scale).astype(np.float32)
     w[3] *= np.float32(small)

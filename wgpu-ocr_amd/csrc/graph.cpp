@@ -8,6 +8,7 @@
 #include "graph.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <map>
 #include <memory>
@@ -118,10 +119,20 @@ Graph Graph::build(Ctx &ctx, const Onnx &onnx, const char *stop, Node *stop_node
                 }
                 s.w = ctx.upload_weights(w.data.data(), w.data.size());
                 if (kh == 3 && kw == 3 && cout % 16 == 0 && cout <= 64) {
-                    std::vector<uint16_t> frag(size_t(cout) / 16 * 64 * 8), lo(frag.size());
-                    const int parts = pack_conv1_frags(w.data.data(), cout, frag.data(), lo.data(), &s.w1unscale);
-                    if (parts >= 1) s.w1frag = ctx.upload_weights(frag.data(), frag.size());
-                    if (parts == 2) s.w1frag_lo = ctx.upload_weights(lo.data(), lo.size());
+                    bool exact = true, finite = true;
+                    for (float v : w.data) {
+                        exact = exact && float(_Float16(v)) == v;
+                        finite = finite && std::isfinite(v);
+                    }
+                    if (exact) {
+                        std::vector<uint16_t> frag(size_t(cout) / 16 * 64 * 8);
+                        pack_conv1_frags(w.data.data(), cout, frag.data());
+                        s.w1frag.f16 = ctx.upload_weights(frag.data(), frag.size());
+                    } else if (finite) {
+                        std::vector<float> frag(size_t(cout) * 12);
+                        pack_conv1_f32(w.data.data(), cout, frag.data());
+                        s.w1frag.f32 = ctx.upload_weights(frag.data(), frag.size());
+                    }
                 }
             } else if (group == 1) {
                 s.kind = OpKind::Conv;
@@ -541,9 +552,9 @@ struct Graph::Exec {
     void direct_fallback(size_t i, const Act &a, const Act &y, const Act &yp) {
         const Step &s = g.steps[i];
         if (s.pool_output.empty()) {
-            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, s.ph, s.pw, st, s.w1frag, s.w1frag_lo, s.w1unscale);
+            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, s.ph, s.pw, st, s.w1frag);
         } else {
-            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, 1, 1, st, s.w1frag, s.w1frag_lo, s.w1unscale);
+            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, 1, 1, st, s.w1frag);
             maxpool(y, yp, s.ph, s.pw, st);
         }
     }
@@ -572,8 +583,8 @@ void Graph::Exec::step(size_t i) {
         Act yp;
         direct_views(i, y, yp);
         if (s.pool_output.empty()) {
-            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, s.ph, s.pw, st, s.w1frag, s.w1frag_lo, s.w1unscale);
-        } else if (!(direct_mfma(i) && conv1_mfma(a, y, s.w1frag, s.w1frag_lo, s.w1unscale, s.b, s.act, s.ph, s.pw, st, &yp))) {
+            conv_direct(a, y, s.w, s.b, s.kh, s.kw, s.pt, s.act, s.ph, s.pw, st, s.w1frag);
+        } else if (!(direct_mfma(i) && conv1_mfma(a, y, s.w1frag, s.b, s.act, s.ph, s.pw, st, &yp))) {
             direct_fallback(i, a, y, yp);
         }
         break;
@@ -767,8 +778,8 @@ bool Graph::run_multi_tm(Ctx &ctx, const std::vector<Act> &xs, int kh, float *X,
                 es[k]->direct_views(i, ys[k], yps[k]);
             }
             const bool pooled = !s.pool_output.empty();
-            if (!conv1_mfma_multi(as.data(), ys.data(), pooled ? yps.data() : nullptr, int(es.size()), s.w1frag,
-                                  s.w1frag_lo, s.w1unscale, s.b, s.act, s.ph, s.pw, ctx.stream()))
+            if (!conv1_mfma_multi(as.data(), ys.data(), pooled ? yps.data() : nullptr, int(es.size()), s.w1frag, s.b,
+                                  s.act, s.ph, s.pw, ctx.stream()))
                 for (size_t k = 0; k < es.size(); k++) es[k]->direct_fallback(i, as[k], ys[k], yps[k]);
             for (size_t k = 0; k < es.size(); k++) es[k]->done(i, ys[k]);
         } else if (all && es.size() > 1) {

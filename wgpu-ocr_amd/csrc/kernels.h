@@ -102,25 +102,28 @@ void conv1x1_narrow(const Act &x, const Act &y, const float *w, const float *b, 
 // Any conv (grouped, strided) in float32, one thread per output: the fallback path.
 void conv_generic(const Act &x, const Act &y, const float *w, const float *b, int kh, int kw, int sh, int sw,
                   int pt, int pl, int group, int act, hipStream_t s);
+// Weights of conv1_mfma: float16 fragments when every weight is a float16 value, else float32 ones.
+struct Conv1Frags {
+    const uint16_t *f16 = nullptr;
+    const float *f32 = nullptr;
+    explicit operator bool() const { return f16 || f32; }
+};
 // One input channel, stride 1, act, and a fused MaxPool (ph, pw) (gpu.rs:385-422).
 void conv_direct(const Act &x, const Act &y, const float *w, const float *b, int kh, int kw, int pad, int act,
-                 int ph, int pw, hipStream_t s,
-                 const uint16_t *frag = nullptr, const uint16_t *frag_lo = nullptr, float unscale = 1.f);
+                 int ph, int pw, hipStream_t s, const Conv1Frags &frag = {});
 // The matrix-core path of conv_direct (kernels/conv1.hip): 3 x 3, pad 1, 16 to 64 output channels
-// (a multiple of 16), no pool or a 2 x 2 one. Returns false for anything else. pack_conv1_frags
-// packs the weights ([cout][9] float32 in, cout / 16 KiB of float16 fragments out, and as much
-// of their remainders), scaled by a power of two that *unscale undoes. It returns how many of the
-// two the kernel needs: 1 when every weight is a float16 value (frag_lo is then null), 2 when the
-// two parts stand for the weights to 2^-23 of their channel's largest, 0 when they do not (a
-// channel 2^14 below the largest, a weight that is no number).
-int pack_conv1_frags(const float *w, int cout, uint16_t *frag, uint16_t *frag_lo, float *unscale);
+// (a multiple of 16), no pool or a 2 x 2 one. Returns false for anything else. The weights
+// [cout][9] are packed by pack_conv1_frags (float16 values only; cout / 16 KiB of fragments) or by
+// pack_conv1_f32 (any finite ones; cout * 12 floats).
+void pack_conv1_frags(const float *w, int cout, uint16_t *frag);
+void pack_conv1_f32(const float *w, int cout, float *frag);
 // With ypool (2 x 2 pool, full-size y) both outputs are written.
-bool conv1_mfma(const Act &x, const Act &y, const uint16_t *frag, const uint16_t *frag_lo, float unscale, const float *b, int act,
-                int ph, int pw, hipStream_t s, const Act *ypool = nullptr);
+bool conv1_mfma(const Act &x, const Act &y, const Conv1Frags &frag, const float *b, int act, int ph, int pw,
+                hipStream_t s, const Act *ypool = nullptr);
 // The same over count inputs of one height (any widths and image counts), one launch for up to
 // 32 of them; ypool is null or an array of count pooled outputs.
-bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, const uint16_t *frag,
-                      const uint16_t *frag_lo, float unscale, const float *b, int act, int ph, int pw, hipStream_t s);
+bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, const Conv1Frags &frag, const float *b,
+                      int act, int ph, int pw, hipStream_t s);
 // ConvTranspose gather form (gpu.rs:424-460); w re-laid out as [ky][kx][cin][cout].
 void conv_transpose(const Act &x, const Act &y, const float *w, const float *b, int kh, int kw, int stride,
                     int act, hipStream_t s);

@@ -4,8 +4,7 @@
 //
 // One v_mfma_f32_16x16x32_f16 gives 16 output channels of 16 pixels: the K = 32 side holds the
 // pixel's 3 x 3 patch twice, as float16 hi parts (k 0-15) and float16 remainders lo (k 16-31) of
-// the float32 input (x = hi + lo to about 2^-22), against the float16 weights; weights that are
-// not all float16 values take a second instruction, against their float16 remainders. Each half
+// the float32 input (x = hi + lo to about 2^-22), against the exact float16 weights. Each half
 // holds the patch's three rows as (left, centre, right, 0) quadruples and a fourth quadruple the
 // zero weights cancel. The weights are the A operand, so a lane's 4 accumulators are 4
 // neighbouring output channels of one pixel and leave as one 16-byte NHWC store; for a pooled-only
@@ -20,9 +19,16 @@
 // twice. A wavefront takes groups of 16 pixels laid out as four 2 x 2 squares (a fused pool is a
 // max over 4 neighbouring lanes, or over a lane's own accumulators in the pooled-only form).
 //
-// Bound by its stores (32 channels a pixel against 1 read). The second instruction hides under
-// them: with trained (float32) weights the first layer of 36 recogniser lines takes 20 us in one
-// launch for all widths, against 278 us in 12 launches of the vector-ALU kernel.
+// Weights that are not all float16 values (a trained model's) keep float32 operands and products:
+// three v_mfma_f32_16x16x4_f32, one a kernel row with its three taps and a zero, read from the
+// window as it is. So neither the weights' range nor the input's is narrowed, and a product is
+// rounded as on the vector ALU.
+//
+// The first layer of 36 recogniser lines (1316 tiles, 43 MB of pooled output) takes 25 us with
+// trained weights, in one launch for all widths, against 278 us in 12 launches of the vector-ALU
+// kernel, and 18 with float16 ones. Neither its stores (1.7 TB/s) nor its matrix instructions (7 us)
+// bound it: a workgroup's window load, its barriers and its products follow one another, five
+// workgroups a CU.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -66,8 +72,8 @@ struct C1Seg {
 constexpr int C1MAXSEG = 32;
 struct C1Params {
     int h, xcs, oh, ycs, poh, ypcs, tiles_y, nseg;
-    const half8 *wf, *wl;
-    float unscale;
+    const half8 *wf;
+    const float *wf32;
     const float *bias;
     C1Seg seg[C1MAXSEG];
 };
@@ -75,11 +81,11 @@ struct C1Params {
 constexpr int FILL = (WROWS * WW + 255) / 256;  // window values a thread loads
 
 // POOL 0: the output y only; 1: the 2 x 2 pooled output only (in yp); 2: both, the full output
-// in y and the pooled one in yp. LO: wl holds the weights' remainders.
-template <int NT, int POOL, int ACT, bool LO>
+// in y and the pooled one in yp. F32: float32 weights (wf32).
+template <int NT, int POOL, int ACT, bool F32>
 __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
     __shared__ float s_win[WROWS * WW];
-    __shared__ uint2 s_q[2 * QPLANE];  // hi plane, then lo plane; an entry is 4 halves
+    __shared__ uint2 s_q[F32 ? 1 : 2 * QPLANE];  // hi plane, then lo plane; an entry is 4 halves
     static_assert(TY / 2 * (TX / 8) % 8 == 0, "groups come in pairs per wavefront");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, r = lane & 15;
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
     }
     __syncthreads();
     // The quadruples: (x, x + 1, x + 2, 0) of each window row, split into hi and lo.
-    for (int e = tid; e < QROWS * TX; e += 256) {
+    for (int e = tid; e < (F32 ? 0 : QROWS * TX); e += 256) {
         const int row = e / TX, x = e - row * TX;
         float t[3] = {0.f, 0.f, 0.f};
         if (row < WROWS)
@@ -131,13 +137,18 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
     }
     // Weights of the NT 16-channel tiles (the A operand, or B in the pooled-only form), bias of
     // this lane's 4 channels per tile.
-    half8 a[NT], al[NT];
+    half8 a[F32 ? 1 : NT];
+    float af[F32 ? NT : 1][3];  // lane group g: tap g of each kernel row (0 for g = 3)
     float4 b4[NT];
     float bc[NT];  // the bias of channel 16 j + r (pooled-only form)
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        a[j] = p.wf[j * 64 + lane];
-        if (LO) al[j] = p.wl[j * 64 + lane];
+        if constexpr (F32) {
+#pragma unroll
+            for (int row = 0; row < 3; row++) af[j][row] = p.wf32[(j * 3 + row) * 64 + lane];
+        } else {
+            a[j] = p.wf[j * 64 + lane];
+        }
         const int co = j * 16 + 4 * g;
         b4[j] = p.bias ? *reinterpret_cast<const float4 *>(p.bias + co) : make_float4(0.f, 0.f, 0.f, 0.f);
         bc[j] = p.bias ? p.bias[j * 16 + r] : 0.f;
@@ -148,8 +159,8 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
     const int pdy = q >> 1, pdx = 2 * sq + (q & 1);
     // This lane's plane (hi for g < 2) and first quadruple row (patch row 0, or row 2 for odd g).
     const int lbase = (g >= 2 ? QPLANE : 0) + ((g & 1) ? 2 * QSTRIDE : 0) + pdy * QSTRIDE + pdx;
-    // The weights' parts are scaled by a power of two; (v, bias) -> v / scale + bias.
-    auto out = [&](float v, float b) __attribute__((always_inline)) { return LO ? fmaf(v, p.unscale, b) : v + b; };
+    // F32: tap g of patch row 0 (lane group 3 takes zeros).
+    const int wbase = pdy * WW + pdx + min(g, 2);
     constexpr int NG = TY / 2 * (TX / 8);  // groups of 16 pixels in the tile
     const int oh = p.oh, ow = sd.ow, poh = p.poh, pow_ = sd.pow_;
     float *const y = sd.y, *const yp = sd.yp;
@@ -161,20 +172,33 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
         for (int u = 0; u < 2; u++) {
             const int G = G0 + 4 * u;
             const int gy = G / (TX / 8), gx = G - gy * (TX / 8);
-            const uint2 *src = s_q + lbase + 2 * gy * QSTRIDE + 8 * gx;
-            const uint4 q4 = make_uint4(src[0].x, src[0].y, src[QSTRIDE].x, src[QSTRIDE].y);
-            half8 bf;
-            __builtin_memcpy(&bf, &q4, 16);
             // Pooled output only: the patches are the A operand, so a lane's 4 accumulators are
             // one channel of the 4 pixels of one 2 x 2 window and the pool is a max over them.
+            if constexpr (F32) {
+                float t[3];
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                floatx4 c = {0.f, 0.f, 0.f, 0.f};
-                if (LO)
-                    c = POOL == 1 ? __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, al[j], c, 0, 0, 0)
-                                  : __builtin_amdgcn_mfma_f32_16x16x32_f16(al[j], bf, c, 0, 0, 0);
-                acc[u][j] = POOL == 1 ? __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, a[j], c, 0, 0, 0)
-                                      : __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], bf, c, 0, 0, 0);
+                for (int row = 0; row < 3; row++) {
+                    const float v = s_win[wbase + (2 * gy + row) * WW + 8 * gx];
+                    t[row] = g < 3 ? v : 0.f;
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[u][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int row = 0; row < 3; row++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        acc[u][j] = POOL == 1 ? __builtin_amdgcn_mfma_f32_16x16x4f32(t[row], af[j][row], acc[u][j], 0, 0, 0)
+                                              : __builtin_amdgcn_mfma_f32_16x16x4f32(af[j][row], t[row], acc[u][j], 0, 0, 0);
+            } else {
+                const uint2 *src = s_q + lbase + 2 * gy * QSTRIDE + 8 * gx;
+                const uint4 q4 = make_uint4(src[0].x, src[0].y, src[QSTRIDE].x, src[QSTRIDE].y);
+                half8 bf;
+                __builtin_memcpy(&bf, &q4, 16);
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[u][j] = POOL == 1
+                                    ? __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, a[j], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0)
+                                    : __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], bf, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             }
         }
 #pragma unroll
@@ -191,10 +215,10 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
                     for (int j = 0; j < NT; j++) {
                         const floatx4 v = acc[u][j];
                         if (ACT == ACT_SIGMOID)
-                            dst[16 * j] = fmaxf(fmaxf(act1<ACT>(out(v[0], bc[j])), act1<ACT>(out(v[1], bc[j]))),
-                                                fmaxf(act1<ACT>(out(v[2], bc[j])), act1<ACT>(out(v[3], bc[j]))));
+                            dst[16 * j] = fmaxf(fmaxf(act1<ACT>(v[0] + bc[j]), act1<ACT>(v[1] + bc[j])),
+                                                fmaxf(act1<ACT>(v[2] + bc[j]), act1<ACT>(v[3] + bc[j])));
                         else
-                            dst[16 * j] = act1<ACT>(out(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), bc[j]));
+                            dst[16 * j] = act1<ACT>(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])) + bc[j]);
                     }
                 }
                 continue;
@@ -203,8 +227,8 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
             const int oy = y0 + 2 * gy + pdy, ox = x0 + 8 * gx + pdx;
 #pragma unroll
             for (int j = 0; j < NT; j++) {
-                float o[4] = {act1<ACT>(out(acc[u][j][0], b4[j].x)), act1<ACT>(out(acc[u][j][1], b4[j].y)),
-                              act1<ACT>(out(acc[u][j][2], b4[j].z)), act1<ACT>(out(acc[u][j][3], b4[j].w))};
+                float o[4] = {act1<ACT>(acc[u][j][0] + b4[j].x), act1<ACT>(acc[u][j][1] + b4[j].y),
+                              act1<ACT>(acc[u][j][2] + b4[j].z), act1<ACT>(acc[u][j][3] + b4[j].w)};
                 if (POOL != 1 && oy < oh && ox < ow)
                     *reinterpret_cast<float4 *>(y + ((size_t(img) * oh + oy) * ow + ox) * p.ycs + j * 16 + 4 * g) =
                         make_float4(o[0], o[1], o[2], o[3]);
@@ -226,32 +250,7 @@ __global__ __launch_bounds__(256) void conv1_kernel(const C1Params p) {
 
 }  // namespace
 
-int pack_conv1_frags(const float *w, int cout, uint16_t *frag, uint16_t *frag_lo, float *unscale) {
-    float top = 0.f;
-    bool exact = true;
-    for (int i = 0; i < cout * 9; i++) {
-        if (!std::isfinite(w[i])) return 0;
-        top = std::max(top, std::fabs(w[i]));
-        exact = exact && float(_Float16(w[i])) == w[i];
-    }
-    // Scaled by a power of two that puts the largest weight in [2^12, 2^13): the remainders are
-    // then normal float16 values also where a channel's weights are small.
-    const int e = exact ? 0 : 12 - std::ilogb(top);
-    *unscale = std::ldexp(1.f, -e);
-    auto part = [&](float v, float &lo) {
-        v = std::ldexp(v, e);
-        const float hi = float(_Float16(v));
-        lo = v - hi;
-        return hi;
-    };
-    for (int co = 0; co < cout && !exact; co++) {
-        float ctop = 0.f, lo;
-        for (int k = 0; k < 9; k++) ctop = std::max(ctop, std::fabs(std::ldexp(w[co * 9 + k], e)));
-        for (int k = 0; k < 9; k++) {
-            part(w[co * 9 + k], lo);
-            if (std::fabs(lo - float(_Float16(lo))) > ctop * 0x1p-23f) return 0;
-        }
-    }
+void pack_conv1_frags(const float *w, int cout, uint16_t *frag) {
     // frag [cout / 16][64 lanes][8]: lane (g, r) holds k = 8 g .. 8 g + 7 of channel 16 t + r.
     // Each 16-k half (hi side, lo side) is rows 0, 1, 2 of the 3 x 3 kernel as (left, centre,
     // right, 0) quadruples, then a zero quadruple.
@@ -261,16 +260,23 @@ int pack_conv1_frags(const float *w, int cout, uint16_t *frag, uint16_t *frag_lo
                 const int g = lane >> 4, r = lane & 15;
                 const int row = 2 * (g & 1) + (e >> 2), col = e & 3;
                 const float v = row < 3 && col < 3 ? w[size_t(t * 16 + r) * 9 + row * 3 + col] : 0.f;
-                float rest;
-                const _Float16 hv = (_Float16)part(v, rest), lv = (_Float16)rest;
+                const _Float16 hv = (_Float16)v;
                 std::memcpy(&frag[(size_t(t) * 64 + lane) * 8 + e], &hv, 2);
-                std::memcpy(&frag_lo[(size_t(t) * 64 + lane) * 8 + e], &lv, 2);
             }
-    return exact ? 1 : 2;
 }
 
-bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, const uint16_t *frag,
-                      const uint16_t *frag_lo, float unscale, const float *b, int act, int ph, int pw, hipStream_t s) {
+void pack_conv1_f32(const float *w, int cout, float *frag) {
+    // frag [cout / 16][3 rows][64 lanes]: lane (g, r) holds tap g of the row of channel 16 t + r.
+    for (int t = 0; t < cout / 16; t++)
+        for (int row = 0; row < 3; row++)
+            for (int lane = 0; lane < 64; lane++) {
+                const int g = lane >> 4, r = lane & 15;
+                *frag++ = g < 3 ? w[size_t(t * 16 + r) * 9 + row * 3 + g] : 0.f;
+            }
+}
+
+bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, const Conv1Frags &frag, const float *b,
+                      int act, int ph, int pw, hipStream_t s) {
     if (!frag || count < 1) return false;
     if (act != ACT_NONE && act != ACT_RELU && act != ACT_SIGMOID) return false;
     if (b && (reinterpret_cast<uintptr_t>(b) & 15)) return false;
@@ -298,7 +304,7 @@ bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, c
         bytes += 4.0 * double(xk.pixels() + yk.count() + (pool == 2 ? ypool[k].count() : 0));
     }
     const int tiles_y = (x[0].h + TY - 1) / TY;
-    ProbeScope probe("conv_direct", s, flops, bytes);
+    ProbeScope probe("conv_direct", s, flops, bytes, frag.f32 ? "conv1_f32" : "conv1_f16");
     const int nt = cout / 16;
     for (int k0 = 0; k0 < count; k0 += C1MAXSEG) {
         const int cnt = std::min(C1MAXSEG, count - k0);
@@ -307,9 +313,8 @@ bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, c
         p.xcs = x[0].cs;
         p.tiles_y = tiles_y;
         p.nseg = cnt;
-        p.wf = reinterpret_cast<const half8 *>(frag);
-        p.wl = reinterpret_cast<const half8 *>(frag_lo);
-        p.unscale = unscale;
+        p.wf = reinterpret_cast<const half8 *>(frag.f16);
+        p.wf32 = frag.f32;
         p.bias = b;
         // POOL 1 writes the pooled output through (yp, poh, pow_, ypcs) = y.
         const Act &y0 = y[k0];
@@ -338,7 +343,7 @@ bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, c
         if (blocks == 0) continue;
         const dim3 grid{unsigned(blocks)};
 #define C1_LAUNCH(NT, P, A)                                                                        \
-    if (frag_lo) hipLaunchKernelGGL((conv1_kernel<NT, P, A, true>), grid, dim3(256), 0, s, p);        \
+    if (frag.f32) hipLaunchKernelGGL((conv1_kernel<NT, P, A, true>), grid, dim3(256), 0, s, p);        \
     else hipLaunchKernelGGL((conv1_kernel<NT, P, A, false>), grid, dim3(256), 0, s, p)
 #define C1_ACT(NT, P)                                                      \
     if (act == ACT_RELU) { C1_LAUNCH(NT, P, ACT_RELU); }                    \
@@ -364,9 +369,9 @@ bool conv1_mfma_multi(const Act *x, const Act *y, const Act *ypool, int count, c
     return true;
 }
 
-bool conv1_mfma(const Act &x, const Act &y, const uint16_t *frag, const uint16_t *frag_lo, float unscale, const float *b, int act,
-                int ph, int pw, hipStream_t s, const Act *ypool) {
-    return conv1_mfma_multi(&x, &y, ypool, 1, frag, frag_lo, unscale, b, act, ph, pw, s);
+bool conv1_mfma(const Act &x, const Act &y, const Conv1Frags &frag, const float *b, int act, int ph, int pw,
+                hipStream_t s, const Act *ypool) {
+    return conv1_mfma_multi(&x, &y, ypool, 1, frag, b, act, ph, pw, s);
 }
 
 }  // namespace ocr
