@@ -399,6 +399,16 @@ def test_fused_attention_shapes(ctx, tmp_path, n, t, dim, heads):
     assert calls == {"nd_attention": 1, "nd_attention_mfma": int(4 <= dim // heads <= 16)}
 
 
+@pytest.mark.parametrize("d,form", [(1, "nd_attention_16"), (2, "nd_attention_16"), (3, "nd_attention_16"),
+                                    (4, "nd_attention_mfma"), (16, "nd_attention_mfma"), (17, "nd_attention_32"),
+                                    (32, "nd_attention_32"), (33, "nd_attention_64")])
+def test_attention_head_sizes(ctx, tmp_path, d, form):
+    # Each kernel at the ends of its head sizes: the smallest vectors that hold a head.
+    p = build(tmp_path, "hs", lambda g, x: _attention(g, x, 3 * d, 3), (2, 45, 3 * d))
+    x = RNG.standard_normal((2, 45, 3 * d)).astype(np.float32)
+    assert ran([form], lambda: check(ctx, p, x)) == {form: 1}
+
+
 def _pool2(g, x):
     return g.add("MaxPool", [x], kernel_shape=[2, 2], strides=[2, 2])
 
