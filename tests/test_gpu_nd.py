@@ -375,8 +375,11 @@ def test_conv_transpose_nchw_shapes(ctx, tmp_path, cin, cout, k, s, act):
 
 
 def _attention(g, x, dim, heads):
+    return _attention_of(g, g.add("MatMul", [x, w(g, (dim, 3 * dim), dim)]), dim, heads)
+
+
+def _attention_of(g, qkv, dim, heads):
     hd = dim // heads
-    qkv = g.add("MatMul", [x, w(g, (dim, 3 * dim), dim)])
     t5 = g.add("Transpose", [g.add("Reshape", [qkv, ints(g, [0, 0, 3, heads, hd])])], perm=[2, 0, 3, 1, 4])
     parts = [g.add("Squeeze", [g.add("Slice", [t5, ints(g, [i]), ints(g, [i + 1]), ints(g, [0])]), ints(g, [0])])
              for i in range(3)]
@@ -407,6 +410,39 @@ def test_attention_head_sizes(ctx, tmp_path, d, form):
     p = build(tmp_path, "hs", lambda g, x: _attention(g, x, 3 * d, 3), (2, 45, 3 * d))
     x = RNG.standard_normal((2, 45, 3 * d)).astype(np.float32)
     assert ran([form], lambda: check(ctx, p, x)) == {form: 1}
+
+
+@pytest.mark.parametrize("proj", [False, True])
+@pytest.mark.parametrize("t,d,heads", [(77, 15, 3), (33, 4, 8), (70, 6, 2), (40, 3, 4), (70, 16, 1)])
+def test_attention_infinities(ctx, tmp_path, t, d, heads, proj):
+    # Keys that a query scores at -inf weigh nothing, wherever they lie: all of the first 37 keys or
+    # but one, the score's infinity in the head's first value or in one of its last (which the
+    # kernels' loads may hold twice). An infinite value of the last key is an infinite output, not
+    # NaN (without the projection, whose float16 parts hold no infinities).
+    dim = heads * d
+    x = RNG.standard_normal((2, t, 3, heads, d)).astype(np.float32)
+    where = (0, d - 1, max(0, d - 4))
+    for v in where:
+        x[:, :, 0, :, v] = np.abs(x[:, :, 0, :, v]) + np.float32(0.1)
+    x[0, :min(37, t - 1), 1, :, where[0]] = -np.inf
+    x[1, 5, 1, :, where[1]] = x[1, 7, 1, :, where[2]] = -np.inf
+    if not proj:
+        x[1, t - 1, 2, :, d // 2] = np.inf
+    x = x.reshape(2, t, 3 * dim)
+
+    def fn(g, xi):
+        y = _attention_of(g, xi, dim, heads)
+        return _linear(g, g.add("Relu", [_linear(g, y, dim, 20, True)]), 20, 8, True) if proj else y
+    p = build(tmp_path, "inf", fn, x.shape)
+    import ocrhip
+    form = "nd_attention_16" if d < 4 else "nd_attention_proj" if proj else "nd_attention_mfma"
+    got = []
+    assert ran([form], lambda: got.append(ocrhip.NdGraph(ctx, p).run(x))) == {form: 1}
+    want, _ = og.run(onnx_read.load(p), x)
+    assert not np.isnan(want).any() and np.isinf(want).any() == (not proj)
+    assert np.array_equal(np.isinf(got[0]), np.isinf(want)), "infinities"
+    fin = np.isfinite(want)
+    assert (np.abs(got[0][fin] - want[fin]) <= 1e-4 * (1 + np.abs(want[fin]))).all()
 
 
 def _pool2(g, x):

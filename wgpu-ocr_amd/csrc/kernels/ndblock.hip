@@ -223,10 +223,13 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
     const float *base = p.x + size_t(img) * p.t * row + size_t(h) * p.d;
     // Lane group g holds values at .. at + 3 of a head: its values in order, but the quadruple that
     // would end past the head starts 4 before its end (and any after it), and the values it then
-    // repeats are zeros on the queries' side. Nothing outside the head is read.
+    // repeats are zeros on both sides (a zero on one does not cancel an infinity on the other).
+    // Nothing outside the head is read.
     const int at = min(4 * g, p.d - 4), vr = min(r, p.d - 1);
+    const int fresh = 4 * g - at;  // the first value of the quadruple that is not a repeated one
     // 32-bit offsets from the group's first key (an image holds fewer than 2^31 values, checked by
-    // the host); keys past the last read the group's first, and their probabilities are zeros.
+    // the host); keys past the last read the group's first, and their values and probabilities are
+    // made zeros.
     unsigned ko[2], vo[2][4];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
@@ -252,7 +255,7 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
     __builtin_amdgcn_sched_barrier(0);
     float q[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) q[i] = at + i >= 4 * g ? q4[i] * p.scale : 0.f;
+    for (int i = 0; i < 4; i++) q[i] = i >= fresh ? q4[i] * p.scale : 0.f;
     // Four partial sums of the output and of l, so that no sum is a long chain.
     float m = -INFINITY, l[2][2];
     floatx4 acc[2][2];
@@ -273,12 +276,20 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
             for (int u = 0; u < 2; u++) {
                 floatx4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int i = 0; i < 4; i++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(kg[a].k[u][i], q[i], c, 0, 0, 0);
+                for (int i = 0; i < 4; i++)
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(i >= fresh ? kg[a].k[u][i] : 0.f, q[i], c, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    s[u][i] = k0 + 16 * u + 4 * g + i < p.t ? c[i] : -INFINITY;
+                    s[u][i] = c[i];
                     v[u][i] = kg[a].v[u][i];
                 }
+            }
+            if (k0 + 32 > p.t) {
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (k0 + 16 * u + 4 * g + i >= p.t) s[u][i] = -INFINITY, v[u][i] = 0.f;
             }
             if (k0 + 32 * AHEAD < p.t) load(kg[a], k0 + 32 * AHEAD);
             float mt = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
@@ -286,6 +297,8 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
             mt = fmaxf(mt, __shfl_xor(mt, 16));
             mt = fmaxf(mt, __shfl_xor(mt, 32));
             const float mn = fmaxf(m, mt);
+            // While every score is -inf the exponents are taken from 0: weights of 0, not of NaN.
+            const float m0 = mn == -INFINITY ? 0.f : mn;
             if (k0 && __any(mn > m)) {
                 const float f = m == -INFINITY ? 0.f : expf(m - mn);
 #pragma unroll
@@ -302,7 +315,7 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float e = expf(s[u][i] - m);
+                    const float e = expf(s[u][i] - m0);
                     l[u][i & 1] += e;
                     acc[u][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[u][i], e, acc[u][i & 1], 0, 0, 0);
                 }
