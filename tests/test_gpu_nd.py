@@ -445,6 +445,16 @@ def test_attention_infinities(ctx, tmp_path, t, d, heads, proj):
     assert (np.abs(got[0][fin] - want[fin]) <= 1e-4 * (1 + np.abs(want[fin]))).all()
 
 
+@pytest.mark.parametrize("heads,d", [(4, 3), (2, 24), (20, 16)])
+def test_attention_and_projection_apart(ctx, tmp_path, heads, d):
+    # Sizes that the joined kernel does not take: attention, then the projection as any Linear runs.
+    dim = heads * d
+    p = build(tmp_path, "ap", lambda g, x: g.add("Relu", [_linear(g, _attention(g, x, dim, heads), dim, 40, False)]), (2, 37, dim))
+    x = RNG.standard_normal((2, 37, dim)).astype(np.float32)
+    calls = ran(["nd_attention", "nd_attention_proj", "nd_gemm_rows"], lambda: check(ctx, p, x))
+    assert calls == {"nd_attention": 1, "nd_attention_proj": 0, "nd_gemm_rows": 2}
+
+
 def _pool2(g, x):
     return g.add("MaxPool", [x], kernel_shape=[2, 2], strides=[2, 2])
 

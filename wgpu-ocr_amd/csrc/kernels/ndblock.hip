@@ -227,8 +227,8 @@ __device__ inline void attend(const AttnParams &p, int img, int h, int q0, int r
     // Nothing outside the head is read.
     const int at = min(4 * g, p.d - 4), vr = min(r, p.d - 1);
     const int fresh = 4 * g - at;  // the first value of the quadruple that is not a repeated one
-    // 32-bit offsets from the group's first key (an image holds fewer than 2^31 values, checked by
-    // the host); keys past the last read the group's first, and their values and probabilities are
+    // 32-bit offsets from the group's first key (an image holds fewer than 2^31 values,
+    // nd_attention_mfma_fits); keys past the last read the group's first, and their values and probabilities are
     // made zeros.
     unsigned ko[2], vo[2][4];
 #pragma unroll
@@ -447,9 +447,8 @@ void nd_rows_block(const NdRowsArgs &a, const NdRowsArgs *b, hipStream_t s) {
     OCR_HIP(hipGetLastError());
 }
 
-bool nd_attention_proj_fits(int heads, int d, const ConvPack &pk) {
-    return d >= 4 && d <= 16 && heads >= 1 && pk.kh == 1 && pk.kw == 1 && pk.cin == heads * d &&
-           pk.chunks <= PROJ_C;
+bool nd_attention_proj_fits(int n, int t, int heads, int d, const ConvPack &pk) {
+    return nd_attention_mfma_fits(n, t, heads, d) && pk.kh == 1 && pk.kw == 1 && pk.cin == heads * d && pk.chunks <= PROJ_C;
 }
 
 static AttnParams attn_params(const float *x, int n, int t, int heads, int d, float scale, float *y) {
@@ -462,14 +461,12 @@ static AttnParams attn_params(const float *x, int n, int t, int heads, int d, fl
     p.d = d;
     p.scale = scale;
     p.qtiles = (t + 15) / 16;
-    if (double(n) * p.qtiles > 0x7fffffff) fail("nd_attention: too many queries");
-    if (double(t) * 3.0 * heads * d > 0x7fffffff) fail("nd_attention: too many values an image");
     return p;
 }
 
 void nd_attention_proj(const float *x, int n, int t, int heads, int d, float scale, const NdRowsArgs &w, hipStream_t s) {
     if (n <= 0 || t <= 0) return;
-    if (!nd_attention_proj_fits(heads, d, w.pk) || w.k != heads * d || w.pk.cout != w.n) fail("nd_attention_proj: shapes");
+    if (!nd_attention_proj_fits(n, t, heads, d, w.pk) || w.k != heads * d || w.pk.cout != w.n) fail("nd_attention_proj: shapes");
     AttnParams p = attn_params(x, n, t, heads, d, scale, w.y);
     p.res = w.res;
     p.w = packed(w);
@@ -483,7 +480,7 @@ void nd_attention_proj(const float *x, int n, int t, int heads, int d, float sca
 }
 
 bool nd_attention_mfma(const float *x, int n, int t, int heads, int d, float scale, float *y, hipStream_t s) {
-    if (d < 4 || d > 16 || heads > 4 * 65535) return false;
+    if (!nd_attention_mfma_fits(n, t, heads, d)) return false;
     if (n <= 0 || t <= 0) return true;
     const AttnParams p = attn_params(x, n, t, heads, d, scale, y);
     const double tt = double(t);

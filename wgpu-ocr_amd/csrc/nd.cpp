@@ -392,6 +392,21 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         ra.eps = op.eps;
         return ra;
     };
+    // A Linear in a launch of its own.
+    auto linear = [&](const NdOp &op, const NdRowsArgs &ra) {
+        if (!no_ndconv() && nd_gemm_rows(ra, st)) return;
+        ConvArgs ca;
+        ca.x = Act{const_cast<float *>(ra.x), 1, 1, ra.m, op.k, op.k};
+        ca.y = Act{ra.y, 1, 1, ra.m, op.n, op.n};
+        ca.wt_hi = op.whi;
+        ca.wt_lo = op.wlo;
+        ca.bias = op.b;
+        ca.act = op.act;
+        ca.pk = op.pk;
+        ca.res = ra.res;
+        ca.res_cs = op.n;
+        conv_mfma(ca, st);
+    };
     // A tensor in memory: t itself, or its parts written out.
     auto solid = [&](const NdTensor &t) {
         if (t.parts.empty()) return t;
@@ -598,18 +613,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 nd_rows_block(ra, nullptr, st);
                 break;
             }
-            if (!no_ndconv() && nd_gemm_rows(ra, st)) break;
-            ConvArgs ca;
-            ca.x = Act{a.p, 1, 1, int(m), op.k, op.k};
-            ca.y = Act{out.t.p, 1, 1, int(m), op.n, op.n};
-            ca.wt_hi = op.whi;
-            ca.wt_lo = op.wlo;
-            ca.bias = op.b;
-            ca.act = op.act;
-            ca.pk = op.pk;
-            ca.res = ra.res;
-            ca.res_cs = op.n;
-            conv_mfma(ca, st);
+            linear(op, ra);
             break;
         }
         case NdKind::Attention: {
@@ -659,14 +663,14 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
             const size_t m = size_t(nb * tt);
             if (m > 0x7fffffff) fail("MatMul: too many rows");
             NdRowsArgs ra = rows_args(*op.then, nullptr, m, shape, out.t.p);
-            if (nd_attention_proj_fits(int(heads), int(hd), op.then->pk)) {
+            if (nd_attention_proj_fits(int(nb), int(tt), int(heads), int(hd), op.then->pk)) {
                 nd_attention_proj(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, ra, st);
                 break;
             }
             const DBuf rows(ctx, m * size_t(od3) * sizeof(float));
             nd_attention(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, rows.as<float>(), st);
             ra.x = rows.as<float>();
-            if (!nd_gemm_rows(ra, st)) fail("attention projection: shape");
+            linear(*op.then, ra);
             break;
         }
         case NdKind::LayerNorm: {

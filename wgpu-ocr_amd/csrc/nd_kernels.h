@@ -137,9 +137,14 @@ void nd_attention(const float *x, int n, int t, int heads, int d, float scale, f
 // The same on the matrix cores, for heads of 4 to 16 values (kernels/ndblock.hip). False
 // (nothing launched) otherwise.
 bool nd_attention_mfma(const float *x, int n, int t, int heads, int d, float scale, float *y, hipStream_t s);
+// Its grid and its 32-bit offsets within an image.
+inline bool nd_attention_mfma_fits(int n, int t, int heads, int d) {
+    return d >= 4 && d <= 16 && heads >= 1 && heads <= 4 * 65535 && double(n) * ((double(t) + 15) / 16) <= 0x7fffffff &&
+           double(t) * 3.0 * heads * d <= 0x7fffffff;
+}
 // And with the projection w of its rows (w.x unused, w.m = n t), whose input is never written:
 // heads of 4 to 16 values, 256 values in all.
-bool nd_attention_proj_fits(int heads, int d, const ConvPack &pk);
+bool nd_attention_proj_fits(int n, int t, int heads, int d, const ConvPack &pk);
 void nd_attention_proj(const float *x, int n, int t, int heads, int d, float scale, const NdRowsArgs &w, hipStream_t s);
 
 // Batched C[b] = A[b] (M x K) * B[b] (K x N) on the matrix cores, both operands float32 split
