@@ -455,6 +455,35 @@ def test_attention_and_projection_apart(ctx, tmp_path, heads, d):
     assert calls == {"nd_attention": 1, "nd_attention_proj": 0, "nd_gemm_rows": 2}
 
 
+@pytest.mark.parametrize("kind,m,hidden,n,joined", [
+    ("norm", 33, 0, 720, True), ("norm", 33, 0, 736, False), ("norm", 800, 0, 800, True), ("norm", 799, 0, 800, False),
+    ("norm", 13200, 0, 56, True), ("norm", 13201, 0, 56, False), ("norm", 24100, 0, 200, True),
+    ("mlp", 8000, 16, 20, True), ("mlp", 8001, 16, 20, False), ("normmlp", 20, 64, 750, False),
+    ("attention", 74, 0, 700, True), ("attention", 74, 0, 740, False)])
+def test_joined_steps_where_they_pay(ctx, tmp_path, kind, m, hidden, n, joined):
+    # Both sides of the lines up to which a step joined into one launch is the faster, with a residual
+    # and inexact weights in the second product.
+    k = 120
+    def fn(g, x):
+        if kind == "attention":
+            y = _attention_of(g, x, k, 8)
+        else:
+            y = _layer_norm(g, x, k) if "norm" in kind else x
+        if hidden:
+            y = _linear(g, y, k, hidden, True, act=True)
+        y = _linear(g, y, hidden or k, n, not hidden)
+        if n <= 200:
+            y = g.add("Add", [y, _linear(g, x, 3 * k if kind == "attention" else k, n, True)])
+        return g.add("Relu", [y])
+    shape = (2, m // 2, 3 * k) if kind == "attention" else (1, m, k)
+    p = build(tmp_path, "pays", fn, shape)
+    x = RNG.standard_normal(shape).astype(np.float32)
+    form = {"norm": "nd_rows_norm", "attention": "nd_attention_proj"}.get(kind, "nd_mlp")
+    norms = int("norm" in kind)
+    calls = ran([form, "nd_layer_norm"], lambda: check(ctx, p, x))
+    assert calls == {form: int(joined), "nd_layer_norm": 0 if joined else norms}
+
+
 def _pool2(g, x):
     return g.add("MaxPool", [x], kernel_shape=[2, 2], strides=[2, 2])
 

@@ -275,6 +275,7 @@ void NdGraph::join_ops() {
         if (j < 0 || gone[size_t(j)]) continue;
         NdOp &a = ops[size_t(j)], &b = ops[k];
         if (a.kind == NdKind::LayerNorm && a.len == b.k && nd_rows_fit(b.pk)) {
+            b.gb = a.gb;
             b.gb32 = a.gb32;
             b.len = a.len;
             b.eps = a.eps;
@@ -601,19 +602,32 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
             out.t = alloc(shape);
             if (shapes_only || m == 0) break;
             if (m > 0x7fffffff) fail("MatMul: too many rows");
+            // A joined step (a LayerNorm first, or a second product) in one launch, or in parts.
+            NdRowsArgs ra = rows_args(op, a.p, m, shape, out.t.p), rb;
             if (op.then) {
-                NdRowsArgs ra = rows_args(op, a.p, m, shape, nullptr);
+                rb = rows_args(*op.then, nullptr, m, shape, out.t.p);
                 ra.res = nullptr;
-                const NdRowsArgs rb = rows_args(*op.then, nullptr, m, shape, out.t.p);
-                nd_rows_block(ra, &rb, st);
+                ra.y = nullptr;
+            }
+            if ((op.gb32 || op.then) &&
+                nd_block_pays(double(m), op.k, op.then ? op.n : 0, op.then ? op.then->n : op.n, op.gb32 != nullptr)) {
+                nd_rows_block(ra, op.then ? &rb : nullptr, st);
                 break;
             }
-            const NdRowsArgs ra = rows_args(op, a.p, m, shape, out.t.p);
-            if (ra.gb) {
-                nd_rows_block(ra, nullptr, st);
-                break;
+            DBuf normed, hidden;
+            if (op.gb32) {
+                normed = DBuf(ctx, m * size_t(op.k) * sizeof(float));
+                nd_layer_norm(a.p, op.gb, normed.as<float>(), m, op.k, op.eps, st);
+                ra.x = normed.as<float>();
+                ra.gb = nullptr;
+            }
+            if (op.then) {
+                hidden = DBuf(ctx, m * size_t(op.n) * sizeof(float));
+                ra.y = hidden.as<float>();
+                rb.x = hidden.as<float>();
             }
             linear(op, ra);
+            if (op.then) linear(*op.then, rb);
             break;
         }
         case NdKind::Attention: {
@@ -663,7 +677,8 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
             const size_t m = size_t(nb * tt);
             if (m > 0x7fffffff) fail("MatMul: too many rows");
             NdRowsArgs ra = rows_args(*op.then, nullptr, m, shape, out.t.p);
-            if (nd_attention_proj_fits(int(nb), int(tt), int(heads), int(hd), op.then->pk)) {
+            if (nd_attention_proj_fits(int(nb), int(tt), int(heads), int(hd), op.then->pk) &&
+                nd_block_pays(double(m), 0, 0, op.then->n, false)) {
                 nd_attention_proj(qkv.p, int(nb), int(tt), int(heads), int(hd), op.scale, ra, st);
                 break;
             }

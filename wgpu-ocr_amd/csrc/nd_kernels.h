@@ -115,6 +115,26 @@ bool nd_gemm_rows(const NdRowsArgs &a, hipStream_t s);
 // and with b at most 256 hidden values.
 bool nd_rows_fit(const ConvPack &w1);
 bool nd_mlp_fits(const ConvPack &w1, const ConvPack &w2);
+// Whether a joined step of m rows is worth one launch, against one each. n: the columns it gives,
+// from k inputs with a LayerNorm first (norm) and hidden columns between (0: no second product; an
+// attention's projection has neither).
+//
+// Few rows fill the chip only by their columns, which a joined workgroup walks 384 (an MLP: 128) at a
+// time: 17 and 109 rows, 120 -> n with its LayerNorm, take 12 us for n = 720 against 13.5 apart, 14.7
+// against 13.8 for 960, 51 against 13.6 for 6000; at 1744 rows n = 1440 is 23 against 25 and 6000 58
+// against 49, at 8000 rows 6000 119 against 176. An attention's projection of 109 rows: 13.2 against
+// 19.1 for n = 120, 19.8 against 19.2 for 768; of 1744 rows 28 against 33 for 1200 and 76 against 60 for
+// 6000.
+// Many rows take 16 to a workgroup whose start is most of its time when it makes few products (work: the
+// columns of both products, and the LayerNorm's): work 152 20.0 us against 19.6 at 12 000 rows, 184 22.5
+// against 23.6 at 16 000 and 31.2 against 25.5 at 24 000, 240 25.8 against 26.9 at 16 000 and 35.8
+// against 32.7 at 24 000, 64 (k = 32) 12 against 13 at 8000 and 20 against 16 at 16 000; 360 is faster at
+// every size (100 000 rows 136 against 153).
+inline bool nd_block_pays(double m, double k, double hidden, double n, bool norm) {
+    const double work = n + hidden + (norm ? k : 0);
+    const bool joined_rows = norm || hidden;
+    return (n <= 720 || m >= n) && (!joined_rows || m <= 8000 || m <= 75 * work || work >= 320);
+}
 void nd_rows_block(const NdRowsArgs &a, const NdRowsArgs *b, hipStream_t s);
 // The CTC head without its logits: per row of x, nd_head_parts partial (max, index bits) pairs of
 // x W + b (first index on ties) at part[row * parts + j], for nd_argmax_partials. Needs 64-column
