@@ -56,8 +56,6 @@ struct NchwParams {
     int ksplit;      // wavefronts sharing one tile's K steps (1, 2 or 4 of 4; 8 or 16 of 16)
 };
 
-// WPB wavefronts a workgroup: 4, or 16 for launches of few tiles and long K (up to 16 wavefronts
-// share one tile's K steps).
 // The outputs of a wavefront's tile: pixels x0 .. (of row oy, or of the flattened plane) of image
 // img, channels of block nb.
 template <int MT, int NT, bool EXT>
@@ -130,9 +128,12 @@ __device__ inline void store_nchw(const NchwParams &p, const floatx4 (&acc)[MT][
     }
 }
 
-// EXT: an input scale, a second input tensor or an upscaled residual (the plain form needs fewer
-// registers: 52 against 60, 17 against 21 us for the recogniser's 64 -> 128 conv).
-template <int MT, int NT, bool LO, int WPB, bool EXT>
+// WPB wavefronts a workgroup: 4, or 16 for launches of few tiles and long K (up to 16 wavefronts
+// share one tile's K steps).
+// EXT 1: an input scale; 2: also a second input tensor or an upscaled residual. Each takes registers
+// (2 x 4 tiles 116, 118 and 150): scaled 128 -> 256 channels at 16 x 24 x 218 71 us, and 88 with the
+// form of all three.
+template <int MT, int NT, bool LO, int WPB, int EXT>
 __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
     extern __shared__ float s_red[];  // ksplit > 1: [wave][MT * NT * 4][64 lanes]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -162,8 +163,8 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             oy = line - img * p.oh;
         }
         const int taps = p.kh * p.kw, steps = p.chunks * taps;
-        const float *xim = p.x + size_t(img) * (EXT && p.x2 ? p.c1 : p.cin) * plane;
-        const float *xim2 = EXT && p.x2 ? p.x2 + size_t(img) * (p.cin - p.c1) * plane : nullptr;
+        const float *xim = p.x + size_t(img) * (EXT == 2 && p.x2 ? p.c1 : p.cin) * plane;
+        const float *xim2 = EXT == 2 && p.x2 ? p.x2 + size_t(img) * (p.cin - p.c1) * plane : nullptr;
         // K step s is (chunk, tap); steps whose kernel row reads only padding are skipped (the
         // same for the whole wavefront).
         auto valid_from = [&](int s) {
@@ -174,10 +175,19 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             }
             return steps;
         };
-        // Operands of one K step: the weight fragments and the float32 inputs (split at use).
+        // Operands of one K step: the weight fragments and the float32 inputs. These are scaled,
+        // zeroed outside (in: pixels inside, ch: channels from the lane's first to the last) and
+        // split at use: looked at next to its load, a value is waited for before the step's matrix
+        // work (1 x 1 convs of 64 -> 128 channels at 4 x 240 x 184 61 us against 49, of 128 -> 256 at
+        // 16 x 24 x 218 87 against 62).
         half8 a[NT], al[NT];
         float v[MT][8];
-        auto load = [&](int s, half8 (&wa)[NT], half8 (&wl)[NT], float (&xv)[MT][8]) {
+        struct Use {
+            bool in[MT];
+            int ch;
+            float sc[EXT ? 8 : 1];
+        } use;
+        auto load = [&](int s, half8 (&wa)[NT], half8 (&wl)[NT], float (&xv)[MT][8], Use &xu) {
             const int chunk = s / taps, tap = s - chunk * taps;
             const int ky = tap / p.kw, kx = tap - ky * p.kw;
             const size_t wo = (size_t(nb * p.chunks + chunk) * taps + tap) * (p.bn * 4) + size_t(r) * 4 + g;
@@ -191,42 +201,49 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             // offsets from it (an image holds fewer than 2^30 values, checked by the host). The
             // reads are unconditional, from a position inside the image (channel clamped to the
             // last, pixel to the row's first), and the values outside are zeroed after.
-            const bool second = EXT && p.x2 && chunk * 32 >= p.c1;
+            const bool second = EXT == 2 && p.x2 && chunk * 32 >= p.c1;
             const int cs = second ? p.c1 : 0;
             const float *xrow = (second ? xim2 : xim) + (p.flat ? 0 : size_t(oy + ky - p.pt) * p.w);
             const bool full = c0 + 8 <= p.cin;
+            xu.ch = p.cin - c0;
             // The input scales of the lane's channels, once for its pixels.
-            float sc[8];
-            if (EXT && p.in_scale) {
+            if constexpr (EXT) {
+                if (p.in_scale) {
 #pragma unroll
-                for (int j = 0; j < 8; j++) sc[j] = p.in_scale[size_t(img) * p.cin + min(c0 + j, p.cin - 1)];
+                    for (int j = 0; j < 8; j++) xu.sc[j] = p.in_scale[size_t(img) * p.cin + min(c0 + j, p.cin - 1)];
+                }
             }
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 const int px = x0 + 16 * m + r + (p.flat ? 0 : kx - p.pl);
                 const bool in = px >= 0 && px < lim;
                 const unsigned pxc = in ? unsigned(px) : 0u;
+                xu.in[m] = in;
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     const int ci = full ? c0 + j : min(c0 + j, p.cin - 1);
                     const unsigned boff = (unsigned(ci - cs) * planeu + pxc) * 4u;
-                    float t = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xrow) + boff);
-                    if (EXT && p.in_scale) t *= sc[j];
-                    xv[m][j] = (in && (full || c0 + j < p.cin)) ? t : 0.f;
+                    xv[m][j] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xrow) + boff);
                 }
             }
         };
         int s = valid_from(kpart);
-        if (s < steps) load(s, a, al, v);
+        if (s < steps) load(s, a, al, v, use);
         while (s < steps) {
             // The next step's loads go out before this step's matrix work.
             const int sn = valid_from(s + p.ksplit);
             half8 na[NT], nal[NT];
             float nv[MT][8];
-            if (sn < steps) load(sn, na, nal, nv);
+            Use nuse;
+            if (sn < steps) load(sn, na, nal, nv, nuse);
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 half8 hi, lo;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    if constexpr (EXT) v[m][j] *= p.in_scale ? use.sc[j] : 1.f;
+                    v[m][j] = use.in[m] && j < use.ch ? v[m][j] : 0.f;
+                }
                 split8(v[m], hi, lo);
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
@@ -237,6 +254,7 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
             }
             if (sn >= steps) break;
             s = sn;
+            use = nuse;
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 a[t] = na[t];
@@ -273,7 +291,7 @@ __global__ __launch_bounds__(64 * WPB) void conv_nchw_kernel(NchwParams p) {
         }
     }
     if (!live) return;
-    store_nchw<MT, NT, EXT>(p, acc, img, oy, x0, nb, r, g);
+    store_nchw<MT, NT, EXT == 2>(p, acc, img, oy, x0, nb, r, g);
 }
 
 // 1 x 1 convs: a wavefront makes 16 pixels of the flattened plane x 16 NT channels, with the
@@ -365,11 +383,14 @@ void launch_px_kc(const NchwParams &p, bool lo, dim3 grid, hipStream_t s) {
 
 template <int MT, int NT, int WPB>
 void launch_nchw(const NchwParams &p, bool lo, dim3 grid, size_t lds, hipStream_t s) {
-    const bool ext = p.in_scale || p.x2 || p.res_up;
-    if (lo && ext) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, true, WPB, true>), grid, dim3(64 * WPB), lds, s, p);
-    else if (lo) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, true, WPB, false>), grid, dim3(64 * WPB), lds, s, p);
-    else if (ext) hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, false, WPB, true>), grid, dim3(64 * WPB), lds, s, p);
-    else hipLaunchKernelGGL((conv_nchw_kernel<MT, NT, false, WPB, false>), grid, dim3(64 * WPB), lds, s, p);
+    const int ext = p.x2 || p.res_up ? 2 : p.in_scale ? 1 : 0;
+    auto launch = [&](auto *exact, auto *inexact) {
+        if (lo) hipLaunchKernelGGL(inexact, grid, dim3(64 * WPB), lds, s, p);
+        else hipLaunchKernelGGL(exact, grid, dim3(64 * WPB), lds, s, p);
+    };
+    if (ext == 2) launch(conv_nchw_kernel<MT, NT, false, WPB, 2>, conv_nchw_kernel<MT, NT, true, WPB, 2>);
+    else if (ext == 1) launch(conv_nchw_kernel<MT, NT, false, WPB, 1>, conv_nchw_kernel<MT, NT, true, WPB, 1>);
+    else launch(conv_nchw_kernel<MT, NT, false, WPB, 0>, conv_nchw_kernel<MT, NT, true, WPB, 0>);
 }
 
 template <int MT, int WPB = 4>
