@@ -493,16 +493,20 @@ def _up(g, x, f):
     return g.add("Resize", [x, "", sc], mode="nearest", coordinate_transformation_mode="asymmetric", nearest_mode="floor")
 
 
-@pytest.mark.parametrize("n,cin,cout,h,w,exact", [(3, 20, 16, 41, 101, True), (1, 64, 40, 64, 289, False),
-                                                  (2, 33, 64, 120, 90, True), (1, 3, 70, 96, 200, True)])
-def test_3x3_nchw_many_rows(ctx, tmp_path, n, cin, cout, h, w, exact):
+@pytest.mark.parametrize("n,cin,cout,h,w,exact,tiled", [
+    (3, 20, 16, 41, 101, True, 0), (1, 64, 40, 64, 289, False, 2), (1, 64, 40, 64, 249, False, 0), (2, 33, 64, 120, 90, True, 0), (1, 3, 70, 96, 200, True, 2),
+    (3, 20, 16, 81, 101, True, 2), (1, 64, 40, 121, 417, False, 2), (2, 130, 64, 120, 138, True, 1), (1, 100, 16, 96, 174, False, 1),
+    (2, 36, 30, 105, 155, False, 2), (4, 64, 64, 60, 46, True, 0)])
+def test_3x3_nchw_many_rows(ctx, tmp_path, n, cin, cout, h, w, exact, tiled):
     # Images of many rows: tiles of 8 x 32 pixels with a part of a tile left on both sides, channel
-    # counts that end inside a chunk or block, with a residual.
+    # counts that end inside a chunk or block, with a residual. From the sizes on at which tiles are
+    # the faster, by block, channels and row length (tiled: how many of the two convs).
     def fn(g, x):
         y = g.add("Relu", [bn(g, conv(g, x, cin, cout, exact=exact, bias=False), cout)])
         return g.add("Add", [g.add("Relu", [conv(g, y, cout, cout)]), y])
     p = build(tmp_path, "c3r", fn, (n, cin, h, w))
-    check(ctx, p, RNG.standard_normal((n, cin, h, w)).astype(np.float32))
+    x = RNG.standard_normal((n, cin, h, w)).astype(np.float32)
+    assert ran(["nd_conv_tile"], lambda: check(ctx, p, x)) == {"nd_conv_tile": tiled}
 
 
 @pytest.mark.parametrize("n,c,h,w,cout", [(4, 16, 64, 96, 16), (1, 16, 16, 24, 16), (2, 8, 88, 160, 40), (2, 12, 64, 96, 16),

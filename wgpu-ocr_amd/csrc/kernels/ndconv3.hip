@@ -23,11 +23,24 @@ namespace ocr {
 
 namespace {
 
-// Fewer tiles than this leave CUs without one, and tiles of which over half lies outside the image
-// (one-row tensors) are work for nothing: conv_nchw splits such launches' K steps instead.
-// 64 tiles (4 x 60 x 46) 14 -> 18 us and its Concat part read in place; a one-row tensor's 512 -> 32
-// conv 122 against 14.
-constexpr double TILE_BLOCKS = 64;
+// A Concat's parts are read in place from this many workgroups on: written out first, they cost a
+// launch each. Below, CUs without a tile cost more.
+constexpr double PART_BLOCKS = 64;
+// Any other input, which conv_nchw reads as it is: from this many pixels on (counted once a block of
+// output channels). conv_nchw splits smaller launches' K steps; its time grows with its rows of 16
+// pixels, which more wavefronts hide up to about 32 000 pixels, and the tile's with its K steps and
+// its stores (8-byte aligned rows leave as single floats). us, conv_nchw against tiles:
+//   32 -> 32 channels: 160-pixel rows 28 160 pixels 14.1 and 14.1, 34 560 17.8 and 14.4; 46-pixel rows
+//   27 600 15.2 and 18.0, 33 120 18.7 and 18.4. 128 -> 64: 27 600 44.7 and 52.3, 33 120 59.2 and 53.1. 256 ->
+//   64: 27 600 78 and 78, 33 120 106 and 80. 64 -> 128 (two blocks): 28 160 24.3 and 25.8, 33 120 35.6 and 34.6.
+//   64 -> 64: 160-pixel rows 28 160 25.1 and 28.2, 34 560 33.3 and 30.8; rows of 190 41 040 36.8 and 40.2,
+//   53 200 43.7 and 42.2.
+//   16 channels a block: 64 -> 16 13 800 13.8 and 16.0, 16 560 16.4 and 16.0, 22 080 17.5 and 16.2; 16 -> 16
+//   22 800 12.1 and 12.6, 27 600 13.4 and 12.8.
+double plain_pixels(int bn, int cin, int w) {
+    if (bn == 16) return cin >= 64 ? 16500 : 24000;
+    return bn == 64 && cin <= 64 && w % 4 ? 50000 : 32000;
+}
 
 constexpr int TH = 8, TW = 32, HW = TW + 2, HPX = (TH + 2) * HW, ITEMS = HPX * 4, NI = 3;
 
@@ -167,7 +180,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void conv_tile_kernel(TilePar
 
 }  // namespace
 
-bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hipStream_t s) {
+bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, bool saves, hipStream_t s) {
     const ConvPack &pk = a.pk;
     if (pk.kh != 3 || pk.kw != 3 || a.pt != 1 || a.pl != 1 || a.oh != a.h || a.ow != a.w || a.in_scale || a.res_up || a.x2) return false;
     if (pk.cin != a.cin || pk.cout != a.cout || !a.wt_hi || (!pk.exact && !a.wt_lo)) return false;
@@ -192,7 +205,11 @@ bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hi
     p.tiles_y = (a.h + TH - 1) / TH;
     const double blocks = double(a.n) * p.tiles_x * p.tiles_y;
     if (blocks > 0x7fffffff || pk.nblocks > 65535) return false;
-    if (blocks * pk.nblocks < TILE_BLOCKS || blocks * TH * TW > 2.0 * a.n * a.h * a.w) return false;
+    // Tiles of which over half lies outside the image (one-row tensors) are work for nothing: a one-row
+    // tensor's 512 -> 32 conv 122 us against 14.
+    const double px = double(a.n) * a.h * a.w;
+    if (blocks * TH * TW > 2.0 * px) return false;
+    if (saves ? blocks * pk.nblocks < PART_BLOCKS : px * pk.nblocks < plain_pixels(pk.bn, a.cin, a.w)) return false;
     if (blocks == 0) return true;
     p.y = a.y;
     p.wt = reinterpret_cast<const half8 *>(a.wt_hi);
@@ -207,7 +224,6 @@ bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hi
     p.bn = pk.bn;
     p.chunks = pk.chunks;
     p.act = a.act;
-    const double px = double(a.n) * a.h * a.w;
     double in = 0;
     for (int k = 0; k < nsrc; k++) in += double(a.n) * src[k].c * src[k].h * src[k].w;
     ProbeScope probe("nd_conv_nchw", s, 2.0 * px * a.cout * a.cin * 9,

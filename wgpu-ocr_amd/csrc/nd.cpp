@@ -525,8 +525,10 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                     std::vector<NdConvSource> src;
                     for (const NdPart &part : a.parts)
                         src.push_back({part.t.p, 0, int(part.t.shape[1]), int(part.t.shape[2]), int(part.t.shape[3]), part.up});
-                    if (nd_conv_tile(ma, src.empty() ? nullptr : src.data(), int(src.size()), st)) break;
-                    if (src.size() == 2 && !src[0].up && !src[1].up && src[0].c % 32 == 0) {
+                    // Two tensors that the general kernel reads where they lie.
+                    const bool two = src.size() == 2 && !src[0].up && !src[1].up && src[0].c % 32 == 0;
+                    if (nd_conv_tile(ma, src.empty() ? nullptr : src.data(), int(src.size()), src.size() > 1 && !two, st)) break;
+                    if (two) {
                         ma.x = src[0].p;
                         ma.x2 = src[1].p;
                         ma.c1 = src[0].c;

@@ -89,9 +89,10 @@ struct NdConvSource {
     int c0, c, h, w, up;
 };
 // 3 x 3, pad 1 over images of many rows (kernels/ndconv3.hip), the input a.x or the nsrc sources
-// in order (c0 is set here), each from a multiple of 8 channels. False (nothing launched) for
-// shapes it does not take: few tiles (of one plain source), x2, res_up, in_scale.
-bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, hipStream_t s);
+// in order (c0 is set here), each from a multiple of 8 channels. saves: the sources would be written
+// out as several parts if it did not take them. False (nothing launched) for what it does not take:
+// few tiles or pixels, tiles mostly outside the image, x2, res_up, in_scale.
+bool nd_conv_tile(const NdMfmaConvArgs &a, const NdConvSource *src, int nsrc, bool saves, hipStream_t s);
 bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s);
 
 // y [m][n] = act(x [m][k] W + b) (+ res [m][n]) with W packed as n rows of k (pack_conv_weights,
