@@ -529,15 +529,25 @@ int gcu_count() {
     return n;
 }
 
-// Calls of at most this many 16 x 16 x 32 blocks take gemm_thin. At the line both forms take
-// about the same: 1536 columns, K = 256: 400 rows (19 200) 12.3 us against gemm_tile's 14.4, 800
-// rows 16.7 against 14.7; K = 512: 200 rows (20 000) 14.2 against 17.7, 400 rows 20.8 against 17.3;
-// 97 columns, K = 512: 1600 rows (11 200) 8 against 14, 4500 rows (31 600) 17 against 13.
-constexpr double THIN_BLOCKS = 20000;
+// Calls of at most this many wavefronts (16 x 16 tiles) take gemm_thin: its operands cost each
+// wavefront the same however many there are, until there are more than about two a SIMD; with few K
+// chunks there is less of a latency to hide and gemm_tile is as fast from fewer on. us, thin against
+// tile: 97 columns, K = 128, 1500 wavefronts 9.8 and 11.2, 2250 12.4 and 11.3, 5000 18.0 and 11.8; K = 256,
+// 2000 10.4 and 13.8, 2500 13.0 and 13.9, 3250 15.6 and 14.1; K = 512, 2000 11 and 18.8, 2500 19.9 and 19.4. 1536
+// columns: K = 128, 1500 9.2 and 10.0, 2300 11.5 and 10.1; K = 256, 2000 9.7 and 12.5, 2500 12.4 and 12.5;
+// K = 512, 2000 14.1 and 17.4, 2500 18.9 and 17.3.
+double thin_waves(int chunks) { return chunks < 8 ? 1536 : 2048; }
 // Calls of at least this many 256 x 256 tiles take gemm_dma (two and a half a CU): 30 000 rows x
 // 1536 (708 tiles) 81 and 123 us for K = 256 and 512 against gemm_tile's 96 and 130, 71 700 rows
-// 176 and 275 against 223 and 310; 16 000 rows (378) 59 and 81 for gemm_tile.
+// 176 and 275 against 223 and 310.
 constexpr double BIG_TILES = 640;
+// Smaller ones too when its rounds of tiles, one a CU, are this full. us, gemm_dma against gemm_tile, by
+// fullness: 256 columns, K = 128, 0.59 42.9 and 39.1, 0.76 44.6 and 53.2, 0.78 26.3 and 32.9, 0.88 26.2 and 34.9;
+// K = 256, 0.76 70.4 and 72.9, 0.88 34.5 and 43.5. 512 columns, K = 256, 0.59 56.0 and 48.0, 0.76 63.2 and 61.2, 0.86
+// 64.2 and 65.5, 0.88 33.4 and 40.8; K = 512, 0.76 96.8 and 94.1, 0.86 96.8 and 92.1, 0.88 48.3 and 55.1. 1536 columns,
+// K = 512, 0.60 83 and 61, 0.79 87.3 and 82.3, 0.81 47.6 and 46.4, 0.88 88.7 and 89.5, 0.90 48.5 and 50.9, 1 49.1 and
+// 51.9.
+double full_rounds(int n) { return n <= 256 ? 0.75 : 0.85; }
 
 const float *gzero() { return static_cast<const float *>(zero_block64()); }
 
@@ -574,15 +584,18 @@ bool gemm_dma(const ConvArgs &a, hipStream_t s) {
     if (p.M == 0) return true;
     const double thin = std::ceil(p.M / 16.0) * p.ntiles;
     const double big = std::ceil(p.M / double(GBM)) * std::ceil(N / 256.0);
-    const bool few = thin * p.chunks <= THIN_BLOCKS, many = N > 128 && big >= BIG_TILES;
+    // gemm_dma's launch: runs of row tiles, one a CU for each column block.
+    p.mtiles = (p.M + GBM - 1) / GBM;
+    p.nblocks = (N + 255) / 256;
+    p.runs = std::max(1, std::min(p.mtiles, gcu_count() / p.nblocks));
+    const double slots = std::max(1, gcu_count() / p.nblocks), rounds = std::ceil(p.mtiles / slots);
+    const bool few = thin <= thin_waves(p.chunks);
+    const bool many = N > 128 && (big >= BIG_TILES || p.mtiles >= full_rounds(N) * slots * rounds);
     const bool narrow = p.ntiles <= 8;
     double blocks;
     if (few) {
         blocks = std::ceil(thin / 4);
     } else if (many) {
-        p.mtiles = (p.M + GBM - 1) / GBM;
-        p.nblocks = (N + 255) / 256;
-        p.runs = std::max(1, std::min(p.mtiles, gcu_count() / p.nblocks));
         blocks = double(p.runs) * p.nblocks;
     } else {
         p.nblocks = (p.ntiles + (narrow ? 7 : 15)) / (narrow ? 8 : 16);
