@@ -509,9 +509,9 @@ def test_3x3_nchw_many_rows(ctx, tmp_path, n, cin, cout, h, w, exact, tiled):
     assert ran(["nd_conv_tile"], lambda: check(ctx, p, x)) == {"nd_conv_tile": tiled}
 
 
-@pytest.mark.parametrize("n,c,h,w,cout", [(4, 16, 64, 96, 16), (1, 16, 16, 24, 16), (2, 8, 88, 160, 40), (2, 12, 64, 96, 16),
-                                          (4, 32, 32, 104, 32)])
-def test_conv_of_upscaled_parts(ctx, tmp_path, n, c, h, w, cout):
+@pytest.mark.parametrize("n,c,h,w,cout,inplace", [(4, 16, 64, 96, 16, True), (1, 16, 16, 24, 16, False), (2, 8, 88, 160, 40, True),
+                                                  (2, 12, 64, 96, 16, False), (4, 32, 32, 104, 32, True)])
+def test_conv_of_upscaled_parts(ctx, tmp_path, n, c, h, w, cout, inplace):
     # What a Concat of Resizes would write is read from the parts: by the 3 x 3 conv on tiles, or
     # written out after all (few tiles, a part of 12 channels). A Resize is also a 1 x 1 and a
     # 3 x 3 conv's residual, and one is read by an op that is no conv.
@@ -525,7 +525,32 @@ def test_conv_of_upscaled_parts(ctx, tmp_path, n, c, h, w, cout):
         b = g.add("Add", [conv(g, a, c, c), _up(g, p1, 2.0)])
         return g.add("Add", [b, g.add("Relu", [_up(g, p2, 4.0)])])
     p = build(tmp_path, "parts", fn, (n, c, h, w))
-    check(ctx, p, RNG.standard_normal((n, c, h, w)).astype(np.float32))
+    x = RNG.standard_normal((n, c, h, w)).astype(np.float32)
+    calls = ran(["nd_copy", "nd_resize"], lambda: check(ctx, p, x))
+    assert calls == {"nd_copy": 0 if inplace else 3, "nd_resize": 1 if inplace else 3}
+
+
+def test_parts_written_out_once(ctx, tmp_path):
+    # Readers that cannot take parts share one written-out value: a Resize of two 1 x 1 convs, which
+    # a Concat of two 3 x 3 convs (few pixels) holds as well, and a Concat whose first part does not
+    # end with a chunk, of two 1 x 1 convs.
+    def fn(g, x):
+        a = g.add("Relu", [conv(g, x, 8, 24, k=1)])
+        u = _up(g, _pool2(g, a), 2.0)
+        v = _up(g, _pool2(g, _pool2(g, a)), 4.0)
+        y = [conv(g, u, 24, 16, k=1), conv(g, u, 24, 16, k=1)]
+        cat = g.add("Concat", [u, v], axis=1)
+        y += [conv(g, cat, 48, 16), conv(g, cat, 48, 16)]
+        two = g.add("Concat", [a, g.add("Relu", [conv(g, x, 8, 9, k=1)])], axis=1)
+        y += [conv(g, two, 33, 16, k=1), conv(g, two, 33, 16, k=1)]
+        out = y[0]
+        for v in y[1:]:
+            out = g.add("Add", [g.add("Relu", [out]), g.add("Sigmoid", [v])])
+        return out
+    p = build(tmp_path, "once", fn, (1, 8, 12, 20))
+    x = RNG.standard_normal((1, 8, 12, 20)).astype(np.float32)
+    calls = ran(["nd_resize", "nd_copy", "nd_conv_tile"], lambda: check(ctx, p, x))
+    assert calls == {"nd_resize": 2, "nd_copy": 4, "nd_conv_tile": 0}
 
 
 @pytest.mark.parametrize("n,c1,c2,h,w,k", [(2, 256, 256, 1, 109, 3), (1, 32, 40, 5, 61, 1), (3, 64, 16, 9, 30, 3), (2, 24, 40, 6, 50, 1)])

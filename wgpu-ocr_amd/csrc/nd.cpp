@@ -408,40 +408,35 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         ca.res_cs = op.n;
         conv_mfma(ca, st);
     };
-    // A tensor in memory: t itself, or its parts written out.
-    auto solid = [&](const NdTensor &t) {
-        if (t.parts.empty()) return t;
-        NdTensor y;
+    // A tensor in memory: t itself, or its parts written out, once for all readers.
+    std::function<NdTensor(const NdTensor &)> solid = [&](const NdTensor &t) {
+        if (!t.parts) return t;
+        NdTensor &y = t.parts->solid;
+        if (y.p) return y;
         y.shape = t.shape;
         y.buf = std::make_shared<DBuf>(ctx, std::max<size_t>(y.count(), 1) * sizeof(float));
         y.p = y.buf->as<float>();
         const auto os = strides_of(y.shape);
         size_t c0 = 0;
-        for (const NdPart &part : t.parts) {
-            const auto &ps = part.t.shape;
-            const float *src = part.t.p;
-            std::vector<int64_t> us = {ps[0], ps[1], ps[2] << part.up, ps[3] << part.up};
-            DBuf up;
-            if (part.up) {
-                const bool whole = t.parts.size() == 1;
-                if (!whole) up = DBuf(ctx, size_t(us[0] * us[1] * us[2] * us[3]) * sizeof(float));
-                float *dst_up = whole ? y.p : up.as<float>();
-                nd_resize_nearest(src, dst_up, size_t(us[0] * us[1]), int(ps[2]), int(ps[3]), int(us[2]), int(us[3]),
-                                  float(1 << part.up), float(1 << part.up), st);
-                if (whole) break;
-                src = dst_up;
+        for (const NdPart &part : t.parts->list) {
+            if (part.up && t.parts->list.size() == 1) {
+                const auto &ps = part.t.shape;
+                nd_resize_nearest(part.t.p, y.p, size_t(ps[0] * ps[1]), int(ps[2]), int(ps[3]), int(y.shape[2]),
+                                  int(y.shape[3]), float(1 << part.up), float(1 << part.up), st);
+                break;
             }
-            const auto is = strides_of(us);
+            const NdTensor src = part.up ? solid(part.of) : part.t;
+            const auto is = strides_of(src.shape);
             NdIndex ix;
-            ix.total = size_t(us[0] * us[1] * us[2] * us[3]);
+            ix.total = src.count();
             ix.rank = 4;
             for (size_t d = 0; d < 4; d++) {
-                ix.dims[d] = size_t(us[d]);
+                ix.dims[d] = size_t(src.shape[d]);
                 ix.s0[d] = is[d];
                 ix.s1[d] = os[d];
             }
-            nd_copy(src, y.p, ix, 0, c0 * os[1], st);
-            c0 += size_t(us[1]);
+            nd_copy(src.p, y.p, ix, 0, c0 * os[1], st);
+            c0 += size_t(src.shape[1]);
         }
         return y;
     };
@@ -452,7 +447,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         auto flt = [&](size_t k) {
             NdValue v = arg(k);
             if (v.is_int) fail(n.op + ": input " + std::to_string(k) + " is not float");
-            if (v.t.parts.empty()) return std::move(v.t);
+            if (!v.t.parts) return std::move(v.t);
             return solid(v.t);
         };
         auto ints = [&](size_t k) {
@@ -516,18 +511,23 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 ma.pt = pt;
                 ma.pl = pl;
                 ma.act = op.act;
-                if (!res.parts.empty()) {
-                    if (res.parts.size() != 1) res = solid(res);
-                    else ma.res_up = res.parts[0].up;
-                    ma.res = res.parts.empty() ? res.p : res.parts[0].t.p;
+                if (res.parts && res.parts->list.size() == 1) {
+                    ma.res_up = res.parts->list[0].up;
+                    ma.res = res.parts->list[0].t.p;
+                } else {
+                    res = solid(res);
+                    ma.res = res.p;
                 }
                 if (!no_ndconv()) {
                     std::vector<NdConvSource> src;
-                    for (const NdPart &part : a.parts)
-                        src.push_back({part.t.p, 0, int(part.t.shape[1]), int(part.t.shape[2]), int(part.t.shape[3]), part.up});
+                    if (a.parts)
+                        for (const NdPart &part : a.parts->list)
+                            src.push_back({part.t.p, 0, int(part.t.shape[1]), int(part.t.shape[2]), int(part.t.shape[3]), part.up});
                     // Two tensors that the general kernel reads where they lie.
                     const bool two = src.size() == 2 && !src[0].up && !src[1].up && src[0].c % 32 == 0;
-                    if (nd_conv_tile(ma, src.empty() ? nullptr : src.data(), int(src.size()), src.size() > 1 && !two, st)) break;
+                    if (nd_conv_tile(ma, src.empty() ? nullptr : src.data(), int(src.size()),
+                                     src.size() > 1 && !two && !a.parts->solid.p, st))
+                        break;
                     if (two) {
                         ma.x = src[0].p;
                         ma.x2 = src[1].p;
@@ -905,16 +905,17 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                     shape[size_t(ax)] += p.t.shape[size_t(ax)];
                 }
                 if (op.parts && !shapes_only && r == 4 && ax == 1 &&
-                    std::all_of(parts.begin(), parts.end(), [](const NdValue &v) { return v.t.parts.size() <= 1; })) {
+                    std::all_of(parts.begin(), parts.end(), [](const NdValue &v) { return !v.t.parts || v.t.parts->list.size() == 1; })) {
                     out.t.shape = shape;
+                    out.t.parts = std::make_shared<NdParts>();
                     for (const auto &p : parts) {
-                        if (p.t.parts.empty()) out.t.parts.push_back({p.t, 0});
-                        else out.t.parts.push_back(p.t.parts[0]);
+                        if (!p.t.parts) out.t.parts->list.push_back({p.t, 0, {}});
+                        else if (!p.t.parts->list[0].up) out.t.parts->list.push_back(p.t.parts->list[0]);
+                        else out.t.parts->list.push_back({p.t.parts->list[0].t, p.t.parts->list[0].up, p.t});
                     }
                     break;
                 }
-                for (auto &p : parts)
-                    if (!p.t.parts.empty()) p.t = solid(p.t);
+                for (auto &p : parts) p.t = solid(p.t);
                 out.t = alloc(shape);
                 if (shapes_only) break;
                 const auto os = strides_of(shape);
@@ -970,7 +971,8 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
                 const int up = sc[2] == 2.f ? 1 : sc[2] == 4.f ? 2 : sc[2] == 8.f ? 3 : 0;
                 if (op.parts && !shapes_only && up && sc[2] == sc[3] && a.count()) {
                     out.t.shape = {a.shape[0], a.shape[1], oh, ow};
-                    out.t.parts.push_back({a, up});
+                    out.t.parts = std::make_shared<NdParts>();
+                    out.t.parts->list.push_back({a, up, {}});
                     break;
                 }
                 out.t = alloc({a.shape[0], a.shape[1], oh, ow});

@@ -17,17 +17,23 @@ namespace ocr {
 
 // A float tensor in device memory, or one that no memory holds yet: the parts that a Concat over
 // axis 1 would write, each a nearest-neighbour upscaling of a tensor by 2^up (p is then null).
-struct NdPart;
+struct NdParts;
 struct NdTensor {
     std::shared_ptr<DBuf> buf;  // owner (null for weights and caller memory)
     float *p = nullptr;
     std::vector<int64_t> shape;
-    std::vector<NdPart> parts;
+    std::shared_ptr<NdParts> parts;
     size_t count() const;
 };
 struct NdPart {
     NdTensor t;
     int up = 0;
+    NdTensor of;  // up > 0: the upscaled value itself
+};
+// The parts of a value that a run makes, one for all that hold the value.
+struct NdParts {
+    std::vector<NdPart> list;
+    NdTensor solid;  // the value in memory, from the first reader on that needs it there
 };
 
 struct NdValue {
