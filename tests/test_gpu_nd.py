@@ -339,13 +339,16 @@ def test_depthwise_row_ends(ctx, tmp_path, c, h, wd, stride, k):
     assert ran(["nd_conv_dw", "nd_conv_dw_wide"], lambda: check(ctx, p, x)) == {"nd_conv_dw": 1, "nd_conv_dw_wide": int(wd >= 4)}
 
 
-@pytest.mark.parametrize("cin,cout,h,wd,s", [(6, 5, 7, 9, 2), (4, 3, 16, 17, 2), (3, 6, 5, 5, 1), (4, 2, 3, 3, 3)])
-def test_conv_transpose_channel_blocks(ctx, tmp_path, cin, cout, h, wd, s):
+@pytest.mark.parametrize("cin,cout,h,wd,s,form", [
+    (6, 5, 7, 9, 2, "nd_convt_1"), (4, 3, 16, 17, 2, "nd_convt_1"), (3, 6, 5, 5, 1, "nd_convt_1"), (4, 2, 3, 3, 3, "nd_convt_1"),
+    (6, 5, 130, 252, 2, "nd_convt_4"), (6, 5, 127, 256, 2, "nd_convt_1"), (3, 6, 257, 131, 1, "nd_convt_4"), (4, 2, 300, 300, 3, "nd_convt_1")])
+def test_conv_transpose_channel_blocks(ctx, tmp_path, cin, cout, h, wd, s, form):
     # Output channels that do not fill a thread's four, and planes that end inside a workgroup.
     p = build(tmp_path, "ctb", lambda g, x: g.add("ConvTranspose", [x, w(g, (cin, cout, s, s), cin, exact=False),
                                                                      g.init("tb", np.full(cout, 0.1, np.float32))],
                                                   kernel_shape=[s, s], strides=[s, s]), (2, cin, h, wd))
-    check(ctx, p, RNG.standard_normal((2, cin, h, wd)).astype(np.float32))
+    x = RNG.standard_normal((2, cin, h, wd)).astype(np.float32)
+    assert ran([form], lambda: check(ctx, p, x)) == {form: 1}
 
 
 @pytest.mark.parametrize("h,wd", [(1, 1), (3, 31), (2, 32), (5, 33), (4, 64), (3, 255), (2, 257), (7, 736)])

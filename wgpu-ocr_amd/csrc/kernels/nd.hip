@@ -315,9 +315,8 @@ __global__ void convt_nchw_kernel(const float *x, int n, int cin, int h, int w, 
 // ConvTranspose with kernel = stride S (no overlap: input pixel (iy, ix) alone makes the S x S
 // outputs (S iy + a, S ix + b)): a thread an input pixel and CB output channels (a block's: their
 // weights are scalar loads), the channel sum in the order convt_nchw_kernel takes it, the S x S
-// results stored as S rows of S neighbours. Bound by its stores; with an output channel a thread
-// and its place from three 64-bit divisions it was bound by those: 4 x 16 -> 16
-// channels at 240 x 184 45 -> 22 us.
+// results stored as S rows of S neighbours. With an output channel a thread and its place from three
+// 64-bit divisions it was bound by those: 4 x 16 -> 16 channels, 2 x 2, at 240 x 184 45 -> 22 us.
 template <int S, int CB>
 __global__ __launch_bounds__(256) void convt_ks_nchw_kernel(const float *x, int cin, int h, int w, const float *wt,
                                                             const float *b, float *y, int cout, int act) {
@@ -498,16 +497,24 @@ void nd_conv_transpose(const float *x, int n, int cin, int h, int w, const float
     const int oh = (h - 1) * stride + kh, ow = (w - 1) * stride + kw;
     const size_t total = size_t(n) * cout * oh * ow;
     if (!total) return;
+    const bool no_overlap = kh == stride && kw == stride && stride >= 1 && stride <= 4 && n <= 65535 && cout <= 65535 &&
+                            double(h) * w < 2147483392.0;
+    // Four channels a thread, or one while four would make under two workgroups a CU: 64 -> 64 channels, 2 x
+    // 2, at 30 x 30 (64 workgroups of four) 15.8 us with four and 10.7 with one, at 80 x 80 (400) 17.1 and 14.0, at
+    // 100 x 100 (640) 18.2 and 21.4; 1 x 1 at 80 x 80 11.8 and 11.7, at 100 x 100 12.9 and 18.1.
+    const bool four = no_overlap && stride <= 2 &&
+                      std::ceil(double(h) * w / 256) * ((cout + 3) / 4) * n >= 512;
     ProbeScope probe("nd_conv_transpose", s, 2.0 * double(n) * h * w * cin * cout * kh * kw,
-                     4.0 * (double(n) * cin * h * w + double(total)));
+                     4.0 * (double(n) * cin * h * w + double(total)), four ? "nd_convt_4" : no_overlap ? "nd_convt_1" : nullptr);
     auto ks = [&](auto *kernel, int cb) {
         hipLaunchKernelGGL(kernel, dim3(unsigned((h * w + 255) / 256), unsigned((cout + cb - 1) / cb), unsigned(n)), dim3(256), 0, s,
                            x, cin, h, w, wt, b, y, cout, act);
     };
-    if (kh == stride && kw == stride && stride >= 1 && stride <= 4 && n <= 65535 && cout <= 65535 &&
-        double(h) * w < 2147483392.0) {
-        if (stride == 2) ks(convt_ks_nchw_kernel<2, 4>, 4);
-        else if (stride == 1) ks(convt_ks_nchw_kernel<1, 4>, 4);
+    if (no_overlap) {
+        if (four && stride == 2) ks(convt_ks_nchw_kernel<2, 4>, 4);
+        else if (four) ks(convt_ks_nchw_kernel<1, 4>, 4);
+        else if (stride == 2) ks(convt_ks_nchw_kernel<2, 1>, 1);
+        else if (stride == 1) ks(convt_ks_nchw_kernel<1, 1>, 1);
         else if (stride == 3) ks(convt_ks_nchw_kernel<3, 1>, 1);
         else ks(convt_ks_nchw_kernel<4, 1>, 1);
     } else {
