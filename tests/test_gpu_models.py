@@ -83,6 +83,17 @@ def test_recognition_config1_float32_weights(ctx, f16):
     assert calls["conv3x3_dma"] >= 1 and calls["gemm_dma"] >= 1 and calls["conv_mfma"] == 0, calls
 
 
+def test_one_line_forms(recognizer, rec_oracle):
+    # One line: the trunk's 3 x 3 layers of few pixels run straight from memory, the last one, whose
+    # four rows are pooled to one, on the persistent kernel, which is the faster there.
+    import ocrhip
+    d = np.random.Generator(np.random.PCG64(3)).uniform(-0.5, 0.5, (1, 64, 200)).astype(np.float32)
+    for f in ("conv3_thin", "conv3_persistent"):
+        ocrhip.probe_start(f)
+    check_recognition(recognizer, rec_oracle, [(d, 1, 200)], [200])
+    assert {f: ocrhip.probe_stop(f)["calls"] for f in ("conv3_thin", "conv3_persistent")} == {"conv3_thin": 3, "conv3_persistent": 1}
+
+
 def test_recognition_edge_shapes(recognizer, rec_oracle):
     # one narrow line (T = 2), a width not a multiple of 4, and a single-line batch
     rng = np.random.Generator(np.random.PCG64(9))

@@ -43,13 +43,14 @@
 // of them x 16 * NT channels.
 //
 // conv3_thin, for launches of few pixels (one recogniser line, the detector's deepest level): a
-// wavefront makes 16 pixels (one 2 x 8 row tile, two in pool mode 3) x 16 channels with its
-// operands read straight from memory, kernel row (3 taps) by kernel row with the next two in
-// flight. Such launches have fewer 256-pixel tiles than the chip has CUs and each walks
-// 3 stages a slice one after another; here every SIMD has a wavefront. It adds the products in
-// the same order, so a line gives the same bits alone as in a large pass. One 200-pixel line: 9, 11,
-// 17 and 16 us a layer -> 5, 8, 13 and 17 (few taps in flight against the latency of other XCDs'
-// outputs; twice as many took the registers of a second wavefront and were no faster).
+// wavefront makes 16 pixels (one 2 x 8 row tile) x 16 channels with its operands read straight from
+// memory, kernel row (3 taps) by kernel row with the next two in flight. Such launches have fewer
+// 256-pixel tiles than the chip has CUs and each walks 3 stages a slice one after another; here
+// every SIMD has a wavefront. It adds the products in the same order, so a line gives the same bits
+// alone as in a large pass. One 200-pixel line: 8.6, 10.8 and 16.5 us a layer -> 6.1, 8.8 and 13.4
+// (twice as many rows in flight took the registers of a second wavefront and were no faster). The
+// recogniser's last layer (pool mode 3) is not faster so: two row tiles a wavefront leave half the
+// wavefronts, 18 us against 16 from 1 line to 8.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void conv3_dma_kernel(C3Params p) 
     }
 }
 
-template <int MT, int ACT>
+template <int ACT>
 __global__ __launch_bounds__(256) void conv3_thin_kernel(C3Params p) {
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
     const int wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -522,7 +523,7 @@ __global__ __launch_bounds__(256) void conv3_thin_kernel(C3Params p) {
     while (sg + 1 < p.nseg && tile >= p.seg[sg + 1].t0) sg++;
     const C3Seg &sd = p.seg[sg];
     const int l = tile - sd.t0, trow = l / sd.tiles_x;
-    const int img = trow / p.tiles_y, oy0 = (trow - img * p.tiles_y) * (2 * MT), ox0 = (l - trow * sd.tiles_x) * 8;
+    const int img = trow / p.tiles_y, oy0 = (trow - img * p.tiles_y) * 2, ox0 = (l - trow * sd.tiles_x) * 8;
     // This lane's pixel of a row tile as an operand: square r >> 2, position r & 3.
     const int py = oy0 + ((r >> 1) & 1), px = ox0 + 2 * (r >> 2) + (r & 1);
     const float *xi = sd.x + size_t(img) * p.h * sd.w * p.xcs;
@@ -530,44 +531,37 @@ __global__ __launch_bounds__(256) void conv3_thin_kernel(C3Params p) {
     constexpr int D = 3;  // kernel rows in flight
     struct Row {
         half8 w[3];
-        float4 x[MT][3][2];
+        float4 x[3][2];
     } R[D];
     auto load = [&](Row &b, int k) __attribute__((always_inline)) {
         const int c = k / 3, ky = k - 3 * c, ch = (c >= p.xchunks ? c - p.xchunks : c) * 32 + 8 * g;
 #pragma unroll
         for (int kx = 0; kx < 3; kx++) {
             b.w[kx] = wp[(c * 9 + ky * 3 + kx) * 64];
+            const int iy = py + ky - 1, ix = px + kx - 1;
+            const bool ok = unsigned(iy) < unsigned(p.h) && unsigned(ix) < unsigned(sd.w);
+            const float *src = xi + (iy * sd.w + ix) * p.xcs + ch;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                const int iy = py + 2 * mt + ky - 1, ix = px + kx - 1;
-                const bool ok = unsigned(iy) < unsigned(p.h) && unsigned(ix) < unsigned(sd.w);
-                const float *src = xi + (iy * sd.w + ix) * p.xcs + ch;
-#pragma unroll
-                for (int e = 0; e < 2; e++)
-                    b.x[mt][kx][e] = *(ok && ch + 4 * e < p.cin ? reinterpret_cast<const float4 *>(src + 4 * e) : p.zero);
-            }
+            for (int e = 0; e < 2; e++)
+                b.x[kx][e] = *(ok && ch + 4 * e < p.cin ? reinterpret_cast<const float4 *>(src + 4 * e) : p.zero);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    floatx4 acc[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
     auto compute = [&](const Row &b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kx = 0; kx < 3; kx++)
+        for (int kx = 0; kx < 3; kx++) {
+            const float4 u = b.x[kx][0], v = b.x[kx][1];
+            const float xs[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+            half8 hi, lo;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                const float4 u = b.x[mt][kx][0], v = b.x[mt][kx][1];
-                const float xs[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-                half8 hi, lo;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    hi[e] = (_Float16)xs[e];
-                    lo[e] = (_Float16)__builtin_fmaf(-1.f, (float)hi[e], xs[e]);
-                }
-                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, b.w[kx], acc[mt], 0, 0, 0);
-                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, b.w[kx], acc[mt], 0, 0, 0);
+            for (int e = 0; e < 8; e++) {
+                hi[e] = (_Float16)xs[e];
+                lo[e] = (_Float16)__builtin_fmaf(-1.f, (float)hi[e], xs[e]);
             }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, b.w[kx], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, b.w[kx], acc, 0, 0, 0);
+        }
     };
     const int rows = 3 * p.chunks;
 #pragma unroll
@@ -584,39 +578,29 @@ __global__ __launch_bounds__(256) void conv3_thin_kernel(C3Params p) {
         }
     // Lane (g, r) holds square g's four pixels of channel r of the tile.
     if (co >= p.cout) return;
-    float v[MT][4];
+    float v[4];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[mt][i] = act3(acc[mt][i] + bias, ACT);
+    for (int i = 0; i < 4; i++) v[i] = act3(acc[i] + bias, ACT);
     const int x = ox0 + 2 * g;
-    if (MT == 2) {
-        // Pool mode 3: max over each pair of rows, then the mean of the two maxima.
-        const size_t line = size_t(sd.noff + img);
-        float *dst = p.tm + (size_t(x) * p.tm_ntot + line) * p.cout + co;
-        if (x < sd.ow) dst[0] = (fmaxf(v[0][0], v[0][2]) + fmaxf(v[MT - 1][0], v[MT - 1][2])) / 2.f;
-        if (x + 1 < sd.ow)
-            dst[size_t(p.tm_ntot) * p.cout] = (fmaxf(v[0][1], v[0][3]) + fmaxf(v[MT - 1][1], v[MT - 1][3])) / 2.f;
-        return;
-    }
     if (sd.y) {
         float *yt = sd.y + (size_t(img) * p.oh + oy0) * sd.ow * p.ycs + co;
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (oy0 + (i >> 1) < p.oh && x + (i & 1) < sd.ow) yt[size_t((i >> 1) * sd.ow + x + (i & 1)) * p.ycs] = v[0][i];
+            if (oy0 + (i >> 1) < p.oh && x + (i & 1) < sd.ow) yt[size_t((i >> 1) * sd.ow + x + (i & 1)) * p.ycs] = v[i];
     }
     if (!p.pool || oy0 / 2 >= p.poh) return;
     float *pt = sd.yp + (size_t(img) * p.poh + oy0 / 2) * sd.pow_ * p.ypcs + co;
     if (p.pool == 1) {
-        if (x / 2 < sd.pow_) pt[size_t(x / 2) * p.ypcs] = fmaxf(fmaxf(v[0][0], v[0][1]), fmaxf(v[0][2], v[0][3]));
+        if (x / 2 < sd.pow_) pt[size_t(x / 2) * p.ypcs] = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
     } else {
-        if (x < sd.pow_) pt[size_t(x) * p.ypcs] = fmaxf(v[0][0], v[0][2]);
-        if (x + 1 < sd.pow_) pt[size_t(x + 1) * p.ypcs] = fmaxf(v[0][1], v[0][3]);
+        if (x < sd.pow_) pt[size_t(x) * p.ypcs] = fmaxf(v[0], v[2]);
+        if (x + 1 < sd.pow_) pt[size_t(x + 1) * p.ypcs] = fmaxf(v[1], v[3]);
     }
 }
 
-// Launches of at most this many wavefronts of conv3_thin take it (one a SIMD): 832 (32 -> 64 at
-// 32 x 100) 8.6 us against 4.9, 448 11 against 8; 2000 (128 -> 256 at 50 x 37) 17 against 22.
+// Launches of at most this many wavefronts of conv3_thin take it (one a SIMD): 992 wavefronts of 32 ->
+// 64 channels 11.6 us on tiles and 8.9, 960 of 128 -> 128 19.7 and 16.4, 896 of 512 -> 256 51.2 and 44.2; 2000 (128 ->
+// 256 at 50 x 37) 17 and 22.
 constexpr double THIN_WAVES = 1024;
 
 int cu_count3() {
@@ -715,13 +699,12 @@ void c3_launch(const ConvArgs *args, int count, int pool, hipStream_t s) {
     }
     if (!fits) fail("conv3x3_dma: no tile fits");
     if (best == 1e300) return;  // no output pixels
-    // Few pixels: conv3_thin's tiles of 2 x 8 (4 x 8 in pool mode 3) pixels x 16 channels.
+    // Few pixels: conv3_thin's tiles of 2 x 8 pixels x 16 channels.
     double thin = 0;
-    for (int k = 0; k < count; k++)
-        thin += double(args[k].y.n) * ((p.oh + (pool == 3 ? 3 : 1)) / (pool == 3 ? 4 : 2)) * ((args[k].y.w + 7) / 8);
+    for (int k = 0; k < count; k++) thin += double(args[k].y.n) * ((p.oh + 1) / 2) * ((args[k].y.w + 7) / 8);
     thin *= (cout + 15) / 16;
-    const bool few = thin <= THIN_WAVES;
-    if (few) p.tw = 8, p.th = pool == 3 ? 4 : 2;
+    const bool few = pool != 3 && thin <= THIN_WAVES;
+    if (few) p.tw = 8, p.th = 2;
     p.hw = p.tw + 2;
     p.hh = p.th + 2;
     p.npx = p.hh * p.hw;
@@ -765,8 +748,7 @@ void c3_launch(const ConvArgs *args, int count, int pool, hipStream_t s) {
         // 16 wavefronts (4 a SIMD): 128-channel blocks as 4 x 4 wavefronts of 2 n-tiles, 64-channel
         // blocks as 4 x 4 of one, 32-channel blocks as 8 x 2 of one (two row tiles each).
         const dim3 gd{unsigned(grid)}, bd{1024}, gt{unsigned((p.tiles * p.nblocks + 3) / 4)}, bt{256};
-        if (few && pool == 3) hipLaunchKernelGGL((conv3_thin_kernel<2, A>), gt, bt, 0, s, p);
-        else if (few) hipLaunchKernelGGL((conv3_thin_kernel<1, A>), gt, bt, 0, s, p);
+        if (few) hipLaunchKernelGGL((conv3_thin_kernel<A>), gt, bt, 0, s, p);
         else if (nt == 4) hipLaunchKernelGGL((conv3_dma_kernel<4, 4, 2, A, 0>), gd, bd, 0, s, p);
         else if (nt == 2 && p.chunks == 1) hipLaunchKernelGGL((conv3_dma_kernel<4, 4, 1, A, 1>), gd, bd, 0, s, p);
         else if (nt == 2) hipLaunchKernelGGL((conv3_dma_kernel<4, 4, 1, A, 0>), gd, bd, 0, s, p);
