@@ -335,9 +335,10 @@ def _timed(ctx, fn, reps, warmup=3):
     return (time.perf_counter() - t) / reps
 
 
-# The recurrence's floor a time step: a SIMD issues the 96 v_mfma_f32_16x16x32_f16 of its four
-# wavefronts (16 cycles each) at 2.4 GHz; the gate arithmetic and the step's barrier come on top.
-GRU_FLOOR_US = 96 * 16 / 2400.0
+# The recurrence's floor a time step: 3 x 256 gate rows by 256 units take 192 sparse
+# v_smfmac_f32_16x16x64_f16, 48 of them (16 cycles each) on each of a CU's four SIMDs, at 2.4 GHz; the
+# gate arithmetic and the step's barrier come on top.
+GRU_FLOOR_US = 3 * 256 // 16 * (256 // 64) // 4 * 16 / 2400.0
 
 
 def _gru_latency(k, steps):
