@@ -105,8 +105,8 @@ __device__ inline void split(const float4 (&v)[2], half8 &hi, half8 &lo) {
     }
 }
 
-// Columns n .. n + 3 of a row (row m of the GEMM). STREAM: stored past L2, for outputs larger
-// than it (4500 x 1536: 21.3 -> 17.0 us).
+// Columns n .. n + 3 of a row (row m of the GEMM). STREAM: stored past L2, as the 256-column tiles
+// store theirs (1.5 MB of output at least, or gemm_thin would have made it; 4500 x 1536 21.3 -> 17.0 us).
 template <int ACT, bool STREAM>
 __device__ inline void put(const GParams &p, int m, int row, int n, const floatx4 &acc, const float4 &b4) {
     if (m >= p.M || n >= p.N) return;

@@ -27,11 +27,13 @@
 // ahead, the new state goes to a double-buffered LDS copy of the A operand: one barrier a step,
 // for LDS only (the loads and the Y stores stay in flight).
 //
-// Measured (a 200-step pass, us a layer): 36 lines 303 -> 129, 540 lines 424 -> 190, against 8
-// lines a workgroup on the dense instruction with the state as its 16-column operand; 200-pixel
-// line alone (50 steps) 77 -> 39. A step takes 0.59 us with 2 lines, of it 0.32 of matrix
-// instructions; 16 wavefronts (4 a SIMD, part of R in LDS) took 1.6, 4 wavefronts (one unit of
+// Measured (us a layer, kernel trace): 36 lines of at most 200 steps 303 -> 127, 540 lines 424 -> 186, one
+// line of 50 steps 77 -> 36, against 8 lines a workgroup on the dense instruction with the state as its
+// 16-column operand. So with 2 lines a step takes 0.61 us, of it 0.32 of matrix instructions, and the
+// launch 6 besides; 16 wavefronts (4 a SIMD, part of R in LDS) took 1.6 a step, 4 wavefronts (one unit of
 // one line a lane, R in 384 registers) 0.89.
+//
+// A workgroup's R takes its CU's register file whole, so nothing else runs on that CU meanwhile.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -272,10 +274,12 @@ __global__ __launch_bounds__(256) void gru_f32_kernel(const float *__restrict__ 
 
 }  // namespace
 
-// 2 lines a workgroup while every workgroup has a CU of its own (256 of them, two directions):
-// 0.65 us a step against 0.81 with 4 lines at 36 lines, 0.82 against 0.86 at 256. Past that 4
-// lines: the longest lines start first, so a 540-line pass (270 workgroups) still ends with its
-// longest line, 190 us against 265 with 2 lines.
+// 2 lines a workgroup while every workgroup has a CU of its own (256 of them, two directions; a layer's
+// time over its 200 steps): 0.64 us against 0.81 with 4 lines at 36 lines, 0.82 against 0.86 at 256. Past
+// that 4 lines: the longest lines start first, so a 540-line pass (270 workgroups) still ends with its
+// longest line, 186 us against 265 with 2 lines. Beside other work (the page pipeline's second stream)
+// 4 lines for every pass, which leave more CUs, measured the same: 12 pages 13.18-13.19 ms against
+// 13.12-13.21.
 int gru_lines(int ntot) { return ntot <= 256 ? 2 : 4; }
 
 void gru_pack_r(const uint16_t *r, uint16_t *out) {

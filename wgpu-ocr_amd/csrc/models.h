@@ -52,8 +52,9 @@ class Recognizer {
     // layer and the arg-max): each recurrence waits for its input projection on the context's
     // stream, which waits for the first only before the second projection and returns without
     // waiting for the second. What the caller queues meanwhile (from between(), or its next
-    // pass's trunk) runs beside the recurrence, whose workgroups occupy one CU per 2 or 4
-    // lines (gru_lines) and direction. logits and best are then written in gru_stream's order: the caller orders its
+    // pass's trunk) runs beside the recurrence, where that leaves CUs: a workgroup takes one whole
+    // per 2 or 4 lines (gru_lines) and direction, and near 256 and past 512 lines all of them at first.
+    // logits and best are then written in gru_stream's order: the caller orders its
     // reads after that stream and marks the buffers as used on it.
     void recognize_device(const Batch *batches, int count, float *logits, uint32_t *best, uint32_t *lens,
                           const std::function<void()> &between = {}, hipStream_t gru_stream = nullptr);
