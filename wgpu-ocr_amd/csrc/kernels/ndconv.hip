@@ -895,11 +895,8 @@ bool nd_conv_nchw_mfma(const NdMfmaConvArgs &a, hipStream_t s) {
     if (waves < 1024 && steps >= 16 && (nt <= 2 || pk.exact)) ks = waves < 512 ? 16 : 8, wpb = 16, mt = 1;
     else if (waves < 1024 && steps >= 8) ks = 4;
     else if (waves < 2048 && steps >= 4) ks = 2;
-    // 1 x 1 convs of few K steps: conv_px, unsplit; of 8 and more from 512 wavefronts on, below which
-    // the split covers more latency (256 -> 64 channels: 98 wavefronts 8.5 us split, 9.7 with conv_px, 328
-    // 9.5 and 10.0, 656 13.4 and 12.0; 400 -> 64 9.6 and 11.6, 11.1 and 12.2, 18.3 and 14.8; 128 -> 64, 4
-    // steps, 8.4 and 8.3, 8.6 and 8.6, 11.3 and 10.4).
-    const bool px = p.flat && mt == 1 && wpb == 4 && steps <= 16 && (steps < 8 || waves >= 512);
+    // 1 x 1 convs of few K steps: conv_px, unsplit.
+    const bool px = p.flat && mt == 1 && wpb == 4 && steps <= 16;
     if (px) ks = 1;
     if (ks > 1 && mt * nt > 8) mt = std::max(1, 8 / nt);
     p.tiles_line = int(std::ceil(lim / (16.0 * mt)));
