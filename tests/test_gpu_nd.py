@@ -631,7 +631,9 @@ def test_transformer_block_shapes(ctx, tmp_path, n, t, dim, heads, hidden, exact
         x = g.add("Add", [x, _linear(g, _attention(g, _layer_norm(g, x, dim), dim, heads), dim, dim, exact)])
         y = _linear(g, _layer_norm(g, x, dim), dim, hidden, exact, act=True)
         x = g.add("Add", [x, _linear(g, y, hidden, dim, exact)])
-        return g.add("Sqrt", [g.add("Relu", [x])])
+        # The graph's last step stays on its own. (It was a square root: that takes an error e of a value
+        # near zero to sqrt(e), 2e-8 to 1.4e-4, past check's bound for some draws.)
+        return g.add("Relu", [x])
     p = build(tmp_path, "block", fn, (n, t, dim))
     x = RNG.standard_normal((n, t, dim)).astype(np.float32)
     calls = ran(["nd_layer_norm", "nd_rows_norm", "nd_mlp", "nd_attention_proj"], lambda: check(ctx, p, x))
