@@ -68,7 +68,7 @@ def test_conv1x1_gemm(ctx, tmp_path, cin, cout, h, w, act):
     (256, 64, 1537, None, "gemm_thin"), (128, 97, 3072, None, "gemm_thin"), (128, 97, 3073, None, "gemm_tile_128"),
     (256, 128, 4096, None, "gemm_thin"), (256, 128, 4097, None, "gemm_tile_128"), (128, 256, 56000, None, "gemm_persistent"),
     (128, 256, 48000, None, "gemm_tile_256"), (512, 1536, 9700, None, "gemm_persistent"), (512, 1536, 8900, None, "gemm_tile_256"),
-    (160, 300, 28001, None, "gemm_persistent"), (160, 300, 33000, None, "gemm_tile_256")])
+    (128, 20480, 100, None, "gemm_tile_256"), (160, 300, 28001, None, "gemm_persistent"), (160, 300, 33000, None, "gemm_tile_256")])
 def test_conv1x1_row_counts(ctx, tmp_path, cin, cout, w, act, form):
     # The GEMM's three forms at the edges of their tiles: one row, few rows (16 x 16), 128 and 64
     # row tiles with a part of a tile left, K and N that end inside a slice or tile, and enough

@@ -541,7 +541,7 @@ double thin_waves(int chunks) { return chunks < 8 ? 1536 : 2048; }
 // 1536 (708 tiles) 81 and 123 us for K = 256 and 512 against gemm_tile's 96 and 130, 71 700 rows
 // 176 and 275 against 223 and 310.
 constexpr double BIG_TILES = 640;
-// Smaller ones too when its rounds of tiles, one a CU, are this full. us, gemm_dma against gemm_tile, by
+// Smaller ones too when their rows fill its rounds of tiles, one a CU, so far. us, gemm_dma against gemm_tile, by
 // fullness: 256 columns, K = 128, 0.59 42.9 and 39.1, 0.76 44.6 and 53.2, 0.78 26.3 and 32.9, 0.88 26.2 and 34.9;
 // K = 256, 0.76 70.4 and 72.9, 0.88 34.5 and 43.5. 512 columns, K = 256, 0.59 56.0 and 48.0, 0.76 63.2 and 61.2, 0.86
 // 64.2 and 65.5, 0.88 33.4 and 40.8; K = 512, 0.76 96.8 and 94.1, 0.86 96.8 and 92.1, 0.88 48.3 and 55.1. 1536 columns,
@@ -590,7 +590,7 @@ bool gemm_dma(const ConvArgs &a, hipStream_t s) {
     p.runs = std::max(1, std::min(p.mtiles, gcu_count() / p.nblocks));
     const double slots = std::max(1, gcu_count() / p.nblocks), rounds = std::ceil(p.mtiles / slots);
     const bool few = thin <= thin_waves(p.chunks);
-    const bool many = N > 128 && (big >= BIG_TILES || p.mtiles >= full_rounds(N) * slots * rounds);
+    const bool many = N > 128 && (big >= BIG_TILES || p.M >= full_rounds(N) * GBM * slots * rounds);
     const bool narrow = p.ntiles <= 8;
     double blocks;
     if (few) {
