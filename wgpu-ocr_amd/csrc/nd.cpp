@@ -418,7 +418,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
         y.p = y.buf->as<float>();
         const auto os = strides_of(y.shape);
         size_t c0 = 0;
-        for (const NdPart &part : t.parts->list) {
+        for (NdPart &part : t.parts->list) {
             if (part.up && t.parts->list.size() == 1) {
                 const auto &ps = part.t.shape;
                 nd_resize_nearest(part.t.p, y.p, size_t(ps[0] * ps[1]), int(ps[2]), int(ps[3]), int(y.shape[2]),
@@ -437,6 +437,7 @@ NdTensor NdGraph::run_ops(Ctx *ctx, const NdTensor &x, size_t nops, std::map<std
             }
             nd_copy(src.p, y.p, ix, 0, c0 * os[1], st);
             c0 += size_t(src.shape[1]);
+            part.of = {};  // the upscaled value in memory goes with its own last reader
         }
         return y;
     };

@@ -28,7 +28,7 @@ struct NdTensor {
 struct NdPart {
     NdTensor t;
     int up = 0;
-    NdTensor of;  // up > 0: the upscaled value itself
+    NdTensor of;  // up > 0: the upscaled value itself, until the Concat that has this part is written out
 };
 // The parts of a value that a run makes, one for all that hold the value.
 struct NdParts {
